@@ -123,7 +123,8 @@ void mbir_run(Ctx &cx, const lam_dataset *ds, int nds, const long long rd[3], co
             autotune_bins(cx, *sub, od, eps, nullptr);
         }
         float *ys[3] = {yT.v().c[0], yT.v().c[1], yT.v().c[2]};
-        adjoint(cx, *grids.back(), od, eps, padded.as<float>(), ys, true);
+        adjoint(cx, *grids.back(), od, eps, padded.as<float>(), ys, true,
+                pr.method == 3 ? SpreadOrder::Tiles : SpreadOrder::Rows);
     }
     raw.release();
     padded.release();

@@ -73,6 +73,8 @@ struct RowPlan {
     std::vector<long long> row_chunk;  // first chunk of each row, then nchunks (Jn + 1 entries)
 };
 
+struct TilePlan;   // tiles.h
+
 struct Grid {
     Ctx *cx = nullptr;
     long long P = 0, R = 0, C = 0;
@@ -84,6 +86,7 @@ struct Grid {
     std::vector<Geo> geo_host;
     std::map<std::vector<long long>, std::unique_ptr<SortedPoints>> bins;
     std::map<std::vector<long long>, std::unique_ptr<RowPlan>> rowplans;
+    std::map<std::vector<long long>, std::unique_ptr<TilePlan>> tileplans;
     ~Grid();
 };
 
@@ -94,6 +97,7 @@ struct NufftPlan {
     float beta = 13.8f;
     DevBuf corr[3];               // float 1/psi_hat per axis, indexed by array index
     DevBuf fine;                  // float2 [nfz][nfy][nfx][3]
+    DevBuf rec;                   // float2 [planes of the jobs][component groups][16][32] of the tile spreader
     DevBuf slab;                  // float2 [rows][nfz][nfx][3] of the row-factorised path
     DevBuf halo;                  // float2 [rows][tiles][halo cells][3] of the row-factorised spreader
 };
@@ -105,12 +109,20 @@ NufftPlan &get_nufft_plan(Ctx &cx, const long long dims[3], double eps);
 std::unique_ptr<Grid> make_grid(Ctx &cx, const double *alpha, const double *gamma, long long P, long long R,
                                 long long C);
 
+// Summation order of the three-component spreader.  Tiles: matrix-core blocks (tiles.h).
+// Rows: the row-factorised spreader, kept for the backprojections that MBIR1 and MBIR2 solve
+// against: conjugate gradients on the normal operator multiply a change in the last bits of
+// yT about a hundredfold (measured over 60 jobs: 2e-7 in yT becomes up to 5e-5 of MBIR1's
+// result and 1.4e-5 of MBIR2's, 2e-7 of MBIR3's), so a job's result stays what it was.
+// Grids whose tilt varies have no row form and take the tiles.
+enum class SpreadOrder { Tiles, Rows };
+
 // Projectors and NUFFT entry points (device pointers, context stream)
 void nufft2_complex(Ctx &cx, Grid &g, const long long dims[3], double eps, float2 *c, const float2 *f);
 void nufft1_complex(Ctx &cx, Grid &g, const long long dims[3], double eps, const float2 *c, float2 *f);
 void forward(Ctx &cx, Grid &g, const long long dims[3], double eps, const float *const m[3], float *proj);
 void adjoint(Ctx &cx, Grid &g, const long long dims[3], double eps, const float *proj, float *const m[3],
-             bool accumulate);
+             bool accumulate, SpreadOrder order = SpreadOrder::Tiles);
 void sysmat_nufft(Ctx &cx, Grid &g, const long long dims[3], double eps, const float *const x[3],
                   float *const y[3]);
 // Several grids at once: one fine-grid transform (and de-apodisation) serves them all.
@@ -127,9 +139,9 @@ std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], doub
 bool bins_tuned(Ctx &cx, Grid &g, const long long dims[3], double eps);
 // Device bytes of the row-factorised projectors of one shared-tilt grid of P
 // projections of R x C on the fine grid of dims: slab: the row group's slabs
-// and halos (kept by the plan, shared by grids of the same dims), kept: the
-// grid's row bins, setup: temporaries while they are built.  Zero when the
-// fine grid has no row tiling.
+// and halos and the tile spreader's records (kept by the plan, shared by grids
+// of the same dims), kept: the grid's point bins, setup: temporaries while
+// they are built.
 struct RowBytes {
     size_t slab = 0, kept = 0, setup = 0;
 };

@@ -16,82 +16,13 @@
 
 #include "fastdiv.h"
 #include "nufft.h"
+#include "nufft_point.h"
+#include "tiles.h"
 
 
 namespace lam {
 
 namespace {
-
-constexpr double kTwoPi = 6.283185307179586476925286766559;
-
-__device__ __forceinline__ int wrapi(int i, int n) {
-    if (i < 0) i += n;
-    else if (i >= n) i -= n;
-    return i;
-}
-
-// Coordinate arithmetic is kept free of FMA contraction so that every kernel
-// that places a point (binning, spreading, interpolation) computes bitwise the
-// same fine coordinate and first kernel cell.
-
-// Folds t into one period and returns the first kernel cell ceil(t - W/2).
-// The fold multiplies by the reciprocal 1/nf: at an exact multiple of nf it
-// may land on -0 ulp or nf, which every caller wraps (wrap0) identically.
-__device__ __forceinline__ int first_cell(double &t, int nf, double rnf, int W) {
-#pragma clang fp contract(off)
-    const double fl = floor(t * rnf);
-    t -= fl * (double)nf;
-    return (int)ceil(t - 0.5 * W);
-}
-
-// ES kernel weights for one axis: cells i0 .. i0+W-1 around the folded coordinate t.
-template <int W>
-__device__ __forceinline__ void es_weights(double t, int i0, float beta, float *wts) {
-    const float z0 = (float)(((double)i0 - t) * (2.0 / W));
-    const float dz = 2.0f / (float)W;
-#pragma unroll
-    for (int m = 0; m < W; ++m) {
-        const float z = z0 + dz * (float)m;
-        const float r = 1.0f - z * z;
-        // r in (0, 1]: the hardware square root (no denormal rescaling needed)
-        wts[m] = r > 0.f ? __expf(beta * (__builtin_amdgcn_sqrtf(r) - 1.0f)) : 0.f;
-    }
-}
-
-struct PointFrame {
-    double dX, dY, k0, j0, sx, sy, sz;  // qX step, qY step, centres, fine scales nf/(2 pi)
-    double rx, ry, rz;                  // 1 / nf per axis
-};
-
-__device__ __forceinline__ void point_coords(const Geo &g, const PointFrame &f, int j, int k, double &tx, double &ty,
-                                             double &tz) {
-#pragma clang fp contract(off)
-    const double qX = ((double)k - f.k0) * f.dX;
-    const double qY = ((double)j - f.j0) * f.dY;
-    tx = (qX * g.ux + qY * g.vx) * f.sx;
-    ty = (qY * g.vy) * f.sy;
-    tz = (qX * g.uz + qY * g.vz) * f.sz;
-}
-
-// Placement of one point: folded coordinates, first cells, weights.
-template <int W>
-struct Placed {
-    int ix, iy, iz;
-    float wx[W], wy[W], wz[W];
-};
-
-template <int W>
-__device__ __forceinline__ void place(const Geo &g, const PointFrame &fr, int j, int k, int nfz, int nfy, int nfx,
-                                      float beta, Placed<W> &pt) {
-    double tx, ty, tz;
-    point_coords(g, fr, j, k, tx, ty, tz);
-    pt.ix = first_cell(tx, nfx, fr.rx, W);
-    pt.iy = first_cell(ty, nfy, fr.ry, W);
-    pt.iz = first_cell(tz, nfz, fr.rz, W);
-    es_weights<W>(tx, pt.ix, beta, pt.wx);
-    es_weights<W>(ty, pt.iy, beta, pt.wy);
-    es_weights<W>(tz, pt.iz, beta, pt.wz);
-}
 
 // Tiling of the fine grid for the spreader: tile (tz,ty,tx) owns the points
 // whose first kernel cell (wrapped into [0,nf)) lies in it, and accumulates
@@ -102,7 +33,6 @@ struct BinParams {
     FastDiv fhx, fhyx;   // halo box row length HX and plane size HY * HX
 };
 
-__device__ __forceinline__ int wrap0(int i, int n) { return i < 0 ? i + n : (i >= n ? i - n : i); }
 
 // ------------------------------------------------------------------ deapodise + pad
 // fine[g][c] = vol_c[i] * corr, array index i <-> mode i - n/2 <-> fine index
@@ -288,48 +218,6 @@ __device__ __forceinline__ long long box_to_fine(const TileBox &b, const BinPara
     return ((long long)gz * nfy + gy) * nfx + gx;
 }
 
-// The three component values a half-set point spreads: v = c(q) + conj c(-q)
-// of plane p (the mirror is q's negative), times d_p.  Paired planes hold
-// Z = P2m + i P2m+1 in plane 2m: the even plane's value is Z(q) + conj Z(-q),
-// the odd one's -i (Z(q) - conj Z(-q)); the centre point (its own mirror)
-// takes Re Z or Im Z.
-// a = c(q) and b = c(-q) of the point's (paired) plane, as loaded by half_point_values
-__device__ __forceinline__ void half_point_combine(float2 a, float2 b, long long p, long long idx, long long S,
-                                                   const Geo &g, int paired, float2 vc[3]) {
-    const long long mir = S - 1 - idx;
-    float2 v;
-    if (!paired) v = mir != idx ? cadd(a, cconj(b)) : a;
-    else if (!(p & 1)) v = mir != idx ? make_float2(a.x + b.x, a.y - b.y) : make_float2(a.x, 0.f);
-    else v = mir != idx ? make_float2(a.y + b.y, b.x - a.x) : make_float2(a.y, 0.f);
-    vc[0] = cscale(v, (float)g.d0);
-    vc[1] = cscale(v, (float)g.d1);
-    vc[2] = cscale(v, (float)g.d2);
-}
-
-__device__ __forceinline__ void half_point_values(const float2 *__restrict__ c, long long p, long long idx,
-                                                  long long S, const Geo &g, int paired, float2 vc[3]) {
-    const long long mir = S - 1 - idx;
-    const long long pl = paired ? (p & ~1ll) : p;
-    const float2 a = c[pl * S + idx];
-    const float2 b = mir != idx ? c[pl * S + mir] : make_float2(0.f, 0.f);
-    half_point_combine(a, b, p, idx, S, g, paired, vc);
-}
-
-// The interpolated value of a half-set point and its mirror: s = sum_i d_i c_i
-// at q, conj(s) at -q; at q = 0 (its own mirror) the transform of a real
-// volume is real.
-__device__ __forceinline__ void store_half_point(float2 *__restrict__ c, long long p, long long idx, long long S,
-                                                 const Geo &g, const float2 acc[3]) {
-    const float d0 = (float)g.d0, d1 = (float)g.d1, d2 = (float)g.d2;
-    float2 s;
-    s.x = d0 * acc[0].x + d1 * acc[1].x + d2 * acc[2].x;
-    s.y = d0 * acc[0].y + d1 * acc[1].y + d2 * acc[2].y;
-    const long long mir = S - 1 - idx;
-    if (mir == idx) s.y = 0.f;
-    c[p * S + idx] = s;
-    if (mir != idx) c[p * S + mir] = cconj(s);
-}
-
 // ---- spreading (type 1)
 // The box accumulator lives in LDS as NC complex planes.  The four waves of
 // the workgroup own the four (z, y) parity classes of box cells; every wave
@@ -364,13 +252,13 @@ struct StageLayout {
 template <int W, int NC>
 constexpr int stage_words() { return StageLayout<W, NC>::SW; }
 
-template <int W, bool HALF>
+template <int W>
 __global__ __launch_bounds__(256) void k_spread_tiled(float2 *__restrict__ fine, const float2 *__restrict__ c,
                                                       const Geo *__restrict__ geo, long long P, int R, int C,
                                                       int nfz, int nfy, int nfx, float beta, PointFrame fr,
                                                       BinParams bp, const unsigned *__restrict__ ids,
-                                                      const uint4 *__restrict__ chunks, int paired) {
-    constexpr int NC = HALF ? 3 : 1;
+                                                      const uint4 *__restrict__ chunks) {
+    constexpr int NC = 1;
     using SL = StageLayout<W, NC>;
     constexpr int SW = SL::SW;
     constexpr int HW = W / 2;
@@ -387,7 +275,7 @@ __global__ __launch_bounds__(256) void k_spread_tiled(float2 *__restrict__ fine,
     const int zpar = wave >> 1, ypar = wave & 1;
     const int HYX = bx.HY * bx.HX;
     const long long S = (long long)R * C;
-    const long long H = HALF ? (S + 1) / 2 : S;
+    const long long H = S;
 
     // this lane's cells of a point: (a, b, e) = (zoff + 2 ia, yoff + 2 ib, e)
     int loff[NCH], wzo[NCH], wyo[NCH], wxo[NCH];
@@ -447,8 +335,7 @@ __global__ __launch_bounds__(256) void k_spread_tiled(float2 *__restrict__ fine,
             const int j = (int)(idx / C), k = (int)(idx - (long long)j * C);
             const Geo g = geo[p];
             float2 vc[NC];
-            if constexpr (HALF) half_point_values(c, p, idx, S, g, paired, vc);
-            else vc[0] = c[p * S + idx];
+            vc[0] = c[p * S + idx];
             Placed<W> pt;
             place<W>(g, fr, j, k, nfz, nfy, nfx, beta, pt);
             const int lz = wrap0(pt.iz, nfz) - bx.oz, ly = wrap0(pt.iy, nfy) - bx.oy, lx = wrap0(pt.ix, nfx) - bx.ox;
@@ -1395,21 +1282,6 @@ void gauss_legendre(int n, double *x, double *wt) {
     }
 }
 
-PointFrame frame(const Grid &g, const NufftPlan &pl) {
-    PointFrame f;
-    f.dX = kTwoPi / (double)g.C;
-    f.dY = kTwoPi / (double)g.R;
-    f.k0 = 0.5 * (double)(g.C - 1);
-    f.j0 = 0.5 * (double)(g.R - 1);
-    f.sx = (double)pl.nf[2] / kTwoPi;
-    f.sy = (double)pl.nf[1] / kTwoPi;
-    f.sz = (double)pl.nf[0] / kTwoPi;
-    f.rx = 1.0 / (double)pl.nf[2];
-    f.ry = 1.0 / (double)pl.nf[1];
-    f.rz = 1.0 / (double)pl.nf[0];
-    return f;
-}
-
 #define LAM_WIDTH_SWITCH(w, CALL)                                          \
     switch (w) {                                                           \
         case 4: { constexpr int W = 4; CALL; } break;                      \
@@ -1548,7 +1420,7 @@ SortedPoints &get_bins(Ctx &cx, Grid &g, NufftPlan &pl, bool half, const BinPara
     DevBuf key0(sizeof(unsigned) * std::max<long long>(total, 1));
     DevBuf count(sizeof(unsigned) * ntiles);
     LAM_HIP(hipMemsetAsync(count.ptr, 0, count.bytes, cx.stream));
-    const PointFrame fr = frame(g, pl);
+    const PointFrame fr = point_frame(g, pl);
     const unsigned grid = grid_for((size_t)total, 256, 1u << 20);
     const Geo *geo = g.geo.as<Geo>();
     if (half) {
@@ -1650,7 +1522,7 @@ bool use_rows(const Grid &g, const NufftPlan &pl) {
     if (!g.shared_tilt) return false;
     const char *e = std::getenv("LAMINO_NUFFT_ROWS");
     if (e && e[0] == '0') return false;
-    return rows_fit(g, row_geom(pl));
+    return rows_fit(g, row_geom(pl)) && tile_plan_fits(g, pl, false);
 }
 
 // Tile edge targets (z, x) the row-path autotuner times; the first is the untuned default.
@@ -1698,7 +1570,7 @@ RowPlan &get_rowplan(Ctx &cx, Grid &g, NufftPlan &pl) {
 
     // Row weights from the same coordinate expression as the kernels (ty = (qY vy) sy),
     // in double; iy is the unwrapped first cell, linear in j and so monotonic.
-    const PointFrame fr = frame(g, pl);
+    const PointFrame fr = point_frame(g, pl);
     const double vy = g.geo_host[0].vy;
     std::vector<float> wyh((size_t)rp->Jn * W);
     std::vector<int> iyh(rp->Jn);
@@ -1811,6 +1683,10 @@ RowBytes row_path_bytes(const long long dims[3], double eps, long long P, long l
         b.kept = std::max(b.kept, 4 * (size_t)half + 20 * cells + 8 * (size_t)Jn * pl.w + cells / 8 + 4 * rg.ntiles);
     }
     b.setup = 16 * (size_t)half + ((size_t)16 << 20);                // sort keys / spare ids, sort scratch
+    const TileBytes tb = tile_bytes(dims, eps, P, R, C);
+    b.slab += tb.records;
+    b.kept += tb.kept;
+    b.setup = std::max(b.setup, tb.setup);
     return b;
 }
 
@@ -1836,7 +1712,7 @@ template <int W>
 void interp_rows_w(Ctx &cx, Grid &g, NufftPlan &pl, float2 *c, RowPlan &rp) {
     const int Jg = rows_per_group(rp, pl);
     pl.slab.ensure(row_slab_bytes(pl) * Jg);
-    const PointFrame fr = frame(g, pl);
+    const PointFrame fr = point_frame(g, pl);
     const size_t lds = rows_interp_lds(rp.rg);
     allow_lds(&k_rows_interp<W>, lds);
     const long long Hh = (g.R * g.C + 1) / 2;
@@ -1878,7 +1754,7 @@ void spread_rows_w(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, RowPlan &rp
     const int Jg = rows_per_group(rp, pl);
     pl.slab.ensure(row_slab_bytes(pl) * Jg);
     pl.halo.ensure(row_halo_bytes(rp.rg) * Jg);
-    const PointFrame fr = frame(g, pl);
+    const PointFrame fr = point_frame(g, pl);
     const size_t lds = rows_spread_lds(rp.rg, W);
     allow_lds(&k_rows_spread<W>, lds);
     // point ids are below 2^31 (the row plan requires it), so 32-bit multiply-shift
@@ -1906,14 +1782,13 @@ void spread_rows_w(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, RowPlan &rp
     }
 }
 
-template <int W, bool HALF>
-void spread_w(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, const BinParams &bp, SortedPoints &sp, bool paired) {
-    constexpr int NC = HALF ? 3 : 1;
-    const size_t lds = spread_lds_bytes(bp.T, W, NC);
-    allow_lds(&k_spread_tiled<W, HALF>, lds);
-    hipLaunchKernelGGL((k_spread_tiled<W, HALF>), dim3((unsigned)sp.nchunks), dim3(256), lds, cx.stream,
+template <int W>
+void spread_w(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, const BinParams &bp, SortedPoints &sp) {
+    const size_t lds = spread_lds_bytes(bp.T, W, 1);
+    allow_lds(&k_spread_tiled<W>, lds);
+    hipLaunchKernelGGL((k_spread_tiled<W>), dim3((unsigned)sp.nchunks), dim3(256), lds, cx.stream,
                        pl.fine.as<float2>(), c, g.geo.as<Geo>(), g.P, (int)g.R, (int)g.C, pl.nf[0], pl.nf[1], pl.nf[2],
-                       pl.beta, frame(g, pl), bp, sp.ids.as<unsigned>(), sp.chunks.as<uint4>(), paired ? 1 : 0);
+                       pl.beta, point_frame(g, pl), bp, sp.ids.as<unsigned>(), sp.chunks.as<uint4>());
 }
 
 template <int W, bool HALF>
@@ -1923,15 +1798,15 @@ void interp_w(Ctx &cx, Grid &g, NufftPlan &pl, float2 *c, const BinParams &bp, S
     allow_lds(&k_interp_tiled<W, HALF>, lds);
     hipLaunchKernelGGL((k_interp_tiled<W, HALF>), dim3((unsigned)sp.nchunks), dim3(256), lds, cx.stream,
                        pl.fine.as<float2>(), c, g.geo.as<Geo>(), g.P, (int)g.R, (int)g.C, pl.nf[0], pl.nf[1], pl.nf[2],
-                       pl.beta, frame(g, pl), bp, sp.ids.as<unsigned>(), sp.chunks.as<uint4>());
+                       pl.beta, point_frame(g, pl), bp, sp.ids.as<unsigned>(), sp.chunks.as<uint4>());
 }
 
 // paired: c holds detector-pair spectra (det_fft2_real_pairs), three-component form only
 // add: accumulate into the fine grid's current contents (no zero fill, no stores)
+// order: which of the three-component spreaders (see SpreadOrder)
 void launch_spread(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, bool half, bool paired = false,
-                   bool add = false) {
-    const int nc = half ? 3 : 1;
-    if (half && use_rows(g, pl)) {
+                   bool add = false, SpreadOrder order = SpreadOrder::Tiles) {
+    if (half && order == SpreadOrder::Rows && use_rows(g, pl)) {
         RowPlan &rp = get_rowplan(cx, g, pl);
         // One row group whose y window does not wrap writes every plane of the window
         // once, and the transforms that follow read only the window: no zeroing.
@@ -1943,18 +1818,19 @@ void launch_spread(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, bool half, 
         LAM_WIDTH_SWITCH(pl.w, (spread_rows_w<W>(cx, g, pl, c, rp, paired, stores)));
         return;
     }
-    const BinParams bp = bin_params(cx, g, pl, nc);
-    SortedPoints &sp = get_bins(cx, g, pl, half, bp);
+    if (half) {
+        TilePlan &tp = get_tileplan(cx, g, pl, !use_rows(g, pl));
+        TimedScope ts(cx, "spread");
+        tile_spread(cx, g, pl, tp, c, paired, add);
+        return;
+    }
+    const BinParams bp = bin_params(cx, g, pl, 1);
+    SortedPoints &sp = get_bins(cx, g, pl, false, bp);
     if (!add)
-        LAM_HIP(hipMemsetAsync(pl.fine.ptr, 0, sizeof(float2) * (size_t)pl.nf[0] * pl.nf[1] * pl.nf[2] * nc,
-                               cx.stream));
+        LAM_HIP(hipMemsetAsync(pl.fine.ptr, 0, sizeof(float2) * (size_t)pl.nf[0] * pl.nf[1] * pl.nf[2], cx.stream));
     if (sp.nchunks == 0) return;
     TimedScope ts(cx, "spread");
-    if (half) {
-        LAM_WIDTH_SWITCH(pl.w, (spread_w<W, true>(cx, g, pl, c, bp, sp, paired)));
-    } else {
-        LAM_WIDTH_SWITCH(pl.w, (spread_w<W, false>(cx, g, pl, c, bp, sp, false)));
-    }
+    LAM_WIDTH_SWITCH(pl.w, (spread_w<W>(cx, g, pl, c, bp, sp)));
     check_launch();
 }
 
@@ -2027,12 +1903,9 @@ void crop_deapod(Ctx &cx, NufftPlan &pl, float *const out[3], float2 *cout, int 
 struct YWin {
     int lo = 0, len = 0;
 };
-YWin y_window(Ctx &cx, Grid &g, NufftPlan &pl) {
+YWin y_window(const Grid &g, const NufftPlan &pl) {
     YWin w;
-    if (!use_rows(g, pl)) return w;
-    const RowPlan &rp = get_rowplan(cx, g, pl);
-    w.lo = rp.ylo;
-    w.len = rp.ly;
+    if (use_rows(g, pl)) row_window(g, pl, w.lo, w.len);
     return w;
 }
 
@@ -2207,7 +2080,7 @@ void forward(Ctx &cx, Grid &g, const long long dims[3], double eps, const float 
     cx.work[0].ensure(sizeof(float2) * M);
     float2 *cbuf = cx.work[0].as<float2>();
     deapod_pad(cx, pl, m, nullptr, 3);
-    const YWin yw = y_window(cx, g, pl);
+    const YWin yw = y_window(g, pl);
     fine_fft(cx, pl, 3, -1, yw.lo, yw.len);
     launch_interp(cx, g, pl, cbuf, true);
     const float scale = 1.0f / (float)(g.R * g.C);
@@ -2216,7 +2089,7 @@ void forward(Ctx &cx, Grid &g, const long long dims[3], double eps, const float 
 }
 
 void adjoint(Ctx &cx, Grid &g, const long long dims[3], double eps, const float *proj, float *const m[3],
-             bool accumulate) {
+             bool accumulate, SpreadOrder order) {
     NufftPlan &pl = get_nufft_plan(cx, dims, eps);
     ensure_fine(pl, 3);
     const size_t M = (size_t)(g.P * g.R * g.C);
@@ -2225,18 +2098,18 @@ void adjoint(Ctx &cx, Grid &g, const long long dims[3], double eps, const float 
     const bool paired = paired_planes(g);
     if (paired) det_fft2_real_pairs(cx, proj, cbuf, (int)g.P, (int)g.R, (int)g.C, -1);
     else det_fft2(cx, proj, true, cbuf, false, (int)g.P, (int)g.R, (int)g.C, -1, 1.0f, cbuf);
-    launch_spread(cx, g, pl, cbuf, true, paired);
-    const YWin yw = y_window(cx, g, pl);
+    launch_spread(cx, g, pl, cbuf, true, paired, false, order);
+    const YWin yw = y_window(g, pl);
     fine_fft(cx, pl, 3, +1, yw.lo, yw.len);
     crop_deapod(cx, pl, m, nullptr, 3, 1.0f / (float)(g.R * g.C), accumulate);
 }
 
 namespace {
 // The y window shared by several grids' projectors: theirs when all agree, else all planes.
-YWin common_window(Ctx &cx, Grid *const *grids, int ngrids, NufftPlan &pl) {
-    YWin w = y_window(cx, *grids[0], pl);
+YWin common_window(Grid *const *grids, int ngrids, NufftPlan &pl) {
+    YWin w = y_window(*grids[0], pl);
     for (int k = 1; k < ngrids; ++k) {
-        const YWin v = y_window(cx, *grids[k], pl);
+        const YWin v = y_window(*grids[k], pl);
         if (v.lo != w.lo || v.len != w.len) return YWin{};
     }
     return w;
@@ -2253,7 +2126,7 @@ void forward_multi(Ctx &cx, Grid *const *grids, int ngrids, const long long dims
     cx.work[0].ensure(sizeof(float2) * M);
     float2 *cbuf = cx.work[0].as<float2>();
     deapod_pad(cx, pl, m, nullptr, 3);
-    const YWin yw = common_window(cx, grids, ngrids, pl);
+    const YWin yw = common_window(grids, ngrids, pl);
     fine_fft(cx, pl, 3, -1, yw.lo, yw.len);
     for (int k = 0; k < ngrids; ++k) {
         Grid &g = *grids[k];
@@ -2273,7 +2146,7 @@ void adjoint_multi(Ctx &cx, Grid *const *grids, int ngrids, const long long dims
     for (int k = 0; k < ngrids; ++k) M = std::max(M, (size_t)(grids[k]->P * grids[k]->R * grids[k]->C));
     cx.work[0].ensure(sizeof(float2) * M);
     float2 *cbuf = cx.work[0].as<float2>();
-    const YWin yw = common_window(cx, grids, ngrids, pl);
+    const YWin yw = common_window(grids, ngrids, pl);
     // the first grid stores its window (or zero-fills); with different windows the
     // union is not what the first grid writes, so the whole fine grid starts at zero
     bool add = false;
@@ -2305,7 +2178,7 @@ void sysmat_nufft(Ctx &cx, Grid &g, const long long dims[3], double eps, const f
     cx.work[0].ensure(sizeof(float2) * M);
     float2 *cbuf = cx.work[0].as<float2>();
     deapod_pad(cx, pl, x, nullptr, 3);
-    const YWin yw = y_window(cx, g, pl);
+    const YWin yw = y_window(g, pl);
     fine_fft(cx, pl, 3, -1, yw.lo, yw.len);
     launch_interp(cx, g, pl, cbuf, true);
     launch_spread(cx, g, pl, cbuf, true);
@@ -2357,11 +2230,11 @@ std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], doub
                 if (std::find(seen.begin(), seen.end(), std::make_pair(rg.Tz, rg.Tx)) != seen.end()) continue;
                 seen.emplace_back(rg.Tz, rg.Tx);
                 cx.bin_tune[rkey] = {rg.Tz, pl.w, rg.Tx};
-                launch_spread(cx, g, pl, cbuf, true);   // builds this tiling's bins
+                launch_spread(cx, g, pl, cbuf, true, false, false, SpreadOrder::Rows);   // builds this tiling's bins
                 float t = 0.f;
                 for (int rep = 0; rep < 2; ++rep) {
                     LAM_HIP(hipEventRecord(e0, cx.stream));
-                    launch_spread(cx, g, pl, cbuf, true);
+                    launch_spread(cx, g, pl, cbuf, true, false, false, SpreadOrder::Rows);
                     launch_interp(cx, g, pl, cbuf, true);
                     LAM_HIP(hipEventRecord(e1, cx.stream));
                     LAM_HIP(hipEventSynchronize(e1));

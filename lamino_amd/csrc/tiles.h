@@ -1,0 +1,67 @@
+// Matrix-core spreading of the three-component projectors over (z, x) tiles of the fine grid
+// (tiles.hip).
+#pragma once
+#include "nufft.h"
+
+namespace lam {
+
+// Cutting of the (z, x) plane into tiles whose first-cell edges Tz x Tx leave room for the
+// kernel inside one 16 x 16 matrix-core block (T + W - 1 <= 16).  Tile (tz, tx) owns the
+// points whose first kernel cell lies in [tz Tz, (tz + 1) Tz) x [tx Tx, (tx + 1) Tx).
+struct TileGeom {
+    int W = 0;
+    int Tz = 0, Tx = 0, ntz = 0, ntx = 0;
+    unsigned ntiles = 0;
+    int nfz = 0, nfy = 0, nfx = 0;
+    int Jn = 0;      // rows of the half point set
+    int nrho = 0;    // row slots: detector rows (shared tilt) or first y cells (direct)
+    int dir = 1;     // slot of row j: j (+1) or Jn - 1 - j (-1), so that first y cells never fall
+    int direct = 0;  // the slot is the point's wrapped first y cell
+    FastDiv fTz, fTx, fntx;
+};
+
+// A share of one tile's points for one wave: ids [beg, end), of the row slots [r0, r1), which
+// reach the planes [y0, y0 + np) (unwrapped; yw = y0 modulo the period), recorded from plane
+// record `plane`.
+struct TileJob {
+    unsigned tile, beg, end;
+    int r0, r1, y0, np, yw;
+    unsigned plane;
+};
+
+// Points of one grid ordered by (tile, row slot, point number), each (tile, slot) padded to
+// a multiple of 4 with kNoPoint.
+struct TilePlan {
+    TileGeom tg;
+    int ylo = 0, ly = 0;           // the y planes touched: [ylo, ylo + ly) mod nfy (ly 0: all)
+    DevBuf off;                    // unsigned [ntiles * nrho + 1] first id of each (tile, slot)
+    DevBuf ids;                    // point numbers
+    DevBuf rowy;                   // RowY [nrho]
+    DevBuf geo;                    // TileGeo [P]
+    DevBuf jobs;                   // TileJob [njobs], tile by tile
+    DevBuf job0;                   // unsigned [ntiles + 1] first job of each tile
+    unsigned njobs = 0, planes = 0;   // planes: recorded by all jobs
+    // cells of each axis as (tile, cell of its block) pairs: starts [nf + 1], then pairs
+    DevBuf zmap, xmap;
+};
+
+// The y planes [ylo, ylo + ly) (mod nfy) that the rows of a shared-tilt grid touch (ly 0: all).
+void row_window(const Grid &g, const NufftPlan &pl, int &ylo, int &ly);
+
+// Whether the plan's buckets and point list have 32-bit numbers.
+bool tile_plan_fits(const Grid &g, const NufftPlan &pl, bool direct);
+
+TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct);
+
+// fine (+)= the type-1 spread of the half point set.  add = false writes every plane of the
+// plan's window (every plane when ly is 0).
+void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c, bool paired, bool add);
+
+// Upper bounds of the device bytes of a plan (kept, and temporaries while it is built) and
+// of the plane records of its spread.
+struct TileBytes {
+    size_t kept = 0, setup = 0, records = 0;
+};
+TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long R, long long C);
+
+}  // namespace lam

@@ -1,0 +1,953 @@
+// Spreading (type 1) of the three-component projectors on the matrix cores.
+//
+// A point touches W x W cells of the (z, x) plane with weights wz (x) wx, times the y
+// weights of its line.  Every point of a line (projection, detector row) has the same y,
+// because the in-plane basis vector u has no y component.  Over the points of one tile and
+// one row, spreading is therefore a matrix product,
+//   H[(z, c)][(x, i)] = sum_points (wz[z] v_c) (wx[x] d_i),
+// c: re, im; i: the component (the value v d_i has rank one), followed by
+// F(z, y, x) += wy[y] H for the W planes of the row.  A stamp of 6 x 6 cells fills 216 of
+// the 1024 products of a 32 x 32 block, but the sums stay in registers, where the vector
+// form walked the points one by one through read-modify-writes of an LDS box and then sent
+// every row's plane through memory (5.4 GB written, 6.7 GB read per launch at
+// (359, 71, 359) / 615): here only the finished planes go out, 42 instead of 308.
+//
+// Measured on MI355X, spread of one dataset with its y pass, per launch: (359, 71, 359) /
+// 615 x 615 x 360: 6.04 -> 3.39 ms; (179, 43, 179) / 305 x 305 x 180: 0.95 -> 0.58 ms;
+// (89, 21, 89) / 89 x 89 x 90: 0.112 -> 0.070 ms; grids whose tilt varies, (127, 31, 127) /
+// 181 x 181 x 120: 1.55 -> 0.50 ms.  fp32 matrix instructions and vector instructions share
+// the SIMD on gfx950 (measured: a wave of each side by side takes the sum of their times;
+// a bf16 one overlaps), so what bounds the kernel is their sum: 2.29e9 + 2.99e9 SIMD cycles
+// of the 7.0e9 of a launch at the largest shape.  Hence the 32 x 32 block of all components:
+// with one wave per component and 16 x 16 blocks the matrix part is half as much again, and
+// the launch took 3.65 ms against 2.9 ms.
+#include <algorithm>
+#include <cmath>
+#include <cstdlib>
+#include <type_traits>
+
+#include "nufft_point.h"
+#include "tiles.h"
+
+namespace lam {
+
+namespace {
+
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+constexpr int kBlock = 16;                 // matrix-core block edge
+constexpr int kRec = kBlock * 32;          // complex values of a tile's record of one plane
+constexpr unsigned kNoPoint = 0xffffffffu; // padding of a (tile, slot)
+
+// Components per matrix block and the x cells they leave room for: the 32 columns hold 10
+// cells of 3 components, or one component's 32 cells for the widest kernels.
+constexpr int tile_comps(int W) { return W <= 8 ? 3 : 1; }
+template <int NI>
+constexpr int kXCells = 32 / NI;
+
+// occupancy hint (waves per SIMD): what the W-plane window leaves room for without spills
+constexpr int spread_waves(int W) { return W <= 6 ? 3 : W <= 8 ? 2 : 1; }
+
+// y weights of a row slot and its first plane (unwrapped); direct plans use iy only
+struct RowY {
+    float w[12];
+    int iy, pad[3];
+};
+
+// ------------------------------------------------------------------ plan building
+// The points of a line cross a tile in one run of consecutive columns, so the points are
+// sorted as runs (about 10 points each) and not one by one.
+
+// Wave per 64 consecutive points of a line: the lanes where a new run starts, with its
+// bucket (tile, slot).  PASS 0 counts points and runs per bucket; PASS 1 stores the runs at
+// a cursor (their order inside the bucket is settled by k_run_expand).
+template <int PASS>
+__global__ __launch_bounds__(256) void k_tile_runs(const Geo *__restrict__ geo, long long nwaves, int R, int C,
+                                                   PointFrame fr, TileGeom tg, unsigned cpl,
+                                                   unsigned long long *__restrict__ count,
+                                                   const unsigned *__restrict__ roff, unsigned *__restrict__ cursor,
+                                                   uint2 *__restrict__ runs) {
+    const long long wave = blockIdx.x * 4ll + (threadIdx.x >> 6);
+    if (wave >= nwaves) return;
+    const int lane = threadIdx.x & 63;
+    const long long line = wave / cpl;
+    const int chunk = (int)(wave - line * cpl);
+    const int p = (int)(line / tg.Jn), j = (int)(line - (long long)p * tg.Jn);
+    const long long S = (long long)R * C, H = (S + 1) / 2;
+    const int k = chunk * 64 + lane;
+    const long long idx = (long long)j * C + k;
+    const bool ok = k < C && idx < H;
+    double tx, ty, tz;
+    point_coords(geo[p], fr, j, k, tx, ty, tz);
+    int bucket = -1;
+    if (ok) {
+        const int ix = wrap0(first_cell(tx, tg.nfx, fr.rx, tg.W), tg.nfx);
+        const int iz = wrap0(first_cell(tz, tg.nfz, fr.rz, tg.W), tg.nfz);
+        const unsigned tile = tg.fTz.div((unsigned)iz) * (unsigned)tg.ntx + tg.fTx.div((unsigned)ix);
+        const int slot = tg.direct ? wrap0(first_cell(ty, tg.nfy, fr.ry, tg.W), tg.nfy)
+                                   : (tg.dir > 0 ? j : tg.Jn - 1 - j);
+        bucket = (int)(tile * (unsigned)tg.nrho + (unsigned)slot);
+    }
+    const int prev = __shfl_up(bucket, 1);
+    const bool start = ok && (lane == 0 || bucket != prev);
+    const unsigned long long starts = __ballot(start), valid = __ballot(ok);
+    if (!start) return;
+    const unsigned long long after = lane == 63 ? 0ull : starts >> (lane + 1);
+    const int end = after ? lane + 1 + __builtin_ctzll(after) : __popcll(valid);
+    const unsigned len = (unsigned)(end - lane);
+    if constexpr (PASS == 0) {
+        atomicAdd(&count[bucket], (1ull << 32) | len);
+    } else {
+        const unsigned pos = roff[bucket] + atomicAdd(&cursor[bucket], 1u);
+        runs[pos] = make_uint2((unsigned)((long long)p * H + idx), len);
+    }
+}
+
+// Exclusive scans of the low and high words of counts (PAD: the low words rounded up to
+// multiples of 4, the buckets' padded point counts).
+constexpr int kScanItems = 8, kScanBlock = 256 * kScanItems;
+
+template <bool PAD>
+__device__ __forceinline__ uint2 scan_item(const unsigned long long *count, long long i, long long n) {
+    if (i >= n) return make_uint2(0u, 0u);
+    const unsigned long long c = count[i];
+    return make_uint2(PAD ? ((unsigned)c + 3u) & ~3u : (unsigned)c, (unsigned)(c >> 32));
+}
+
+// exclusive scan of one value per thread of a 256-thread block; total: the block's sum
+__device__ __forceinline__ uint2 block_scan(uint2 v, uint2 &total) {
+    __shared__ uint2 part[256];
+    const int t = threadIdx.x;
+    part[t] = v;
+    __syncthreads();
+    for (int s = 1; s < 256; s <<= 1) {
+        const uint2 o = t >= s ? part[t - s] : make_uint2(0u, 0u);
+        __syncthreads();
+        part[t].x += o.x;
+        part[t].y += o.y;
+        __syncthreads();
+    }
+    total = part[255];
+    const uint2 incl = part[t];
+    __syncthreads();
+    return make_uint2(incl.x - v.x, incl.y - v.y);
+}
+
+template <bool PAD>
+__global__ __launch_bounds__(256) void k_scan_sums(const unsigned long long *__restrict__ count, long long n,
+                                                   uint2 *__restrict__ sums) {
+    uint2 v = make_uint2(0u, 0u), total;
+    const long long i0 = blockIdx.x * (long long)kScanBlock + threadIdx.x * kScanItems;
+    for (int u = 0; u < kScanItems; ++u) {
+        const uint2 a = scan_item<PAD>(count, i0 + u, n);
+        v.x += a.x;
+        v.y += a.y;
+    }
+    block_scan(v, total);
+    if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+// one block: sums -> exclusive offsets, and the grand totals in sums[nb]
+__global__ __launch_bounds__(256) void k_scan_top(uint2 *__restrict__ sums, int nb) {
+    uint2 carry = make_uint2(0u, 0u);
+    for (int b0 = 0; b0 < nb; b0 += 256) {
+        const int b = b0 + threadIdx.x;
+        uint2 total;
+        const uint2 e = block_scan(b < nb ? sums[b] : make_uint2(0u, 0u), total);
+        if (b < nb) sums[b] = make_uint2(carry.x + e.x, carry.y + e.y);
+        carry.x += total.x;
+        carry.y += total.y;
+    }
+    if (threadIdx.x == 0) sums[nb] = carry;
+}
+
+template <bool PAD>
+__global__ __launch_bounds__(256) void k_scan_apply(const unsigned long long *__restrict__ count, long long n,
+                                                    const uint2 *__restrict__ sums, unsigned *__restrict__ lo,
+                                                    unsigned *__restrict__ hi) {
+    uint2 a[kScanItems], v = make_uint2(0u, 0u), total;
+    const long long i0 = blockIdx.x * (long long)kScanBlock + threadIdx.x * kScanItems;
+    for (int u = 0; u < kScanItems; ++u) {
+        a[u] = scan_item<PAD>(count, i0 + u, n);
+        v.x += a[u].x;
+        v.y += a[u].y;
+    }
+    uint2 e = block_scan(v, total);
+    const uint2 s = sums[blockIdx.x];
+    e.x += s.x;
+    e.y += s.y;
+    for (int u = 0; u < kScanItems; ++u) {
+        if (i0 + u > n) break;
+        lo[i0 + u] = e.x;   // entry n: the grand total
+        hi[i0 + u] = e.y;
+        e.x += a[u].x;
+        e.y += a[u].y;
+    }
+}
+
+// Wave per bucket: its runs in order of their first point number, written out as point ids.
+__global__ __launch_bounds__(256) void k_run_expand(const unsigned long long *__restrict__ count, long long nb,
+                                                    const unsigned *__restrict__ off,
+                                                    const unsigned *__restrict__ roff, const uint2 *__restrict__ runs,
+                                                    unsigned *__restrict__ ids) {
+    const long long b = blockIdx.x * 4ll + (threadIdx.x >> 6);
+    if (b >= nb) return;
+    const int lane = threadIdx.x & 63;
+    const unsigned long long c = count[b];
+    const unsigned n = (unsigned)(c >> 32), npts = (unsigned)c;
+    if (n == 0) return;
+    const unsigned base = off[b];
+    const uint2 *rb = runs + roff[b];
+    for (unsigned i0 = 0; i0 < n; i0 += 64) {
+        const uint2 mine = i0 + lane < n ? rb[i0 + lane] : make_uint2(kNoPoint, 0u);
+        unsigned pos = 0;
+        for (unsigned j0 = 0; j0 < n; j0 += 64) {
+            const uint2 o = j0 + lane < n ? rb[j0 + lane] : make_uint2(kNoPoint, 0u);
+            const int m = (int)min(64u, n - j0);
+            for (int t = 0; t < m; ++t) {
+                const unsigned kt = (unsigned)__builtin_amdgcn_readlane((int)o.x, t);
+                const unsigned lt = (unsigned)__builtin_amdgcn_readlane((int)o.y, t);
+                pos += kt < mine.x ? lt : 0u;
+            }
+        }
+        if (i0 + lane < n)
+            for (unsigned m = 0; m < mine.y; ++m) ids[base + pos + m] = mine.x + m;
+    }
+    const unsigned pad = (4u - (npts & 3u)) & 3u;
+    if ((unsigned)lane < pad) ids[base + npts + lane] = kNoPoint;
+}
+
+// Jobs of one tile: its points, in order, cut into equal parts of at most `most` (a row may be
+// cut too).  emit(i, beg, end, r0, r1): part i holds ids [beg, end) of slots [r0, r1).
+template <class F>
+__device__ __forceinline__ void tile_jobs(const unsigned *__restrict__ o, int nrho, unsigned most, F emit) {
+    const unsigned first = o[0], n = o[nrho] - first;
+    if (n == 0) return;
+    const unsigned parts = (n + most - 1) / most;
+    const unsigned step = ((n + parts - 1) / parts + 3u) & ~3u;
+    auto below = [&](unsigned v) {   // slots whose points start at or before v
+        int lo = 0, hi = nrho;
+        while (lo < hi) {
+            const int m = (lo + hi) / 2;
+            if (o[m] <= v) lo = m + 1;
+            else hi = m;
+        }
+        return lo;
+    };
+    for (unsigned i = 0; i * step < n; ++i) {
+        const unsigned beg = first + i * step, end = min(first + n, beg + step);
+        emit(i, beg, end, below(beg) - 1, below(end - 1));
+    }
+}
+
+// count[tile]: planes its jobs record (low word), jobs (high word)
+__global__ __launch_bounds__(64) void k_job_count(const unsigned *__restrict__ off, const RowY *__restrict__ rowy,
+                                                  unsigned ntiles, int nrho, int W, unsigned most,
+                                                  unsigned long long *__restrict__ count) {
+    const unsigned t = blockIdx.x * 64u + threadIdx.x;
+    if (t >= ntiles) return;
+    unsigned planes = 0, jobs = 0;
+    tile_jobs(off + (long long)t * nrho, nrho, most, [&](unsigned, unsigned, unsigned, int r0, int r1) {
+        planes += (unsigned)(rowy[r1 - 1].iy + W - rowy[r0].iy);
+        ++jobs;
+    });
+    count[t] = ((unsigned long long)jobs << 32) | planes;
+}
+
+__global__ __launch_bounds__(64) void k_job_emit(const unsigned *__restrict__ off, const RowY *__restrict__ rowy,
+                                                 unsigned ntiles, int nrho, int nfy, int W, unsigned most,
+                                                 const unsigned *__restrict__ plane0,
+                                                 const unsigned *__restrict__ job0, TileJob *__restrict__ jobs) {
+    const unsigned t = blockIdx.x * 64u + threadIdx.x;
+    if (t >= ntiles) return;
+    unsigned plane = plane0[t];
+    tile_jobs(off + (long long)t * nrho, nrho, most, [&](unsigned i, unsigned beg, unsigned end, int r0, int r1) {
+        TileJob j;
+        j.tile = t;
+        j.beg = beg;
+        j.end = end;
+        j.r0 = r0;
+        j.r1 = r1;
+        j.y0 = rowy[r0].iy;
+        j.np = rowy[r1 - 1].iy + W - j.y0;
+        j.plane = plane;
+        j.yw = j.y0 % nfy;
+        if (j.yw < 0) j.yw += nfy;
+        plane += (unsigned)j.np;
+        jobs[job0[t] + i] = j;
+    });
+}
+
+// ------------------------------------------------------------------ shared by both kernels
+// Walk over the non-empty row slots of a job: 64 slots' sizes sit in the lanes.
+struct SlotWalk {
+    const unsigned *off;   // the tile's first entry
+    unsigned beg, end;     // the job's ids
+    int next0, r1, base;   // first slot of the next block of 64; end; first slot of this block
+    int groups;            // lane: groups of 4 points of slot base + lane
+    unsigned long long mask;
+    __device__ __forceinline__ void start(const unsigned *tile_off, const TileJob &j) {
+        off = tile_off;
+        beg = j.beg;
+        end = j.end;
+        next0 = j.r0;
+        r1 = j.r1;
+        base = j.r0;
+        groups = 0;
+        mask = 0ull;
+    }
+    // the next non-empty slot and its number of groups; there is one
+    __device__ __forceinline__ int step(int lane, int &left) {
+        while (mask == 0ull && next0 < r1) {
+            base = next0;
+            next0 += 64;
+            const int r = base + lane;
+            groups = r < r1 ? (int)((min(off[r + 1], end) - max(off[r], beg)) >> 2) : 0;
+            mask = __ballot(groups > 0);
+        }
+        const int t = mask ? __builtin_ctzll(mask) : 0;
+        mask &= mask - 1ull;
+        left = __builtin_amdgcn_readlane(groups, t);
+        return base + t;
+    }
+};
+
+// The coordinate of one axis of a point, (qX u + qY v) s, as in point_coords.
+__device__ __forceinline__ double axis_coord(double qX, double qY, double u, double v, double s) {
+#pragma clang fp contract(off)
+    return (qX * u + qY * v) * s;
+}
+__device__ __forceinline__ double line_coord(double qY, double v, double s) {
+#pragma clang fp contract(off)
+    return (qY * v) * s;
+}
+__device__ __forceinline__ double detector_coord(int i, double centre, double step) {
+#pragma clang fp contract(off)
+    return ((double)i - centre) * step;
+}
+
+// A projection's geometry as the staging lanes read it: 16 bytes per axis, and float d_i.
+struct __attribute__((aligned(16))) TileGeo {
+    double uz, vz, ux, vx, vy, pad;
+    float d[4];
+};
+
+struct TileArgs {
+    long long S;
+    float b2;   // beta log2 e
+    PointFrame fr;
+    FastDiv fH, fC;
+};
+
+// ------------------------------------------------------------------ spreading
+// One wave per (job, component group).  Batches of 32 points are staged in LDS by
+// lane pairs: lane p < 32 evaluates the z weights of point p and writes wz (re v, im v) into
+// row p of A (32 entries (z, c), zero outside the stamp), lane p + 32 the x weights and
+// writes wx d_i into row p of B (entries (x, i)); the next batch's points are loaded
+// meanwhile.  Two points then take one v_mfma_f32_32x32x2_f32, rows (z, c) by columns (x, i).
+// After a row's points the block goes into the window of the W planes that later rows can
+// still reach, in registers; a plane that no later row reaches is written to the record.
+constexpr int kSPts = 32;                       // points per batch
+constexpr int kSRow = 34;                       // staged floats per row: 32, padded for the lanes' writes
+constexpr int kSHalf = (kSPts + 4) * kSRow;     // A, then B; 4 rows more are read ahead, never used
+
+template <int W, int NI, bool DIRECT>
+__global__ __launch_bounds__(64, spread_waves(W)) void k_tile_spread(
+    float2 *__restrict__ rec, const float2 *__restrict__ c, const TileGeo *__restrict__ geo,
+    const unsigned *__restrict__ off, const unsigned *__restrict__ ids, const RowY *__restrict__ rowy,
+    const TileJob *__restrict__ jobs, TileArgs A, TileGeom tg, unsigned plane0, int paired) {
+    __shared__ __attribute__((aligned(16))) float st_[2 * kSHalf];
+    __shared__ float sy[DIRECT ? (kSPts + 4) * W : 1];   // [point][plane]
+    constexpr int kGroups = 3 / NI;
+    const unsigned jn = blockIdx.x / kGroups;
+    const int grp = (int)(blockIdx.x - jn * kGroups);
+    const TileJob job = jobs[jn];
+    const unsigned tile = job.tile, beg = job.beg, end = job.end;
+    const unsigned *toff = off + (long long)tile * tg.nrho;
+    const int lane = threadIdx.x, pt = lane & 31, hi = lane >> 5;
+    const bool zl = lane < 32;
+    const int npts = (int)(end - beg), nbat = (npts + kSPts - 1) / kSPts;
+    const unsigned tz = tg.fntx.div(tile), tx = tile - tz * (unsigned)tg.ntx;
+    const int org = zl ? (int)tz * tg.Tz : (int)tx * tg.Tx;      // the axis this lane places points on
+    const int nf = zl ? tg.nfz : tg.nfx, lmax = (zl ? kBlock : kXCells<NI>) - W;
+    const double sc = zl ? A.fr.sz : A.fr.sx, rnf = zl ? A.fr.rz : A.fr.rx;
+    const double dnf = (double)nf;
+
+    struct Pt {
+        unsigned gid;
+        double u, v, vy;
+        float q[4];   // z lanes: c(q), c(-q); x lanes: d_i
+    };
+    auto load_id = [&](int bat) {
+        const int i = bat * kSPts + pt;
+        return i < npts ? ids[beg + i] : kNoPoint;
+    };
+    auto load_pt = [&](unsigned gid, Pt &t) {
+        t.gid = gid;
+        if (gid == kNoPoint) return;
+        const unsigned p = A.fH.div(gid);
+        const TileGeo *g = geo + p;
+        const double2 uv = *reinterpret_cast<const double2 *>(zl ? &g->uz : &g->ux);
+        t.u = uv.x;
+        t.v = uv.y;
+        if (DIRECT) t.vy = g->vy;
+        if (zl) {
+            const long long idx = gid - p * A.fH.d, mir = A.S - 1 - idx;
+            const float2 *pc = c + (long long)(paired ? p & ~1u : p) * A.S;
+            const float2 a = pc[idx], b = pc[mir];
+            t.q[0] = a.x;
+            t.q[1] = a.y;
+            t.q[2] = b.x;
+            t.q[3] = b.y;
+        } else {
+            const float4 d = *reinterpret_cast<const float4 *>(g->d);
+            t.q[0] = d.x;
+            t.q[1] = d.y;
+            t.q[2] = d.z;
+        }
+    };
+    auto stage = [&](const Pt &t) {
+        const bool have = t.gid != kNoPoint;
+        const unsigned gid = have ? t.gid : 0u;
+        const unsigned p = A.fH.div(gid), idx = gid - p * A.fH.d;
+        const unsigned j = A.fC.div(idx), k = idx - j * A.fC.d;
+        const double qY = detector_coord((int)j, A.fr.j0, A.fr.dY);
+        const double qX = detector_coord((int)k, A.fr.k0, A.fr.dX);
+        double x = axis_coord(qX, qY, t.u, t.v, sc);
+        const int i = first_cell(x, dnf, rnf, W);
+        float w[W];
+        es_weights2<W>(x, i, A.b2, w);
+        // i - org folded into the tile (i is in [-W / 2, nf]).  Inside it by the plan (same
+        // arithmetic); the clamp only bounds the LDS index.
+        int l = i - org;
+        l += l < 0 ? nf : 0;
+        l -= l >= nf ? nf : 0;
+        l = min(max(l, 0), lmax);
+        // the wave clears the batch and then writes the stamps (LDS keeps a wave's order)
+        const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int q = 0; q < (2 * kSHalf + 255) / 256; ++q)
+            if (q * 256 + lane * 4 < 2 * kSHalf) *reinterpret_cast<float4 *>(st_ + q * 256 + lane * 4) = z4;
+        if (have) {
+            if (zl) {
+                const float2 v = half_point_value(make_float2(t.q[0], t.q[1]), make_float2(t.q[2], t.q[3]), p, idx,
+                                                  A.S, paired);
+                float *row = st_ + pt * kSRow + 2 * l;
+#pragma unroll
+                for (int m = 0; m < W; ++m)
+                    *reinterpret_cast<float2 *>(row + 2 * m) = make_float2(w[m] * v.x, w[m] * v.y);
+            } else {
+                float *row = st_ + kSHalf + pt * kSRow + NI * l;
+                const float d[3] = {NI == 1 ? (grp == 0 ? t.q[0] : grp == 1 ? t.q[1] : t.q[2]) : t.q[0], t.q[1], t.q[2]};
+#pragma unroll
+                for (int m = 0; m < W; ++m)
+#pragma unroll
+                    for (int q = 0; q < NI; ++q) row[NI * m + q] = w[m] * d[q];
+            }
+        }
+        if constexpr (DIRECT) {
+            double y = line_coord(qY, t.vy, A.fr.sy);
+            const int iy = first_cell(y, (double)tg.nfy, A.fr.ry, W);
+            float wy[W];
+            es_weights2<W>(y, iy, A.b2, wy);
+            if (zl) {
+#pragma unroll
+                for (int m = 0; m < W; ++m) sy[pt * W + m] = have ? wy[m] : 0.f;
+            }
+        }
+    };
+
+    // block of the open row, and the window of W planes from yb
+    struct Plane {
+        float f[16];
+        __device__ __forceinline__ float &operator[](int r) { return f[r]; }
+    };
+    std::conditional_t<DIRECT, v16f, Plane> win[W];   // matrix accumulators, or plain sums
+    v16f h;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        h[r] = 0.f;
+#pragma unroll
+        for (int b = 0; b < W; ++b) win[b][r] = 0.f;
+    }
+    int yb = job.y0;
+    // the window's first plane to the record, the window on by one.  Lane (hi, n) register r
+    // holds row 8 (r / 4) + 4 hi + r % 4 = 2 z + c of column n.
+    auto flush = [&]() {
+        float2 *dst = rec + ((long long)(job.plane - plane0 + (unsigned)(yb - job.y0)) * kGroups + grp) * kRec +
+                      2 * hi * 32 + pt;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) dst[(4 * (t >> 1) + (t & 1)) * 32] = make_float2(win[0][2 * t], win[0][2 * t + 1]);
+#pragma unroll
+        for (int b = 0; b + 1 < W; ++b) win[b] = win[b + 1];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) win[W - 1][r] = 0.f;
+        ++yb;
+    };
+
+    SlotWalk walk;
+    walk.start(toff, job);
+    // groups of 4 points: of the open row, of the next row, of the rows not found yet
+    int left = 0, next_left = 0, todo = npts >> 2;
+    RowY ry{}, rn{};   // the next row's y weights are loaded while the open row's points go through
+    auto find_row = [&]() {
+        const int slot = walk.step(lane, next_left);
+        todo -= next_left;
+        rn = rowy[slot];
+    };
+    auto open_row = [&]() {
+        if constexpr (DIRECT) {
+            const int slot = walk.step(lane, left);
+            todo -= left;
+            while (yb < slot) flush();
+        } else {
+            ry = rn;
+            left = next_left;
+            next_left = 0;
+            if (todo > 0) find_row();
+        }
+    };
+    auto close_row = [&]() {
+        if constexpr (!DIRECT) {
+            while (yb < ry.iy) flush();
+#pragma unroll
+            for (int b = 0; b < W; ++b)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) win[b][r] += ry.w[b] * h[r];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) h[r] = 0.f;
+        }
+        if (DIRECT ? todo > 0 : next_left > 0) open_row();
+    };
+
+    Pt cur{};
+    load_pt(load_id(0), cur);
+    unsigned id1 = load_id(1);
+    if constexpr (!DIRECT) find_row();
+    open_row();
+    for (int k = 0; k < nbat; ++k) {
+        stage(cur);
+        load_pt(id1, cur);
+        id1 = load_id(k + 2);
+        const int ng = min(kSPts / 4, (npts - k * kSPts) >> 2);
+        const float *pa = st_ + hi * kSRow + pt, *pb = pa + kSHalf;
+        float a0 = pa[0], a1 = pa[2 * kSRow], b0 = pb[0], b1 = pb[2 * kSRow];
+        for (int g = 0; g < ng; ++g) {
+            pa += 4 * kSRow;
+            pb += 4 * kSRow;
+            if constexpr (DIRECT) {
+                const float ca0 = a0, ca1 = a1, cb0 = b0, cb1 = b1;
+                a0 = pa[0];
+                a1 = pa[2 * kSRow];
+                b0 = pb[0];
+                b1 = pb[2 * kSRow];
+                const float *wy = sy + (4 * g + hi) * W;
+#pragma unroll
+                for (int b = 0; b < W; ++b) {
+                    win[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(ca0 * wy[b], cb0, win[b], 0, 0, 0);
+                    win[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(ca1 * wy[2 * W + b], cb1, win[b], 0, 0, 0);
+                }
+            } else {
+                h = __builtin_amdgcn_mfma_f32_32x32x2f32(a0, b0, h, 0, 0, 0);
+                a0 = pa[0];
+                b0 = pb[0];
+                h = __builtin_amdgcn_mfma_f32_32x32x2f32(a1, b1, h, 0, 0, 0);
+                a1 = pa[2 * kSRow];
+                b1 = pb[2 * kSRow];
+            }
+            if (--left == 0) close_row();
+        }
+    }
+    while (yb < job.y0 + job.np) flush();
+}
+
+// Adds the jobs' records into the fine grid: every cell takes the blocks that reach it (its
+// own tile's and those of the tiles before it along z and x), in the order of the maps and of
+// a tile's jobs.  A thread owns one value (z, x, component) of kMergePlanes consecutive
+// planes, so that as many loads are in flight for each job it looks up.
+constexpr int kMergePlanes = 8;
+
+template <int NI>
+__global__ __launch_bounds__(256) void k_tile_merge(float2 *__restrict__ fine, const float2 *__restrict__ rec,
+                                                    const TileJob *__restrict__ jobs,
+                                                    const unsigned *__restrict__ job0, unsigned jfirst, unsigned jlast,
+                                                    unsigned plane0, const int *__restrict__ zmap,
+                                                    const int *__restrict__ xmap, TileGeom tg, int ylo, int ly,
+                                                    int add) {
+    const unsigned nxb = (unsigned)(3 * tg.nfx + 255) / 256u;   // workgroups: [plane chunk][z][x block]
+    const unsigned row = blockIdx.x / nxb, chunk = row / (unsigned)tg.nfz;
+    const int e = (int)((blockIdx.x - row * nxb) * 256 + threadIdx.x);
+    if (e >= 3 * tg.nfx) return;
+    const int x = (int)((unsigned)e / 3u), m = e - 3 * x;
+    const int z = (int)(row - chunk * (unsigned)tg.nfz);
+    const int yl0 = (int)chunk * kMergePlanes;
+    int y = ylo + yl0;
+    if (y >= tg.nfy) y -= tg.nfy;
+    float2 acc[kMergePlanes];
+#pragma unroll
+    for (int u = 0; u < kMergePlanes; ++u) acc[u] = make_float2(0.f, 0.f);
+    const int *ze = zmap + tg.nfz + 1, *xe = xmap + tg.nfx + 1;
+    for (int iz = zmap[z]; iz < zmap[z + 1]; ++iz) {
+        const unsigned trow = (unsigned)ze[2 * iz] * (unsigned)tg.ntx;
+        const int zc = ze[2 * iz + 1] * 32;
+        for (int ix = xmap[x]; ix < xmap[x + 1]; ++ix) {
+            const unsigned tile = trow + (unsigned)xe[2 * ix];
+            const int cell = zc + (NI == 3 ? 3 * xe[2 * ix + 1] + m : m * kRec + xe[2 * ix + 1]);
+            const unsigned j1 = min(job0[tile + 1], jlast);
+            for (unsigned j = max(job0[tile], jfirst); j < j1; ++j) {
+                const int np = jobs[j].np;
+                int d = y - jobs[j].yw;   // the job's plane at y, modulo the period
+                const float2 *r = rec + (long long)(jobs[j].plane - plane0) * ((3 / NI) * kRec) + cell;
+                float2 v[kMergePlanes];
+#pragma unroll
+                for (int u = 0; u < kMergePlanes; ++u) {
+                    if (d < 0) d += tg.nfy;
+                    if (d >= tg.nfy) d -= tg.nfy;
+                    v[u] = make_float2(0.f, 0.f);
+                    if (d < np) v[u] = r[(long long)d * ((3 / NI) * kRec)];
+                    if (d + tg.nfy < np) v[u] = cadd(v[u], r[(long long)(d + tg.nfy) * ((3 / NI) * kRec)]);
+                    ++d;
+                }
+#pragma unroll
+                for (int u = 0; u < kMergePlanes; ++u) acc[u] = cadd(acc[u], v[u]);
+            }
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kMergePlanes; ++u) {
+        if (yl0 + u < ly) {
+            float2 *dst = fine + ((long long)z * tg.nfy + y) * tg.nfx * 3 + e;
+            *dst = add ? cadd(*dst, acc[u]) : acc[u];
+        }
+        if (++y == tg.nfy) y = 0;
+    }
+}
+
+// ------------------------------------------------------------------ host
+#define LAM_TILE_WIDTH(w, CALL)                                            \
+    switch (w) {                                                           \
+        case 4: { constexpr int W = 4; CALL; } break;                      \
+        case 6: { constexpr int W = 6; CALL; } break;                      \
+        case 8: { constexpr int W = 8; CALL; } break;                      \
+        case 10: { constexpr int W = 10; CALL; } break;                    \
+        case 12: { constexpr int W = 12; CALL; } break;                    \
+        default: throw Error(LAM_ERR_NUFFT, "Error in finufft_makeplan: unsupported kernel width"); \
+    }
+
+// Tile edge of an axis of nf cells: a block of `cells` leaves cells + 1 - W first cells.  A
+// divisor within a tenth of that gives equal tiles; otherwise the widest tiles, evened out.
+int tile_edge(int nf, int W, int cells) {
+    const int widest = std::min(cells + 1 - W, nf);
+    for (int t = widest; 10 * t >= 9 * widest; --t)
+        if (nf % t == 0) return t;
+    const int nt = (nf + widest - 1) / widest;
+    return (nf + nt - 1) / nt;
+}
+
+TileGeom tile_geom(const int nf[3], int W, long long R, long long C, bool direct) {
+    TileGeom tg;
+    tg.W = W;
+    tg.nfz = nf[0];
+    tg.nfy = nf[1];
+    tg.nfx = nf[2];
+    tg.Tz = tile_edge(nf[0], W, kBlock);
+    tg.Tx = tile_edge(nf[2], W, 32 / tile_comps(W));
+    tg.ntz = (nf[0] + tg.Tz - 1) / tg.Tz;
+    tg.ntx = (nf[2] + tg.Tx - 1) / tg.Tx;
+    tg.ntiles = (unsigned)(tg.ntz * tg.ntx);
+    const long long H = (R * C + 1) / 2;
+    tg.Jn = (int)((H - 1) / C + 1);
+    tg.direct = direct ? 1 : 0;
+    tg.nrho = direct ? nf[1] : tg.Jn;
+    tg.fTz = FastDiv((unsigned)tg.Tz);
+    tg.fTx = FastDiv((unsigned)tg.Tx);
+    tg.fntx = FastDiv((unsigned)tg.ntx);
+    return tg;
+}
+
+// Whether the buckets and the padded point list (up to 3 fillers per non-empty bucket) have
+// 32-bit numbers.
+bool tile_fits(const TileGeom &tg, long long total) {
+    const long long nb = (long long)tg.ntiles * tg.nrho;
+    return nb < (1ll << 31) - kScanBlock && total + 3 * std::min(nb, total) < (1ll << 32);
+}
+
+// Points a job may hold.  Every job records W - 1 planes more than its rows have, and a wave
+// takes its points one batch after another, so the jobs are as large as the waves in flight
+// allow (3 per SIMD), within a range.  Measured, spread + merge in us: (89, 21, 89) / 89 with
+// 128, 256, 512 and 1024 points: 79, 67, 73, 83; (179, 43, 179) / 305 with 684, 1367, 2048:
+// 620, 578, 581; (359, 71, 359) / 615 with 4096, 5543, 8192: 3392, 3403, 3516.
+constexpr unsigned kJobMin = 384, kJobMax = 5120, kJobTarget = 6144;
+
+unsigned job_points(long long total) {
+    return (unsigned)std::max<long long>(kJobMin, std::min<long long>(kJobMax, total / kJobTarget)) & ~3u;
+}
+
+// (tile, block cell) pairs of every cell of an axis
+std::vector<int> axis_map(int nf, int T, int nt, int W) {
+    std::vector<std::vector<std::pair<int, int>>> m(nf);
+    for (int t = 0; t < nt; ++t) {
+        const int o = t * T, w = std::min(T, nf - o);
+        for (int i = 0; i < w + W - 1; ++i) m[(o + i) % nf].emplace_back(t, i);
+    }
+    std::vector<int> out(nf + 1);
+    for (int x = 0; x < nf; ++x) out[x + 1] = out[x] + (int)m[x].size();
+    for (int x = 0; x < nf; ++x)
+        for (auto &e : m[x]) {
+            out.push_back(e.first);
+            out.push_back(e.second);
+        }
+    return out;
+}
+
+void upload_vec(Ctx &cx, DevBuf &b, const std::vector<int> &v) {
+    b.alloc(sizeof(int) * v.size());
+    upload_now(cx, b.ptr, v.data(), sizeof(int) * v.size());
+}
+
+// bytes of one recorded plane of a job
+size_t record_bytes(const TileGeom &tg) { return (size_t)(3 / tile_comps(tg.W)) * kRec * sizeof(float2); }
+
+// Memory of the plane records of one group of jobs (LAMINO_NUFFT_SLAB_BYTES, default 8 GiB):
+// more jobs than it holds are spread and merged group by group.
+size_t record_budget() {
+    const char *e = std::getenv("LAMINO_NUFFT_SLAB_BYTES");
+    if (e && *e) {
+        const long long v = std::atoll(e);
+        if (v > 0) return (size_t)v;
+    }
+    return (size_t)8 << 30;
+}
+
+TileArgs tile_args(const Grid &g, const NufftPlan &pl) {
+    TileArgs a;
+    a.S = g.R * g.C;
+    a.b2 = (float)((double)pl.beta * 1.4426950408889634);
+    a.fr = point_frame(g, pl);
+    a.fH = FastDiv((unsigned)((a.S + 1) / 2));
+    a.fC = FastDiv((unsigned)g.C);
+    return a;
+}
+
+// y coordinate of detector row j of a shared-tilt grid, and its first plane (unwrapped)
+double row_coord(const Grid &g, const NufftPlan &pl, int j) {
+    const PointFrame fr = point_frame(g, pl);
+    const double qY = ((double)j - fr.j0) * fr.dY;
+    return (qY * g.geo_host[0].vy) * fr.sy;
+}
+int row_first(const Grid &g, const NufftPlan &pl, int j) {
+    return (int)std::ceil(row_coord(g, pl, j) - 0.5 * pl.w);
+}
+
+}  // namespace
+
+void row_window(const Grid &g, const NufftPlan &pl, int &ylo, int &ly) {
+    const long long H = (g.R * g.C + 1) / 2;
+    const int a = row_first(g, pl, 0), b = row_first(g, pl, (int)((H - 1) / g.C));
+    const int lo = std::min(a, b), len = std::max(a, b) + pl.w - lo;
+    ylo = ly = 0;
+    if (len < pl.nf[1]) {
+        ylo = ((lo % pl.nf[1]) + pl.nf[1]) % pl.nf[1];
+        ly = len;
+    }
+}
+
+bool tile_plan_fits(const Grid &g, const NufftPlan &pl, bool direct) {
+    return tile_fits(tile_geom(pl.nf, pl.w, g.R, g.C, direct), g.P * ((g.R * g.C + 1) / 2));
+}
+
+TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long R, long long C) {
+    NufftPlan pl;   // shapes only
+    pl.w = width_for_eps(eps);
+    for (int a = 0; a < 3; ++a) pl.nf[a] = (int)nufft_fine_len(dims[a], eps);
+    const size_t total = (size_t)P * (size_t)((R * C + 1) / 2);
+    TileBytes b;
+    for (const bool direct : {false, true}) {
+        const TileGeom tg = tile_geom(pl.nf, pl.w, R, C, direct);
+        const size_t nb = (size_t)tg.ntiles * tg.nrho, ids = total + 3 * std::min(nb, total);
+        const size_t jobs = tg.ntiles + ids / job_points((long long)total) + 1;
+        // a job's planes: its rows' first planes and W - 1 more; the half set spans at most half
+        // the period
+        const size_t planes = (size_t)tg.ntiles * (size_t)(direct ? tg.nfy : tg.nfy / 2 + 2) + jobs * (size_t)pl.w;
+        const size_t largest = record_bytes(tg) * ((size_t)tg.nfy + pl.w);   // of one job
+        b.kept = std::max(b.kept, 4 * (ids + nb + tg.ntiles) + sizeof(TileJob) * jobs + sizeof(TileGeo) * (size_t)P +
+                                      sizeof(RowY) * tg.nrho + 64 * (size_t)(tg.nfz + tg.nfx) + 4096);
+        // counts, run offsets and cursors per bucket, the runs, scan sums
+        b.setup = std::max(b.setup, 17 * nb + 8 * total + 32 * (size_t)tg.ntiles + 65536);
+        b.records = std::max(b.records, std::min(record_bytes(tg) * planes, std::max(record_budget(), largest)));
+    }
+    return b;
+}
+
+TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
+    std::vector<long long> key = {pl.nf[0], pl.nf[1], pl.nf[2], pl.w, direct ? 1 : 0};
+    auto it = g.tileplans.find(key);
+    if (it != g.tileplans.end()) return *it->second;
+    TimedScope ts(cx, "bin_points");
+    const long long S = g.R * g.C, H = (S + 1) / 2, total = g.P * H;
+    LAM_REQUIRE(total < (1ll << 31), LAM_ERR_ARG, "too many points in one polar grid for 32-bit bins");
+    auto tp = std::make_unique<TilePlan>();
+    TileGeom &tg = tp->tg;
+    tg = tile_geom(pl.nf, pl.w, g.R, g.C, direct);
+    const int W = pl.w, Jn = tg.Jn;
+    const long long nb = (long long)tg.ntiles * tg.nrho;
+    LAM_REQUIRE(tile_fits(tg, total), LAM_ERR_ARG, "fine grid too large for 32-bit point bins");
+    const PointFrame fr = point_frame(g, pl);
+
+    // Row slots: first planes, and for a shared tilt the y weights, from the same coordinate
+    // expression as the kernels (ty = (qY vy) sy), in double.  Unwrapped, the first plane of
+    // a detector row is linear in the row and so monotonic.
+    std::vector<RowY> rows(tg.nrho, RowY{});
+    if (direct) {
+        for (int r = 0; r < tg.nrho; ++r) rows[r].iy = r;
+    } else {
+        tg.dir = row_first(g, pl, Jn - 1) >= row_first(g, pl, 0) ? 1 : -1;
+        for (int r = 0; r < Jn; ++r) {
+            const int j = tg.dir > 0 ? r : Jn - 1 - r;
+            const double ty = row_coord(g, pl, j);
+            RowY &y = rows[r];
+            y.iy = row_first(g, pl, j);
+            for (int m = 0; m < W; ++m) {
+                const double z = ((double)(y.iy + m) - ty) * (2.0 / W);
+                const double rr = 1.0 - z * z;
+                y.w[m] = rr > 0 ? (float)std::exp((double)pl.beta * (std::sqrt(rr) - 1.0)) : 0.f;
+            }
+            LAM_REQUIRE(r == 0 || y.iy >= rows[r - 1].iy, LAM_ERR_STATE, "row first cells are not monotonic");
+        }
+        row_window(g, pl, tp->ylo, tp->ly);
+    }
+    tp->rowy.alloc(sizeof(RowY) * rows.size());
+    upload_now(cx, tp->rowy.ptr, rows.data(), sizeof(RowY) * rows.size());
+
+    std::vector<TileGeo> tgeo(g.P);
+    for (long long p = 0; p < g.P; ++p) {
+        const Geo &e = g.geo_host[p];
+        tgeo[p] = TileGeo{e.uz, e.vz, e.ux, e.vx, e.vy, 0.0, {(float)e.d0, (float)e.d1, (float)e.d2, 0.f}};
+    }
+    tp->geo.alloc(sizeof(TileGeo) * tgeo.size());
+    upload_now(cx, tp->geo.ptr, tgeo.data(), sizeof(TileGeo) * tgeo.size());
+
+    upload_vec(cx, tp->zmap, axis_map(tg.nfz, tg.Tz, tg.ntz, W));
+    upload_vec(cx, tp->xmap, axis_map(tg.nfx, tg.Tx, tg.ntx, W));
+
+    // points: runs counted per bucket, scanned, stored, ordered and written out
+    DevBuf count(sizeof(unsigned long long) * nb);
+    LAM_HIP(hipMemsetAsync(count.ptr, 0, count.bytes, cx.stream));
+    const unsigned cpl = (unsigned)((g.C + 63) / 64);
+    const long long nwaves = g.P * Jn * (long long)cpl;
+    const dim3 rgrid((unsigned)((nwaves + 3) / 4));
+    hipLaunchKernelGGL(k_tile_runs<0>, rgrid, dim3(256), 0, cx.stream, g.geo.as<Geo>(), nwaves, (int)g.R, (int)g.C, fr,
+                       tg, cpl, count.as<unsigned long long>(), (const unsigned *)nullptr, (unsigned *)nullptr,
+                       (uint2 *)nullptr);
+    check_launch();
+    const int nsb = (int)((nb + kScanBlock) / kScanBlock);   // covers entry nb too
+    DevBuf sums(sizeof(uint2) * (nsb + 1)), roff(sizeof(unsigned) * (nb + 1));
+    tp->off.alloc(sizeof(unsigned) * (nb + 1));
+    hipLaunchKernelGGL(k_scan_sums<true>, dim3(nsb), dim3(256), 0, cx.stream, count.as<unsigned long long>(), nb,
+                       sums.as<uint2>());
+    check_launch();
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, cx.stream, sums.as<uint2>(), nsb);
+    check_launch();
+    hipLaunchKernelGGL(k_scan_apply<true>, dim3(nsb), dim3(256), 0, cx.stream, count.as<unsigned long long>(), nb,
+                       sums.as<uint2>(), tp->off.as<unsigned>(), roff.as<unsigned>());
+    check_launch();
+    uint2 totals;
+    LAM_HIP(hipMemcpyAsync(&totals, sums.as<uint2>() + nsb, sizeof(totals), hipMemcpyDeviceToHost, cx.stream));
+    LAM_HIP(hipStreamSynchronize(cx.stream));
+    LAM_REQUIRE((long long)totals.x >= total && (long long)totals.y <= total, LAM_ERR_STATE,
+                "bin counts do not add up to the point count");
+    DevBuf runs(sizeof(uint2) * std::max<size_t>(totals.y, 1)), cursor(sizeof(unsigned) * nb);
+    tp->ids.alloc(sizeof(unsigned) * std::max<size_t>(totals.x, 1));
+    LAM_HIP(hipMemsetAsync(cursor.ptr, 0, cursor.bytes, cx.stream));
+    hipLaunchKernelGGL(k_tile_runs<1>, rgrid, dim3(256), 0, cx.stream, g.geo.as<Geo>(), nwaves, (int)g.R, (int)g.C, fr,
+                       tg, cpl, (unsigned long long *)nullptr, roff.as<unsigned>(), cursor.as<unsigned>(),
+                       runs.as<uint2>());
+    check_launch();
+    hipLaunchKernelGGL(k_run_expand, dim3((unsigned)((nb + 3) / 4)), dim3(256), 0, cx.stream,
+                       count.as<unsigned long long>(), nb, tp->off.as<unsigned>(), roff.as<unsigned>(),
+                       runs.as<uint2>(), tp->ids.as<unsigned>());
+    check_launch();
+    // jobs: counted per tile, scanned, written out
+    const unsigned most = job_points(total);
+    const int njb = (int)((tg.ntiles + (long long)kScanBlock) / kScanBlock);
+    DevBuf jcount(sizeof(unsigned long long) * tg.ntiles), jsums(sizeof(uint2) * (njb + 1)),
+        jplane(sizeof(unsigned) * (tg.ntiles + 1));
+    tp->job0.alloc(sizeof(unsigned) * (tg.ntiles + 1));
+    const dim3 jgrid((tg.ntiles + 63) / 64);
+    hipLaunchKernelGGL(k_job_count, jgrid, dim3(64), 0, cx.stream, tp->off.as<unsigned>(), tp->rowy.as<RowY>(),
+                       tg.ntiles, tg.nrho, W, most, jcount.as<unsigned long long>());
+    check_launch();
+    hipLaunchKernelGGL(k_scan_sums<false>, dim3(njb), dim3(256), 0, cx.stream, jcount.as<unsigned long long>(),
+                       (long long)tg.ntiles, jsums.as<uint2>());
+    check_launch();
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, cx.stream, jsums.as<uint2>(), njb);
+    check_launch();
+    hipLaunchKernelGGL(k_scan_apply<false>, dim3(njb), dim3(256), 0, cx.stream, jcount.as<unsigned long long>(),
+                       (long long)tg.ntiles, jsums.as<uint2>(), jplane.as<unsigned>(), tp->job0.as<unsigned>());
+    check_launch();
+    LAM_HIP(hipMemcpyAsync(&totals, jsums.as<uint2>() + njb, sizeof(totals), hipMemcpyDeviceToHost, cx.stream));
+    LAM_HIP(hipStreamSynchronize(cx.stream));
+    tp->planes = totals.x;
+    tp->njobs = totals.y;
+    tp->jobs.alloc(sizeof(TileJob) * std::max<size_t>(totals.y, 1));
+    hipLaunchKernelGGL(k_job_emit, jgrid, dim3(64), 0, cx.stream, tp->off.as<unsigned>(), tp->rowy.as<RowY>(),
+                       tg.ntiles, tg.nrho, tg.nfy, W, most, jplane.as<unsigned>(), tp->job0.as<unsigned>(),
+                       tp->jobs.as<TileJob>());
+    check_launch();
+    LAM_HIP(hipStreamSynchronize(cx.stream));   // the temporaries go
+    TilePlan &ref = *tp;
+    g.tileplans.emplace(std::move(key), std::move(tp));
+    return ref;
+}
+
+void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c, bool paired, bool add) {
+    const TileGeom &tg = tp.tg;
+    const size_t per_plane = record_bytes(tg), cap = std::max<size_t>(1, record_budget() / per_plane);
+    // groups of jobs (first job, first plane) whose records fit the budget; one job at least
+    std::vector<std::pair<unsigned, unsigned>> groups = {{0u, 0u}};
+    size_t most = tp.planes;
+    if (tp.planes > cap) {
+        std::vector<TileJob> jobs(tp.njobs);
+        LAM_HIP(hipMemcpyAsync(jobs.data(), tp.jobs.ptr, sizeof(TileJob) * jobs.size(), hipMemcpyDeviceToHost,
+                               cx.stream));
+        LAM_HIP(hipStreamSynchronize(cx.stream));
+        most = 0;
+        for (unsigned j = 0; j < tp.njobs; ++j) {
+            if (j > groups.back().first && jobs[j].plane + (unsigned)jobs[j].np - groups.back().second > cap)
+                groups.emplace_back(j, jobs[j].plane);
+            most = std::max<size_t>(most, jobs[j].plane + (unsigned)jobs[j].np - groups.back().second);
+        }
+    }
+    pl.rec.ensure(per_plane * most);
+    const TileArgs a = tile_args(g, pl);
+    const int ly = tp.ly > 0 ? tp.ly : tg.nfy, ylo = tp.ly > 0 ? tp.ylo : 0;
+    for (size_t k = 0; k < groups.size(); ++k) {
+        const unsigned j0 = groups[k].first, j1 = k + 1 < groups.size() ? groups[k + 1].first : tp.njobs;
+        if (j1 > j0) {
+            TimedScope ts(cx, "spread_rows2d");
+            const dim3 grid((j1 - j0) * (unsigned)(3 / tile_comps(pl.w)));
+#define LAM_TILE_SPREAD(DIRECT)                                                                                  \
+    LAM_TILE_WIDTH(pl.w, hipLaunchKernelGGL((k_tile_spread<W, tile_comps(W), DIRECT>), grid, dim3(64), 0, cx.stream, \
+                                            pl.rec.as<float2>(), c, tp.geo.as<TileGeo>(), tp.off.as<unsigned>(), \
+                                            tp.ids.as<unsigned>(), tp.rowy.as<RowY>(),                           \
+                                            tp.jobs.as<TileJob>() + j0, a, tg, groups[k].second, paired ? 1 : 0))
+            if (tg.direct) {
+                LAM_TILE_SPREAD(true);
+            } else {
+                LAM_TILE_SPREAD(false);
+            }
+#undef LAM_TILE_SPREAD
+            check_launch();
+        }
+        TimedScope ts(cx, "y_expand");
+        const dim3 mgrid((unsigned)((3 * tg.nfx + 255) / 256) * (unsigned)tg.nfz *
+                         (unsigned)((ly + kMergePlanes - 1) / kMergePlanes));
+        LAM_TILE_WIDTH(pl.w, hipLaunchKernelGGL((k_tile_merge<tile_comps(W)>), mgrid, dim3(256), 0, cx.stream,
+                                                pl.fine.as<float2>(), pl.rec.as<float2>(), tp.jobs.as<TileJob>(),
+                                                tp.job0.as<unsigned>(), j0, j1, groups[k].second, tp.zmap.as<int>(),
+                                                tp.xmap.as<int>(), tg, ylo, ly, add || k > 0 ? 1 : 0));
+        check_launch();
+    }
+}
+
+}  // namespace lam
