@@ -1836,6 +1836,12 @@ void launch_spread(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, bool half, 
 
 void launch_interp(Ctx &cx, Grid &g, NufftPlan &pl, float2 *c, bool half) {
     const int nc = half ? 3 : 1;
+    if (half && use_rows(g, pl) && tile_interp_fits(pl.w)) {
+        TilePlan &tp = get_tileplan(cx, g, pl, false);
+        TimedScope ts(cx, "interp");
+        tile_interp(cx, g, pl, tp, c);
+        return;
+    }
     if (half && use_rows(g, pl)) {
         RowPlan &rp = get_rowplan(cx, g, pl);
         TimedScope ts(cx, "interp");

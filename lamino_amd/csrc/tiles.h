@@ -29,6 +29,14 @@ struct TileJob {
     unsigned plane;
 };
 
+// A share of one unit's rows for one interpolating workgroup (a unit: a few tiles side by
+// side in x): the row slots [r0, r1), or part `part` of `parts` of one slot's points.
+struct UnitJob {
+    unsigned unit;
+    int r0, r1;
+    unsigned part, parts;
+};
+
 // Points of one grid ordered by (tile, row slot, point number), each (tile, slot) padded to
 // a multiple of 4 with kNoPoint.
 struct TilePlan {
@@ -41,6 +49,8 @@ struct TilePlan {
     DevBuf jobs;                   // TileJob [njobs], tile by tile
     DevBuf job0;                   // unsigned [ntiles + 1] first job of each tile
     unsigned njobs = 0, planes = 0;   // planes: recorded by all jobs
+    DevBuf ujobs;                  // UnitJob [nujobs]
+    unsigned nunits = 0, nujobs = 0;
     // cells of each axis as (tile, cell of its block) pairs: starts [nf + 1], then pairs
     DevBuf zmap, xmap;
 };
@@ -56,6 +66,11 @@ TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct);
 // fine (+)= the type-1 spread of the half point set.  add = false writes every plane of the
 // plan's window (every plane when ly is 0).
 void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c, bool paired, bool add);
+
+// c = the type-2 gather of the half point set and its mirror, for shared-tilt grids and the
+// kernel widths tile_interp_fits() names.
+bool tile_interp_fits(int w);
+void tile_interp(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, float2 *c);
 
 // Upper bounds of the device bytes of a plan (kept, and temporaries while it is built) and
 // of the plane records of its spread.

@@ -278,6 +278,60 @@ __global__ __launch_bounds__(64) void k_job_emit(const unsigned *__restrict__ of
     });
 }
 
+// Tiles of one interpolation unit, side by side in x: they share a block of 16 cells.
+constexpr int kUnitTiles = 2;
+
+// Interpolation jobs: a job takes whole row slots [r0, r1) of a unit, or part `part` of `parts`
+// of one slot that alone holds more than a job.
+template <class F>
+__device__ __forceinline__ void unit_jobs(const unsigned *__restrict__ off, unsigned u, const TileGeom &tg,
+                                          unsigned most, F emit) {
+    const int ut = kUnitTiles;
+    const unsigned nux = (unsigned)(tg.ntx + ut - 1) / (unsigned)ut, uz = u / nux, ux = u - uz * nux;
+    const unsigned *o = off + (long long)(uz * (unsigned)tg.ntx + (unsigned)ut * ux) * tg.nrho;
+    const int tiles = min(ut, tg.ntx - ut * (int)ux);
+    int r0 = -1, last = 0;   // last: one past the last slot with points
+    unsigned held = 0;
+    for (int r = 0; r < tg.nrho; ++r) {
+        unsigned n = 0;
+        for (int t = 0; t < tiles; ++t) n += o[t * tg.nrho + r + 1] - o[t * tg.nrho + r];
+        if (n == 0) continue;
+        if (r0 >= 0 && held + n > most) {
+            emit(r0, last, 0u, 1u);
+            r0 = -1;
+            held = 0;
+        }
+        if (n > most) {
+            const unsigned parts = (n + most - 1) / most;
+            for (unsigned k = 0; k < parts; ++k) emit(r, r + 1, k, parts);
+            continue;
+        }
+        if (r0 < 0) r0 = r;
+        held += n;
+        last = r + 1;
+    }
+    if (r0 >= 0) emit(r0, last, 0u, 1u);
+}
+
+__global__ __launch_bounds__(64) void k_unit_count(const unsigned *__restrict__ off, TileGeom tg, unsigned nunits,
+                                                   unsigned most, unsigned long long *__restrict__ count) {
+    const unsigned u = blockIdx.x * 64u + threadIdx.x;
+    if (u >= nunits) return;
+    unsigned jobs = 0;
+    unit_jobs(off, u, tg, most, [&](int, int, unsigned, unsigned) { ++jobs; });
+    count[u] = jobs;
+}
+
+__global__ __launch_bounds__(64) void k_unit_emit(const unsigned *__restrict__ off, TileGeom tg, unsigned nunits,
+                                                  unsigned most, const unsigned *__restrict__ job0,
+                                                  UnitJob *__restrict__ jobs) {
+    const unsigned u = blockIdx.x * 64u + threadIdx.x;
+    if (u >= nunits) return;
+    unsigned j = job0[u];
+    unit_jobs(off, u, tg, most,
+              [&](int r0, int r1, unsigned part, unsigned parts) { jobs[j++] = UnitJob{u, r0, r1, part, parts}; });
+}
+
 // ------------------------------------------------------------------ shared by both kernels
 // Walk over the non-empty row slots of a job: 64 slots' sizes sit in the lanes.
 struct SlotWalk {
@@ -623,6 +677,190 @@ __global__ __launch_bounds__(256) void k_tile_merge(float2 *__restrict__ fine, c
     }
 }
 
+// ------------------------------------------------------------------ interpolation
+// Type 2 of a shared-tilt grid: G(z, x) = sum_b wy[b] F(z, iy + b, x) for each row, then W^2
+// taps per point.  Workgroup per unit job.  A thread owns one cell of the unit's 16 x 16
+// block and keeps the W planes around the rows in registers (one more is loaded ahead); G of
+// several rows goes to LDS, and then the threads take those rows' points, one each.
+// Bound by LDS reads (108 of 8 bytes per point at W = 6; the banks collide 2.6-fold) over
+// vector work (1.4 ms of 2.5).  Before, G of all rows went through memory (1.17 ms to write it,
+// 2.04 ms to read and interpolate): 3.21 -> 2.46 ms per dataset at (359, 71, 359) / 615,
+// (179, 43, 179) / 305 0.45 -> 0.36, (89, 21, 89) / 89 0.047 -> 0.040.  The
+// same products on the fp32 matrix unit (16 x 16 blocks, 16 points at a time) took 4.5 ms.
+constexpr int kUnitThreads = 256;
+constexpr int kUnitRows = 8;                               // most rows staged at a time
+// Staged cells per block row.  The points of a line step through cells in every direction, so
+// a wave's reads fall on banks at random; measured at (359, 71, 359) / 615, per launch: 16 cells
+// (rows on the same banks) 4.18 ms, 17: 2.81, 18: 2.51, 19: 2.41, 21: 2.55.
+constexpr int kUnitRow = 19;
+constexpr int kUnitCells = kBlock * kUnitRow;              // staged cells per detector row
+
+template <int W>
+__global__ __launch_bounds__(kUnitThreads, 4) void k_tile_interp(
+    const float2 *__restrict__ fine, float2 *__restrict__ c, const TileGeo *__restrict__ geo,
+    const unsigned *__restrict__ off, const unsigned *__restrict__ ids, const RowY *__restrict__ rowy,
+    const UnitJob *__restrict__ jobs, TileArgs A, TileGeom tg, int nr) {
+    extern __shared__ float2 gs[];   // [nr][kUnitCells][3]
+    constexpr int kRowF = (W + 4) / 4 * 4;                         // floats per staged row: w[W], iy
+    __shared__ __attribute__((aligned(16))) float rw[2][kUnitRows * kRowF];   // y weights of a step's rows
+    constexpr int UT = kUnitTiles;
+    const UnitJob job = jobs[blockIdx.x];
+    const unsigned nux = (unsigned)(tg.ntx + UT - 1) / (unsigned)UT, uz = job.unit / nux, ux = job.unit - uz * nux;
+    const unsigned *o[UT];   // the unit's tiles (a missing one: no points)
+    int live[UT];
+#pragma unroll
+    for (int t = 0; t < UT; ++t) {
+        live[t] = UT * (int)ux + t < tg.ntx ? 1 : 0;
+        o[t] = off + (long long)(uz * (unsigned)tg.ntx + (unsigned)UT * ux + (live[t] ? t : 0)) * tg.nrho;
+    }
+    const int oz = (int)uz * tg.Tz, ox = UT * (int)ux * tg.Tx;
+    const int tid = threadIdx.x, cz = tid >> 4, cx = tid & 15;
+
+    float2 win[W][3], ahead[3];
+    int yb = rowy[job.r0].iy, yw = yb % tg.nfy;   // first plane of the window; the next to load (wrapped)
+    if (yw < 0) yw += tg.nfy;
+    const float2 *cell;
+    {
+        int z = oz + cz, x = ox + cx;
+        while (z >= tg.nfz) z -= tg.nfz;
+        while (x >= tg.nfx) x -= tg.nfx;
+        cell = fine + ((long long)z * tg.nfy * tg.nfx + x) * 3;
+    }
+    auto load_plane = [&](float2 *dst) {
+        const float2 *src = cell + (long long)yw * tg.nfx * 3;
+#pragma unroll
+        for (int m = 0; m < 3; ++m) dst[m] = src[m];
+        if (++yw == tg.nfy) yw = 0;
+    };
+#pragma unroll
+    for (int b = 0; b < W; ++b) load_plane(win[b]);
+    load_plane(ahead);
+
+    // thread (row, float) of a step's rows
+    auto load_row = [&](int r) {
+        const int q = tid / kRowF, f = tid - q * kRowF;
+        if (q >= nr || r + q >= job.r1) return 0.f;
+        const RowY *y = rowy + (r + q);
+        return f < W ? y->w[f] : __int_as_float(y->iy);
+    };
+    if (tid < nr * kRowF) rw[0][tid] = load_row(job.r0);
+    __syncthreads();
+    const double dnz = (double)tg.nfz, dnx = (double)tg.nfx;
+    int buf = 0;
+    for (int r = job.r0; r < job.r1; r += nr, buf ^= 1) {
+        const int rn = min(r + nr, job.r1);
+        unsigned first[UT], upto[UT], n = 0;   // tile t holds numbers [upto[t - 1], upto[t])
+#pragma unroll
+        for (int t = 0; t < UT; ++t) {
+            first[t] = o[t][r] - n;
+            n += live[t] ? o[t][rn] - o[t][r] : 0u;
+            upto[t] = n;
+        }
+        const unsigned lo = (unsigned)((unsigned long long)n * job.part / job.parts),
+                       hi = (unsigned)((unsigned long long)n * (job.part + 1) / job.parts);
+        auto load_id = [&](unsigned i) {
+            if (i >= hi) return kNoPoint;
+            unsigned f = first[0];
+#pragma unroll
+            for (int t = 1; t < UT; ++t) f = i >= upto[t - 1] ? first[t] : f;
+            return ids[f + i];
+        };
+        unsigned gid = load_id(lo + tid);
+        const float nrow = tid < nr * kRowF ? load_row(r + nr) : 0.f;
+        for (int q = n ? r : rn; q < rn; ++q) {
+            float w[kRowF];
+#pragma unroll
+            for (int f = 0; f < kRowF; f += 4)
+                *reinterpret_cast<float4 *>(w + f) = *reinterpret_cast<const float4 *>(&rw[buf][(q - r) * kRowF + f]);
+            unsigned held = 0;
+#pragma unroll
+            for (int t = 0; t < UT; ++t) held += live[t] ? o[t][q + 1] - o[t][q] : 0u;
+            if (held == 0) continue;
+            const int iy = __builtin_amdgcn_readfirstlane(__float_as_int(w[W]));
+            while (yb < iy) {
+#pragma unroll
+                for (int m = 0; m < 3; ++m) {
+#pragma unroll
+                    for (int b = 0; b + 1 < W; ++b) win[b][m] = win[b + 1][m];
+                    win[W - 1][m] = ahead[m];
+                }
+                ++yb;
+                load_plane(ahead);
+            }
+            float2 *g = gs + (size_t)((q - r) * kUnitCells + cz * kUnitRow + cx) * 3;
+#pragma unroll
+            for (int m = 0; m < 3; ++m) {
+                float2 s = make_float2(0.f, 0.f);
+#pragma unroll
+                for (int b = 0; b < W; ++b) {
+                    s.x += w[b] * win[b][m].x;
+                    s.y += w[b] * win[b][m].y;
+                }
+                g[m] = s;
+            }
+        }
+        if (tid < nr * kRowF) rw[buf ^ 1][tid] = nrow;
+        __syncthreads();
+        for (unsigned i = lo + tid; i < hi; i += kUnitThreads) {
+            if (i >= lo + kUnitThreads) gid = load_id(i);
+            if (gid == kNoPoint) continue;
+            const unsigned p = A.fH.div(gid), idx = gid - p * A.fH.d;
+            const unsigned j = A.fC.div(idx), k = idx - j * A.fC.d;
+            const TileGeo *ge = geo + p;
+            const double2 gz = *reinterpret_cast<const double2 *>(&ge->uz), gx = *reinterpret_cast<const double2 *>(&ge->ux);
+            const float4 d = *reinterpret_cast<const float4 *>(ge->d);
+            const double qY = detector_coord((int)j, A.fr.j0, A.fr.dY), qX = detector_coord((int)k, A.fr.k0, A.fr.dX);
+            double tz = axis_coord(qX, qY, gz.x, gz.y, A.fr.sz), tx = axis_coord(qX, qY, gx.x, gx.y, A.fr.sx);
+            const int iz = first_cell(tz, dnz, A.fr.rz, W), ix = first_cell(tx, dnx, A.fr.rx, W);
+            float wz[W], wx[W];
+            es_weights2<W>(tz, iz, A.b2, wz);
+            es_weights2<W>(tx, ix, A.b2, wx);
+            // folded into the unit; inside it by the plan, the clamps only bound the LDS index
+            int lz = iz - oz, lx = ix - ox;
+            lz += lz < 0 ? tg.nfz : 0;
+            lz -= lz >= tg.nfz ? tg.nfz : 0;
+            lx += lx < 0 ? tg.nfx : 0;
+            lx -= lx >= tg.nfx ? tg.nfx : 0;
+            lz = min(max(lz, 0), kBlock - W);
+            lx = min(max(lx, 0), kBlock - W);
+            const int slot = tg.dir > 0 ? (int)j : tg.Jn - 1 - (int)j;
+            const int row = min(max(slot - r, 0), nr - 1);
+            const float2 *g = gs + (size_t)(row * kUnitCells + lz * kUnitRow + lx) * 3;
+            float2 acc[3];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) acc[m] = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int a = 0; a < W; ++a) {
+                float2 ra[3];
+#pragma unroll
+                for (int m = 0; m < 3; ++m) ra[m] = make_float2(0.f, 0.f);
+#pragma unroll
+                for (int e = 0; e < W; ++e)
+#pragma unroll
+                    for (int m = 0; m < 3; ++m) {
+                        const float2 v = g[(a * kUnitRow + e) * 3 + m];
+                        ra[m].x += v.x * wx[e];
+                        ra[m].y += v.y * wx[e];
+                    }
+#pragma unroll
+                for (int m = 0; m < 3; ++m) {
+                    acc[m].x += ra[m].x * wz[a];
+                    acc[m].y += ra[m].y * wz[a];
+                }
+            }
+            float2 s;
+            s.x = d.x * acc[0].x + d.y * acc[1].x + d.z * acc[2].x;
+            s.y = d.x * acc[0].y + d.y * acc[1].y + d.z * acc[2].y;
+            const long long mir = A.S - 1 - (long long)idx;
+            if (mir == (long long)idx) s.y = 0.f;   // the transform of a real volume is real at q = 0
+            float2 *pc = c + (long long)p * A.S;
+            pc[idx] = s;
+            if (mir != (long long)idx) pc[mir] = cconj(s);
+        }
+        __syncthreads();
+    }
+}
+
 // ------------------------------------------------------------------ host
 #define LAM_TILE_WIDTH(w, CALL)                                            \
     switch (w) {                                                           \
@@ -651,7 +889,8 @@ TileGeom tile_geom(const int nf[3], int W, long long R, long long C, bool direct
     tg.nfy = nf[1];
     tg.nfx = nf[2];
     tg.Tz = tile_edge(nf[0], W, kBlock);
-    tg.Tx = tile_edge(nf[2], W, 32 / tile_comps(W));
+    // 10 cells of 3 components, and the tiles of a unit share the interpolation's 16 cells
+    tg.Tx = tile_edge(nf[2], W, tile_comps(W) == 1 ? 32 : W <= 6 ? std::min(10, (kBlock + 1 - W) / kUnitTiles + W - 1) : 10);
     tg.ntz = (nf[0] + tg.Tz - 1) / tg.Tz;
     tg.ntx = (nf[2] + tg.Tx - 1) / tg.Tx;
     tg.ntiles = (unsigned)(tg.ntz * tg.ntx);
@@ -681,6 +920,22 @@ constexpr unsigned kJobMin = 384, kJobMax = 5120, kJobTarget = 6144;
 
 unsigned job_points(long long total) {
     return (unsigned)std::max<long long>(kJobMin, std::min<long long>(kJobMax, total / kJobTarget)) & ~3u;
+}
+
+// Points an interpolation job may hold: a job loads W planes of its block before its first
+// point, and the launch should be several times the workgroups the chip holds (1280).
+// Measured in us, (256..4096 points, 8192 jobs) against (512..8192, 4096): (89, 21, 89) / 89
+// 39 and 49, (179, 43, 179) / 305 396 and 416, (359, 71, 359) / 615 2817 and 2959.
+unsigned unit_points(long long total) {
+    return (unsigned)std::max<long long>(256, std::min<long long>(4096, total / 8192));
+}
+
+// Rows staged at a time: about a workgroup's worth of points (256), and LDS for 5 workgroups
+// per CU where the rows are dense.  Measured in us with 4 and 8 rows: (89, 21, 89) / 89, 27
+// points per unit and row: 39 and 35; 96 x 24 x 100 / 128, W = 8, 13 points: 128 and 108;
+// (179, 43, 179) / 305, 42 points: 396 and 429; (359, 71, 359) / 615, 63 points: 2817 and 3113.
+int unit_rows(const TilePlan &tp, long long total) {
+    return total < 32ll * tp.nunits * tp.tg.nrho ? 8 : 4;
 }
 
 // (tile, block cell) pairs of every cell of an axis
@@ -894,6 +1149,32 @@ TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
                        tg.ntiles, tg.nrho, tg.nfy, W, most, jplane.as<unsigned>(), tp->job0.as<unsigned>(),
                        tp->jobs.as<TileJob>());
     check_launch();
+    if (tile_interp_fits(pl.w) && !direct) {
+        tp->nunits = (unsigned)tg.ntz * (unsigned)((tg.ntx + kUnitTiles - 1) / kUnitTiles);
+        const unsigned umost = unit_points(total);
+        const int nub = (int)((tp->nunits + (long long)kScanBlock) / kScanBlock);
+        DevBuf ucount(sizeof(unsigned long long) * tp->nunits), usums(sizeof(uint2) * (nub + 1)),
+            ujob(sizeof(unsigned) * (tp->nunits + 1)), uhigh(sizeof(unsigned) * (tp->nunits + 1));
+        const dim3 ugrid((tp->nunits + 63) / 64);
+        hipLaunchKernelGGL(k_unit_count, ugrid, dim3(64), 0, cx.stream, tp->off.as<unsigned>(), tg, tp->nunits, umost,
+                           ucount.as<unsigned long long>());
+        check_launch();
+        hipLaunchKernelGGL(k_scan_sums<false>, dim3(nub), dim3(256), 0, cx.stream, ucount.as<unsigned long long>(),
+                           (long long)tp->nunits, usums.as<uint2>());
+        check_launch();
+        hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, cx.stream, usums.as<uint2>(), nub);
+        check_launch();
+        hipLaunchKernelGGL(k_scan_apply<false>, dim3(nub), dim3(256), 0, cx.stream, ucount.as<unsigned long long>(),
+                           (long long)tp->nunits, usums.as<uint2>(), ujob.as<unsigned>(), uhigh.as<unsigned>());
+        check_launch();
+        LAM_HIP(hipMemcpyAsync(&totals, usums.as<uint2>() + nub, sizeof(totals), hipMemcpyDeviceToHost, cx.stream));
+        LAM_HIP(hipStreamSynchronize(cx.stream));
+        tp->nujobs = totals.x;
+        tp->ujobs.alloc(sizeof(UnitJob) * std::max<size_t>(totals.x, 1));
+        hipLaunchKernelGGL(k_unit_emit, ugrid, dim3(64), 0, cx.stream, tp->off.as<unsigned>(), tg, tp->nunits, umost,
+                           ujob.as<unsigned>(), tp->ujobs.as<UnitJob>());
+        check_launch();
+    }
     LAM_HIP(hipStreamSynchronize(cx.stream));   // the temporaries go
     TilePlan &ref = *tp;
     g.tileplans.emplace(std::move(key), std::move(tp));
@@ -948,6 +1229,31 @@ void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c,
                                                 tp.xmap.as<int>(), tg, ylo, ly, add || k > 0 ? 1 : 0));
         check_launch();
     }
+}
+
+// Wider kernels leave a unit few first cells (9 x 6 at W = 8), so that forming G costs more
+// than the points: 0.10 ms against the row slabs' 0.076 at (100, 24, 96) / 120 x 128, W = 8.
+bool tile_interp_fits(int w) { return w <= 6; }
+
+void tile_interp(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, float2 *c) {
+    const TileGeom &tg = tp.tg;
+    const TileArgs a = tile_args(g, pl);
+    TimedScope ts(cx, "interp_rows2d");
+    const int nr = unit_rows(tp, g.P * ((g.R * g.C + 1) / 2));
+    const size_t lds = (size_t)nr * kUnitCells * 3 * sizeof(float2);
+    auto allow = [&](auto k) {
+        if (lds > 64 * 1024)
+            LAM_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    };
+    allow(pl.w == 4 ? &k_tile_interp<4> : &k_tile_interp<6>);
+#define LAM_TILE_INTERP(WW)                                                                                         \
+    hipLaunchKernelGGL((k_tile_interp<WW>), dim3(tp.nujobs), dim3(kUnitThreads), lds, cx.stream, pl.fine.as<float2>(), \
+                       c, tp.geo.as<TileGeo>(), tp.off.as<unsigned>(), tp.ids.as<unsigned>(), tp.rowy.as<RowY>(),   \
+                       tp.ujobs.as<UnitJob>(), a, tg, nr)
+    if (pl.w == 4) LAM_TILE_INTERP(4);
+    else LAM_TILE_INTERP(6);
+#undef LAM_TILE_INTERP
+    check_launch();
 }
 
 }  // namespace lam

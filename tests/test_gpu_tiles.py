@@ -1,4 +1,4 @@
-"""The tiled matrix-core spreader at the sizes where its cutting can go wrong: fine grids
+"""The tiled spreader and interpolator at the sizes where its cutting can go wrong: fine grids
 shorter than a block, tiles that do not divide the axis, every kernel width, rows cut between
 jobs, and a record budget of one job, for shared-tilt grids (row slots) and for grids whose
 tilt varies (first-cell slots)."""
@@ -24,12 +24,12 @@ def _tol(eps):
 
 CASES = [((3, 2, 4), 5, 7, 3, 1e-5), ((13, 5, 7), 9, 10, 6, 1e-5), ((48, 6, 40), 20, 24, 9, 1e-5),
          ((10, 6, 14), 12, 13, 8, 1e-3), ((10, 6, 14), 12, 13, 8, 1e-6), ((10, 6, 14), 13, 12, 8, 1e-8),
-         ((10, 6, 14), 13, 13, 8, 1e-10), ((21, 9, 23), 31, 33, 150, 1e-5)]
+         ((10, 6, 14), 13, 13, 8, 1e-10), ((21, 9, 23), 31, 33, 150, 1e-5), ((21, 9, 23), 31, 33, 400, 1e-5)]
 
 
 @pytest.mark.parametrize("varying", [False, True])
 @pytest.mark.parametrize("dims,R,C,P,eps", CASES)
-def test_adjoint_over_tile_edges(dims, R, C, P, eps, varying):
+def test_projectors_over_tile_edges(dims, R, C, P, eps, varying):
     import lamino_amd as la
     import oracle as orc
 
@@ -41,6 +41,8 @@ def test_adjoint_over_tile_edges(dims, R, C, P, eps, varying):
     p = rng.standard_normal((P, R, C)).astype(np.float32)
     a = la.adjoint(p, pg, dims, eps=eps)
     assert _rel(a, orc.adjoint(p, dims, al, ga, eps=1e-12)) < _tol(eps)
+    m = rng.standard_normal((3,) + dims).astype(np.float32)
+    assert _rel(la.forward(m, pg, eps=eps), orc.forward(m, al, ga, R, C, eps=1e-12)) < _tol(eps)
 
 
 @pytest.mark.parametrize("varying", [False, True])
