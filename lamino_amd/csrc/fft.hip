@@ -3,6 +3,7 @@
 #include <algorithm>
 #include <complex>
 #include <cstdlib>
+#include <type_traits>
 #include <vector>
 
 #include "fastdiv.h"
@@ -171,12 +172,12 @@ __device__ __forceinline__ void dft(float2 *v) {
         const float s3 = 0.86602540378443864676f * sg;
         float2 a = v[0], b = v[1], c = v[2];
         float2 t1 = cadd(b, c);
-        float2 t2 = make_float2(a.x - 0.5f * t1.x, a.y - 0.5f * t1.y);
+        float2 t2 = make_float2(__builtin_fmaf(-0.5f, t1.x, a.x), __builtin_fmaf(-0.5f, t1.y, a.y));
         float2 d = csub(b, c);
-        float2 t3 = make_float2(-s3 * d.y, s3 * d.x);  // i * s3 * (b - c)
         v[0] = cadd(a, t1);
-        v[1] = cadd(t2, t3);
-        v[2] = csub(t2, t3);
+        // t2 +- i s3 d, fused explicitly: the rounding does not depend on how the two signs are merged
+        v[1] = make_float2(__builtin_fmaf(-s3, d.y, t2.x), __builtin_fmaf(s3, d.x, t2.y));
+        v[2] = make_float2(__builtin_fmaf(s3, d.y, t2.x), __builtin_fmaf(-s3, d.x, t2.y));
     } else if constexpr (R == 4) {
         float2 a = v[0], b = v[1], c = v[2], d = v[3];
         float2 s0 = cadd(a, c), s1 = csub(a, c), s2 = cadd(b, d), s3 = csub(b, d);
@@ -452,6 +453,172 @@ __device__ __forceinline__ bool tile_line(const KParams &P, int l, int o2base, i
     return true;
 }
 
+// The positions of a length-n line that are loaded (stored), as at most four ranges [a, b):
+// [0, nv) and [n - nv2, n), cut with the cyclic window [lo, lo + len) (len 0: none).  The loops
+// over the four stay rolled: unrolled, the load modes' code quadruples and spills.
+struct Ranges {
+    int a[4], b[4];
+    bool all;   // every position
+    __device__ __forceinline__ Ranges(int nv, int nv2, int lo, int len, int n) {
+        const int va[2] = {0, max(nv, n - nv2)}, vb[2] = {min(nv, n), n};
+        int wa[2] = {0, 0}, wb[2] = {n, 0};
+        if (len > 0) {
+            wa[0] = lo;
+            wb[0] = min(lo + len, n);
+            wb[1] = lo + len - n;
+        }
+        int count = 0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                a[2 * i + k] = max(va[i], wa[k]);
+                b[2 * i + k] = min(vb[i], wb[k]);
+                count += max(0, b[2 * i + k] - a[2 * i + k]);
+            }
+        all = count == n;
+    }
+    __device__ __forceinline__ int begin(int r) const { return r == 0 ? a[0] : r == 1 ? a[1] : r == 2 ? a[2] : a[3]; }
+    __device__ __forceinline__ int end(int r) const { return r == 0 ? b[0] : r == 1 ? b[1] : r == 2 ? b[2] : b[3]; }
+    __device__ __forceinline__ bool has(int m) const {
+        return (m >= a[0] && m < b[0]) || (m >= a[1] && m < b[1]) || (m >= a[2] && m < b[2]) || (m >= a[3] && m < b[3]);
+    }
+};
+
+// A thread's lines and positions.  INNER: it stays on line tid % L and takes every (NT / L)-th
+// position (the threads past a whole number of rows of L idle: one of 256 at L = 17, 16 at
+// L = 48), so that a row of the tile is loaded contiguously; otherwise a wave takes every
+// fourth line, its lanes along the line.  Positions are a constant step apart: an element costs
+// an addition to its address.  Numbering the tile's elements instead cost each of them two index
+// divisions, the range tests and a 64-bit product, about half of the vector instructions of
+// these passes, which kept 70 to 98 % of the issue slots busy at the larger grids: the passes of
+// the normal operator at 359 x 71 x 359 went from 1591 to 1408 us, those of the three-dataset
+// adjoint there (615 x 615 detector) from 3209 to 2927 us.
+template <int INNER, int NT>
+struct TileThread {
+    int l, l_step, row, rows;
+    __device__ __forceinline__ explicit TileThread(const KParams &P) {
+        if (INNER) {
+            rows = NT / P.L;
+            row = (int)P.fL.div(threadIdx.x);
+            l = row < rows ? (int)threadIdx.x - row * P.L : P.L;
+            l_step = P.L;
+        } else {
+            rows = 64;
+            row = (int)(threadIdx.x & 63);
+            l = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+            l_step = NT / 64;
+        }
+    }
+};
+
+// Loads the tile: each thread issues the global loads of kLoadBatch elements before it writes
+// any to LDS (one at a time, the passes ran at a latency-bound ~2 TB/s).  Positions outside the
+// ranges read as zero.
+template <int INNER, int NT, int MODE>
+__device__ __forceinline__ void load_tile(float2 *__restrict__ buf, const KParams &P, int kind, const Ranges &rg,
+                                          const long long *base_in, const short *pos, bool has2) {
+    constexpr bool CPLX = MODE == LD_COMPLEX || MODE == LD_COMPLEX_PAIR;
+    using T = std::conditional_t<CPLX, float2, float>;
+    const AxisPass &a = P.a;
+    const int L = P.L, M = P.m, N = P.n;
+    const TileThread<INNER, NT> tt(P);
+    for (int l = tt.l; l < L; l += tt.l_step) {
+        const long long lb = base_in[l];
+        if (lb < 0) continue;
+        auto put = [&](int mm, float2 v) {
+            int n = mm - a.rot_in;
+            n += n < 0 ? N : 0;
+            if (kind == KIND_BLUESTEIN) v = cmul(v, P.chirp[n]);
+            buf[lidx<INNER>(l, kind == KIND_RADER ? (int)pos[n] : n, L, M)] = v;
+        };
+#pragma unroll 1
+        for (int r = 0; r < 4; ++r) {
+            const int end = rg.end(r);
+            if (rg.begin(r) >= end) continue;
+            int mm = rg.begin(r) + tt.row;
+            const long long step = (long long)tt.rows * P.isn;
+            const T *p = static_cast<const T *>(a.in) + lb + (long long)mm * P.isn;
+            const T *p2 = static_cast<const T *>(a.in2) + lb + (long long)mm * P.isn;
+            for (; mm < end; mm += kLoadBatch * tt.rows, p += kLoadBatch * step, p2 += kLoadBatch * step) {
+                T v[kLoadBatch], w[kLoadBatch];
+#pragma unroll
+                for (int u = 0; u < kLoadBatch; ++u)
+                    if (mm + u * tt.rows < end) v[u] = p[u * step];
+                if constexpr (MODE == LD_REAL_PAIR || MODE == LD_COMPLEX_PAIR) {
+#pragma unroll
+                    for (int u = 0; u < kLoadBatch; ++u) {
+                        w[u] = T{};
+                        if (has2 && mm + u * tt.rows < end) w[u] = p2[u * step];
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kLoadBatch; ++u) {
+                    if (mm + u * tt.rows >= end) continue;
+                    float2 x;
+                    if constexpr (MODE == LD_COMPLEX) x = v[u];
+                    else if constexpr (MODE == LD_REAL) x = make_float2(v[u], 0.f);
+                    else if constexpr (MODE == LD_REAL_PAIR) x = make_float2(v[u], w[u]);
+                    else x = make_float2(v[u].x - w[u].y, v[u].y + w[u].x);
+                    put(mm + u * tt.rows, x);
+                }
+            }
+        }
+        if (!rg.all)
+            for (int mm = tt.row; mm < N; mm += tt.rows)
+                if (!rg.has(mm)) put(mm, make_float2(0.f, 0.f));
+    }
+}
+
+// Stores the tile, kLoadBatch LDS reads at a time.
+template <int INNER, int NT, int MODE>
+__device__ __forceinline__ void store_tile(const float2 *__restrict__ buf, const KParams &P, int kind,
+                                           const Ranges &rg, const long long *base_out, const short *pos, bool put2) {
+    using T = std::conditional_t<MODE == ST_COMPLEX, float2, float>;
+    const AxisPass &a = P.a;
+    const int L = P.L, M = P.m, N = P.n;
+    const TileThread<INNER, NT> tt(P);
+    for (int l = tt.l; l < L; l += tt.l_step) {
+        const long long lb = base_out[l];
+        if (lb < 0) continue;
+        auto position = [&](int mm) {
+            const int n = mm - a.rot_out;
+            return n < 0 ? n + N : n;
+        };
+#pragma unroll 1
+        for (int r = 0; r < 4; ++r) {
+            const int end = rg.end(r);
+            if (rg.begin(r) >= end) continue;
+            int mm = rg.begin(r) + tt.row;
+            const long long step = (long long)tt.rows * P.osn;
+            T *p = static_cast<T *>(a.out) + lb + (long long)mm * P.osn;
+            T *p2 = static_cast<T *>(a.out2) + lb + (long long)mm * P.osn;
+            for (; mm < end; mm += kLoadBatch * tt.rows, p += kLoadBatch * step, p2 += kLoadBatch * step) {
+                float2 v[kLoadBatch];
+#pragma unroll
+                for (int u = 0; u < kLoadBatch; ++u)
+                    if (mm + u * tt.rows < end) {
+                        const int n = position(mm + u * tt.rows);
+                        v[u] = buf[lidx<INNER>(l, kind == KIND_RADER ? (int)pos[N + n] : n, L, M)];
+                    }
+#pragma unroll
+                for (int u = 0; u < kLoadBatch; ++u) {
+                    if (mm + u * tt.rows >= end) continue;
+                    float2 x = v[u];
+                    if (kind == KIND_BLUESTEIN) x = cmul(x, P.chirp[position(mm + u * tt.rows)]);
+                    x.x *= a.scale;
+                    x.y *= a.scale;
+                    if constexpr (MODE == ST_COMPLEX) p[u * step] = x;
+                    else if constexpr (MODE == ST_IMAG) p[u * step] = x.y;
+                    else p[u * step] = x.x;
+                    if constexpr (MODE == ST_REAL_PAIR)
+                        if (put2) p2[u * step] = x.y;
+                }
+            }
+        }
+    }
+}
+
 // DQ != 0: the instantiation for qdirect plans with prime factor Q = DQ (the S-point
 // stages, then direct_q_stage); its own kernel so that the other plans' passes keep
 // their register allocation.
@@ -486,76 +653,12 @@ __global__ __launch_bounds__(NT, WAVES) void k_fft_axis(KParams P) {
         for (int i = threadIdx.x; i < 2 * N; i += blockDim.x) pos_lds[i] = P.pos_in[i];
     __syncthreads();
 
-    // Load: each thread computes the addresses of kLoadBatch elements, issues
-    // their global loads, and only then writes them to LDS, so that that many
-    // loads per thread are in flight (one at a time, the passes ran at a
-    // latency-bound ~2 TB/s).
-    const int LN = L * N;
-    for (int e0 = threadIdx.x; e0 < LN; e0 += kLoadBatch * NT) {
-        long long off[kLoadBatch];
-        int line[kLoadBatch], nidx[kLoadBatch];
-#pragma unroll
-        for (int u = 0; u < kLoadBatch; ++u) {
-            const int e = e0 + u * NT;
-            off[u] = -1;
-            line[u] = -1;
-            nidx[u] = 0;
-            if (e < LN) {
-                int l, n;
-                if (INNER) { n = (int)P.fL.div((unsigned)e); l = e - n * L; }
-                else { l = (int)P.fN.div((unsigned)e); n = e - l * N; }
-                int mm = n + a.rot_in;
-                if (mm >= N) mm -= N;
-                const long long lb = base_in[l];
-                if (lb >= 0 && (mm < nv || mm >= N - a.nv2) && in_window(mm, a.ld_lo, a.ld_len, N))
-                    off[u] = lb + (long long)mm * P.isn;
-                line[u] = l;
-                nidx[u] = n;
-            }
-        }
-        float2 val[kLoadBatch];
-#pragma unroll
-        for (int u = 0; u < kLoadBatch; ++u) val[u] = make_float2(0.f, 0.f);
-        if (a.ld_mode == LD_COMPLEX) {
-#pragma unroll
-            for (int u = 0; u < kLoadBatch; ++u)
-                if (off[u] >= 0) val[u] = static_cast<const float2 *>(a.in)[off[u]];
-        } else if (a.ld_mode == LD_REAL) {
-#pragma unroll
-            for (int u = 0; u < kLoadBatch; ++u)
-                if (off[u] >= 0) val[u].x = static_cast<const float *>(a.in)[off[u]];
-        } else if (a.ld_mode == LD_REAL_PAIR) {
-#pragma unroll
-            for (int u = 0; u < kLoadBatch; ++u)
-                if (off[u] >= 0) {
-                    val[u].x = static_cast<const float *>(a.in)[off[u]];
-                    if (has2) val[u].y = static_cast<const float *>(a.in2)[off[u]];
-                }
-        } else {
-            float2 sec[kLoadBatch];
-#pragma unroll
-            for (int u = 0; u < kLoadBatch; ++u) {
-                sec[u] = make_float2(0.f, 0.f);
-                if (off[u] >= 0) {
-                    val[u] = static_cast<const float2 *>(a.in)[off[u]];
-                    if (has2) sec[u] = static_cast<const float2 *>(a.in2)[off[u]];
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kLoadBatch; ++u) {
-                val[u].x -= sec[u].y;
-                val[u].y += sec[u].x;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kLoadBatch; ++u) {
-            if (line[u] >= 0) {
-                float2 v = val[u];
-                if (kind == KIND_BLUESTEIN) v = cmul(v, P.chirp[nidx[u]]);
-                const int p = kind == KIND_RADER ? (int)pos_lds[nidx[u]] : nidx[u];
-                buf[lidx<INNER>(line[u], p, L, M)] = v;
-            }
-        }
+    const Ranges rin(nv, a.nv2, a.ld_lo, a.ld_len, N), rout(ns, a.ns2, a.st_lo, a.st_len, N);
+    switch (a.ld_mode) {
+        case LD_COMPLEX: load_tile<INNER, NT, LD_COMPLEX>(buf, P, kind, rin, base_in, pos_lds, has2); break;
+        case LD_REAL: load_tile<INNER, NT, LD_REAL>(buf, P, kind, rin, base_in, pos_lds, has2); break;
+        case LD_REAL_PAIR: load_tile<INNER, NT, LD_REAL_PAIR>(buf, P, kind, rin, base_in, pos_lds, has2); break;
+        default: load_tile<INNER, NT, LD_COMPLEX_PAIR>(buf, P, kind, rin, base_in, pos_lds, has2); break;
     }
     if (kind == KIND_BLUESTEIN) {
         const int pad = M - N;
@@ -611,51 +714,11 @@ __global__ __launch_bounds__(NT, WAVES) void k_fft_axis(KParams P) {
         }
     }
 
-    // Store, kLoadBatch elements per thread at a time: their LDS reads are issued
-    // together, then their global stores.
-    for (int e0 = threadIdx.x; e0 < LN; e0 += kLoadBatch * NT) {
-        long long off[kLoadBatch];
-        int line[kLoadBatch], nidx[kLoadBatch];
-#pragma unroll
-        for (int u = 0; u < kLoadBatch; ++u) {
-            const int e = e0 + u * NT;
-            off[u] = -1;
-            line[u] = 0;
-            nidx[u] = 0;
-            if (e < LN) {
-                int l, n;
-                if (INNER) { n = (int)P.fL.div((unsigned)e); l = e - n * L; }
-                else { l = (int)P.fN.div((unsigned)e); n = e - l * N; }
-                int mm = n + a.rot_out;
-                if (mm >= N) mm -= N;
-                const long long lb = base_out[l];
-                if (lb >= 0 && (mm < ns || mm >= N - a.ns2) && in_window(mm, a.st_lo, a.st_len, N))
-                    off[u] = lb + (long long)mm * P.osn;
-                line[u] = l;
-                nidx[u] = n;
-            }
-        }
-        float2 val[kLoadBatch];
-#pragma unroll
-        for (int u = 0; u < kLoadBatch; ++u) {
-            const int p = kind == KIND_RADER ? (int)pos_lds[N + nidx[u]] : nidx[u];
-            val[u] = off[u] >= 0 ? buf[lidx<INNER>(line[u], p, L, M)] : make_float2(0.f, 0.f);
-        }
-#pragma unroll
-        for (int u = 0; u < kLoadBatch; ++u) {
-            if (off[u] < 0) continue;
-            float2 v = val[u];
-            if (kind == KIND_BLUESTEIN) v = cmul(v, P.chirp[nidx[u]]);
-            v.x *= a.scale;
-            v.y *= a.scale;
-            if (a.st_mode == ST_COMPLEX) static_cast<float2 *>(a.out)[off[u]] = v;
-            else if (a.st_mode == ST_REAL) static_cast<float *>(a.out)[off[u]] = v.x;
-            else if (a.st_mode == ST_IMAG) static_cast<float *>(a.out)[off[u]] = v.y;
-            else {
-                static_cast<float *>(a.out)[off[u]] = v.x;
-                if (put2) static_cast<float *>(a.out2)[off[u]] = v.y;
-            }
-        }
+    switch (a.st_mode) {
+        case ST_COMPLEX: store_tile<INNER, NT, ST_COMPLEX>(buf, P, kind, rout, base_out, pos_lds, put2); break;
+        case ST_REAL: store_tile<INNER, NT, ST_REAL>(buf, P, kind, rout, base_out, pos_lds, put2); break;
+        case ST_IMAG: store_tile<INNER, NT, ST_IMAG>(buf, P, kind, rout, base_out, pos_lds, put2); break;
+        default: store_tile<INNER, NT, ST_REAL_PAIR>(buf, P, kind, rout, base_out, pos_lds, put2); break;
     }
 }
 
