@@ -42,6 +42,16 @@ constexpr int kLoadBatch = 4;
 // 16 -> 48 took the 90-point passes of the benchmark grid from 94 to 76 us.
 constexpr int kInnerLines = 48;
 
+// A launch of fewer workgroups than kFillBlocks (three to a CU) halves its tiles, down to
+// kMinLines lines (64 bytes of a row, inner): with every workgroup in flight at once the pass
+// takes as long as one of them, and a smaller tile is loaded, transformed and stored sooner.
+// Passes of an 89 x 21 x 89 forward (270 to 1068 workgroups): 96.6 -> 80.1 us; of a 63 x 15 x 63
+// reconstruction job: 5.30 -> 4.49 ms; of CG at 179 x 43 x 179: 4.31 -> 4.22 ms.  Launches of one
+// thousand workgroups or more lose: with the line at 1024 that CG takes 4.37 ms, at 2048 4.63
+// and the small forward 87.1 us; 512 gives 4.31 ms.  With 16 lines as the least the small
+// passes gain nothing, with 4 they lose again (at 2048: 96.2 us).
+constexpr int kFillBlocks = 768, kMinLines = 8;
+
 // A set of nv equal sub-lines of the tile (prime-factor plans): sub-line v is
 // column c of tile line l (INNER: v = c * L + l, else v = l * C + c), and its
 // element t sits at position off + c * coff + t * str of line l.
@@ -1038,16 +1048,21 @@ void run_axis(Ctx &cx, const FftPlan &plan, AxisPass a) {
     P.chirp = plan.chirp.as<float2>();
     P.bhat = plan.bhat.as<float2>();
     const bool inner = a.ci > 1;
-    const int cap = std::max(1, std::min(kLdsComplex / plan.m, kMaxLines));
-    dim3 grid;
-    if (inner) {
-        P.Li = std::min({a.ci, cap, kInnerLines});
-        P.Lo = std::max(1, std::min(a.c2, cap / P.Li));
-        grid = dim3((unsigned)((a.ci + P.Li - 1) / P.Li), (unsigned)((a.c2 + P.Lo - 1) / P.Lo), (unsigned)a.c1);
-    } else {
+    int cap = std::max(1, std::min(kLdsComplex / plan.m, kMaxLines));
+    const auto tiles = [&](int lines) {
+        if (inner) {
+            P.Li = std::min({a.ci, lines, kInnerLines});
+            P.Lo = std::max(1, std::min(a.c2, lines / P.Li));
+            return dim3((unsigned)((a.ci + P.Li - 1) / P.Li), (unsigned)((a.c2 + P.Lo - 1) / P.Lo), (unsigned)a.c1);
+        }
         P.Li = 1;
-        P.Lo = std::min({a.c2, cap, 32});
-        grid = dim3((unsigned)((a.c2 + P.Lo - 1) / P.Lo), (unsigned)a.ci, (unsigned)a.c1);
+        P.Lo = std::min({a.c2, lines, 32});
+        return dim3((unsigned)((a.c2 + P.Lo - 1) / P.Lo), (unsigned)a.ci, (unsigned)a.c1);
+    };
+    dim3 grid = tiles(cap);
+    while ((long long)grid.x * grid.y * grid.z < kFillBlocks && cap >= 2 * kMinLines) {
+        cap /= 2;
+        grid = tiles(cap);
     }
     P.L = P.Li * P.Lo;
     LAM_REQUIRE(a.isn > -(1ll << 31) && a.isn < (1ll << 31) && a.osn > -(1ll << 31) && a.osn < (1ll << 31),

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("shape", [(1, 2, 1), (1, 1, 2), (3, 2, 47), (2, 3, 49), (1, 180, 35), (5, 90, 129), (129, 4, 5),
                                    (33, 5, 64), (2, 65, 256), (1, 256, 513), (7, 205, 50), (2, 53, 100), (1, 12, 3840),
-                                   (1, 3840, 2)])
+                                   (1, 3840, 2), (800, 6, 10)])
 @pytest.mark.parametrize("shifted", [False, True])
 def test_fft2_at_tile_edges(ctx, orc, shape, shifted):
     """Both axes' passes against a transform in 64 bits.  The bound is a single-precision
