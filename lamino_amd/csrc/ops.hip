@@ -218,7 +218,7 @@ __device__ __forceinline__ float dpot(float delta, float sigma_q, float sigma_qp
 // from v is the negated term seen from u (x_v − x_u = −(x_u − x_v) exactly). For δ = 0
 // (and NaN) dpot is the constant 2/(σ_q·0.001) from both ends. A workgroup takes a
 // (j, k) tile of kQJ−2 × kQK−2 interior voxels with a one-voxel halo and marches it
-// along i over kQPlanes planes. On each plane every voxel of the extended tile
+// along i over `planes` planes. On each plane every voxel of the extended tile
 // evaluates its 13 forward edges (o > 0 in (a, b, c) order: 9 to plane i+1, 4 in the
 // plane), keeps them for its own sum and puts the value its neighbour needs (negated
 // unless δ = 0) in LDS; each interior voxel then adds its 26 terms in
@@ -226,10 +226,16 @@ __device__ __forceinline__ float dpot(float delta, float sigma_q, float sigma_qp
 // edges to plane i, the plane's own in-plane edges). The sums are those of a per-voxel
 // loop over the 26 neighbours, bit for bit, with 13/26 of the FP64 powers plus the
 // halo's (0.61 of them for a full tile).
-constexpr int kQJ = 16, kQK = 32, kQPlanes = 16;
+constexpr int kQJ = 16, kQK = 32;
+// Planes per workgroup: kQPlanes (the first plane's backward edges are evaluated once more per
+// workgroup: 9/13 of a plane's powers), halved while the launch has fewer than kQFill workgroups,
+// one per CU: at 16 planes a workgroup takes 230 us, however small the volume.  One component of
+// 21 x 7 x 21: 141 -> 18 us, 63 x 15 x 63: 240 -> 30 us, 89 x 21 x 89: 235 -> 58 us, 127 x 31 x 127:
+// 243 -> 128 us.  Half and twice the line: 73 and 62 us at 89, 132 and 140 us at 127.
+constexpr int kQPlanes = 16, kQFill = 256;
 
 __global__ __launch_bounds__(kQJ * kQK) void k_qggmrf(Vol3 gv, CVol3 xv, int n1, int n2, int n3, float sigma_q,
-                                                    float sigma_qp, float p, int tiles_k) {
+                                                    float sigma_qp, float p, int tiles_k, int planes) {
     // one component per blockIdx.z: the three share one launch (no half-empty last round per component)
     const unsigned comp = blockIdx.z;
     float *g = comp == 0 ? gv.c[0] : comp == 1 ? gv.c[1] : gv.c[2];
@@ -241,7 +247,7 @@ __global__ __launch_bounds__(kQJ * kQK) void k_qggmrf(Vol3 gv, CVol3 xv, int n1,
     const int t = threadIdx.x, jj = t / kQK, kk = t % kQK;
     const int j = (blockIdx.x / tiles_k) * (kQJ - 2) + jj;  // the halo row/column is jj, kk = 0
     const int k = (blockIdx.x % tiles_k) * (kQK - 2) + kk;
-    const int i_lo = 1 + blockIdx.y * kQPlanes, i_hi = min(i_lo + kQPlanes, n1 - 1);
+    const int i_lo = 1 + blockIdx.y * planes, i_hi = min(i_lo + planes, n1 - 1);
     const bool inb = j < n2 && k < n3;
     const bool own = jj >= 1 && jj < kQJ - 1 && kk >= 1 && kk < kQK - 1 && j < n2 - 1 && k < n3 - 1;
     const long long s1 = (long long)n2 * n3;
@@ -631,14 +637,17 @@ void qggmrf3(Ctx &cx, const long long d[3], Vol3 g, CVol3 x, int ncomp, float si
     const float sqp = (float)std::pow((double)sigma, 2.0 - (double)p);
     if (d[0] < 3 || d[1] < 3 || d[2] < 3 || n == 0) return;  // no interior voxel
     const long long tiles_j = (d[1] - 2 + kQJ - 3) / (kQJ - 2), tiles_k = (d[2] - 2 + kQK - 3) / (kQK - 2);
-    const long long chunks = (d[0] - 2 + kQPlanes - 1) / kQPlanes;
+    int planes = kQPlanes;
+    const auto chunks_of = [&] { return (d[0] - 2 + planes - 1) / planes; };
+    while (planes > 1 && tiles_j * tiles_k * chunks_of() * ncomp < kQFill) planes /= 2;
+    const long long chunks = chunks_of();
     if (tiles_j * tiles_k > 0x7fffffffLL || chunks > 65535)
         throw Error(LAM_ERR_ARG, "qggmrf: volume too large for the tiled prior kernel");
     if (ncomp < 1 || ncomp > 3) throw Error(LAM_ERR_ARG, "qggmrf: 1 to 3 components");
     for (int c = 0; c < ncomp; ++c)
         if (!g.c[c] || !x.c[c]) throw Error(LAM_ERR_ARG, "qggmrf: null component");
     hipLaunchKernelGGL(k_qggmrf, dim3((unsigned)(tiles_j * tiles_k), (unsigned)chunks, (unsigned)ncomp),
-                       dim3(kQJ * kQK), 0, cx.stream, g, x, (int)d[0], (int)d[1], (int)d[2], sq, sqp, p, (int)tiles_k);
+                       dim3(kQJ * kQK), 0, cx.stream, g, x, (int)d[0], (int)d[1], (int)d[2], sq, sqp, p, (int)tiles_k, planes);
     check_launch();
 }
 
