@@ -28,6 +28,8 @@ constexpr int kRedBlocks = 1024;
 constexpr size_t kRedPartials = (size_t)kRedBlocks * kMaxRedTerms;
 void reduce_terms_dev(Ctx &cx, long long n, const RedTerm *terms, int nterms, double *out_dev,
                       double *partials = nullptr);
+// out_dev[q] = sum of partials[q * nblocks .. (q + 1) * nblocks), in a fixed order
+void sum_partials(Ctx &cx, const double *partials, int nblocks, int nterms, double *out_dev);
 float max_value(Ctx &cx, long long n, const float *a);
 // sum a*b in FP64 like reduce_terms, with its partial sums in a static device
 // array instead of context memory: no device allocation (n <= kNoAllocMaxElems)

@@ -86,14 +86,13 @@ __global__ __launch_bounds__(256) void k_reduce_nt(RedSpec s, double *partials) 
     }
 }
 
-// fixed-order final sum of the partials of each term
-__global__ __launch_bounds__(256) void k_reduce_final(const double *partials, int nblocks, int nterms, double *out) {
-    for (int q = 0; q < nterms; ++q) {
-        double acc = 0.0;
-        for (int b = threadIdx.x; b < nblocks; b += blockDim.x) acc += partials[(size_t)q * nblocks + b];
-        const double v = block_sum_256(acc);
-        if (threadIdx.x == 0) out[q] = v;
-    }
+// fixed-order final sum of the partials of term blockIdx.x
+__global__ __launch_bounds__(256) void k_reduce_final(const double *partials, int nblocks, double *out) {
+    const int q = blockIdx.x;
+    double acc = 0.0;
+    for (int b = threadIdx.x; b < nblocks; b += blockDim.x) acc += partials[(size_t)q * nblocks + b];
+    const double v = block_sum_256(acc);
+    if (threadIdx.x == 0) out[q] = v;
 }
 
 __global__ __launch_bounds__(256) void k_max_partial(const float *a, long long n, float *partials) {
@@ -368,6 +367,11 @@ unsigned vgrid(long long n) { return grid_for((size_t)n, 256, 1u << 16); }
 
 }  // namespace
 
+void sum_partials(Ctx &cx, const double *partials, int nblocks, int nterms, double *out_dev) {
+    hipLaunchKernelGGL(k_reduce_final, dim3((unsigned)nterms), dim3(256), 0, cx.stream, partials, nblocks, out_dev);
+    check_launch();
+}
+
 void reduce_terms_dev(Ctx &cx, long long n, const RedTerm *terms, int nterms, double *out_dev, double *partials) {
     LAM_REQUIRE(nterms >= 1 && nterms <= kMaxRedTerms, LAM_ERR_ARG, "bad reduction");
     RedSpec s;
@@ -387,8 +391,7 @@ void reduce_terms_dev(Ctx &cx, long long n, const RedTerm *terms, int nterms, do
         default: hipLaunchKernelGGL(k_reduce, dim3(kRedBlocks), dim3(256), 0, cx.stream, s, partials); break;
     }
     check_launch();
-    hipLaunchKernelGGL(k_reduce_final, dim3(1), dim3(256), 0, cx.stream, partials, kRedBlocks, nterms, out_dev);
-    check_launch();
+    sum_partials(cx, partials, kRedBlocks, nterms, out_dev);
 }
 
 void reduce_terms(Ctx &cx, long long n, const RedTerm *terms, int nterms, double *out_host) {

@@ -213,15 +213,6 @@ __global__ __launch_bounds__(256) void k_toep_quad(const float2 *__restrict__ za
     }
 }
 
-__global__ __launch_bounds__(256) void k_sum_partials(const double *partials, int nblocks, int nterms, double *out) {
-    for (int q = 0; q < nterms; ++q) {
-        double acc = 0.0;
-        for (int b = threadIdx.x; b < nblocks; b += blockDim.x) acc += partials[(size_t)q * nblocks + b];
-        const double v = block_sum_256(acc);
-        if (threadIdx.x == 0) out[q] = v;
-    }
-}
-
 __global__ __launch_bounds__(256) void k_add_c(float2 *a, const float2 *b, long long n) {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
         a[i] = cadd(a[i], b[i]);
@@ -476,8 +467,7 @@ void toep_quad_dev(Toep &t, CVol3 x, double *q_dev, double *partials) {
     hipLaunchKernelGGL(k_toep_quad, dim3(nb), dim3(256), 0, cx.stream, t.za.as<float2>(), t.zb.as<float2>(), s,
                        t.L[0], t.L[1], t.L[2], partials);
     check_launch();
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, cx.stream, partials, nb, 3 * t.ngrids, q_dev);
-    check_launch();
+    sum_partials(cx, partials, nb, 3 * t.ngrids, q_dev);
 }
 
 void toep_quad(Toep &t, CVol3 x, double *q_host) {
