@@ -24,7 +24,6 @@ Ctx::~Ctx() {
     nufft_plans.clear();
     for (DevBuf &w : work) w.release();
     red.release();
-    scal.release();
     if (stream) (void)hipStreamSynchronize(stream);
     if (stream && own_stream) (void)hipStreamDestroy(stream);
 }

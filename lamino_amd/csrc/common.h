@@ -127,6 +127,32 @@ struct DevBuf {
     template <class T> T *as() const { return static_cast<T *>(ptr); }
 };
 
+// Pinned host memory of a context that kernels write results to: a kernel's store is on the
+// host once the stream is synchronised, without a copy of its own.  Allocation and release keep
+// out of other threads' graph captures like DevBuf's.
+struct HostSums {
+    static constexpr int kCount = 64;
+    double *ptr = nullptr;
+    HostSums() = default;
+    HostSums(const HostSums &) = delete;
+    HostSums &operator=(const HostSums &) = delete;
+    ~HostSums() {
+        if (!ptr) return;
+        std::shared_lock<std::shared_mutex> lk(capture_mutex());
+        (void)hipHostFree(ptr);
+    }
+    double *get() {
+        if (!ptr) {
+            if (capturing_here()) throw Error(LAM_ERR_STATE, "host allocation inside a graph capture");
+            std::shared_lock<std::shared_mutex> lk(capture_mutex());
+            void *p = nullptr;
+            LAM_HIP(hipHostMalloc(&p, sizeof(double) * kCount));
+            ptr = static_cast<double *>(p);
+        }
+        return ptr;
+    }
+};
+
 struct FftPlan;     // fft.hip
 struct NufftPlan;   // nufft.hip
 struct Ctx;
@@ -166,7 +192,7 @@ struct Ctx {
     std::map<std::vector<long long>, std::array<int, 3>> bin_tune;
     // general scratch used by a single call at a time
     DevBuf red;        // FP64 reduction partials
-    DevBuf scal;       // small device scalar block
+    HostSums sums;     // results of blocking reductions
     DevBuf work[4];    // named workspaces (grow-only)
     ~Ctx();
 };

@@ -244,7 +244,6 @@ void Server::worker(int slot) {
         cx.nufft_plans.clear();
         for (DevBuf &w : cx.work) w.release();
         cx.red.release();
-        cx.scal.release();
         (void)hipStreamSynchronize(cx.stream);
         const size_t peak = tally->peak - base;
         const bool to_writer = st == LAM_OK && stage;

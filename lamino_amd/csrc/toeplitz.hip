@@ -1,5 +1,6 @@
 // Toeplitz normal operator: closed-form FP64 kernel build, packed real FFTs with
 // pruned zero padding, 3x3 spectral multiply, Parseval quadratic forms.
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 
@@ -472,10 +473,11 @@ void toep_quad_dev(Toep &t, CVol3 x, double *q_dev, double *partials) {
 
 void toep_quad(Toep &t, CVol3 x, double *q_host) {
     Ctx &cx = *t.cx;
-    cx.scal.ensure(sizeof(double) * 64);
-    toep_quad_dev(t, x, cx.scal.as<double>());
-    LAM_HIP(hipMemcpyAsync(q_host, cx.scal.ptr, sizeof(double) * 3 * t.ngrids, hipMemcpyDeviceToHost, cx.stream));
+    static_assert(3 * kMaxQuadGrids <= HostSums::kCount);
+    double *sums = cx.sums.get();
+    toep_quad_dev(t, x, sums);
     LAM_HIP(hipStreamSynchronize(cx.stream));
+    std::copy(sums, sums + 3 * t.ngrids, q_host);
 }
 
 }  // namespace lam
