@@ -205,7 +205,12 @@ __device__ __forceinline__ float dpot(float delta, float sigma_q, float sigma_qp
     const float C = 0.001f;
     const float ad = fabsf(delta);
     if (ad > 0.f) {
-        const float t1 = (float)(pow((double)ad, Q - (double)p) / (double)sigma_qp);
+        // |delta|^(2 - p) as 2^((2 - p) log2 |delta|), still in double: half of pow's FP64 instructions,
+        // which are what bounds the prior.  The exponent's rounding leaves the power within
+        // 300 * 2^-53 of itself, a millionth of t1's own rounding to float: of 900 000 values over
+        // |delta| from 1e-40 to 1e15 and p from 1 to 2.5 none changed.  One component of 359 x 71 x 359:
+        // 1325 -> 893 us.  The bound on the logarithm keeps 0 * log2(inf) at pow's inf^0 = 1.
+        const float t1 = (float)(exp2((Q - (double)p) * fmin(log2((double)ad), 1e300)) / (double)sigma_qp);
         const float t3 = C + t1;
         return (float)((double)(delta / (t3 * sigma_q)) * (Q - ((Q - (double)p) * (double)t1) / (double)t3));
     }
@@ -229,9 +234,10 @@ __device__ __forceinline__ float dpot(float delta, float sigma_q, float sigma_qp
 constexpr int kQJ = 16, kQK = 32;
 // Planes per workgroup: kQPlanes (the first plane's backward edges are evaluated once more per
 // workgroup: 9/13 of a plane's powers), halved while the launch has fewer than kQFill workgroups,
-// one per CU: at 16 planes a workgroup takes 230 us, however small the volume.  One component of
-// 21 x 7 x 21: 141 -> 18 us, 63 x 15 x 63: 240 -> 30 us, 89 x 21 x 89: 235 -> 58 us, 127 x 31 x 127:
-// 243 -> 128 us.  Half and twice the line: 73 and 62 us at 89, 132 and 140 us at 127.
+// one per CU: at 16 planes a workgroup takes 170 us, however small the volume.  One component of
+// 21 x 7 x 21 takes 14 us, 63 x 15 x 63 24 us, 89 x 21 x 89 41 us, 127 x 31 x 127 91 us, where all
+// took 170 us and more (measured before the powers became a third cheaper: 141 -> 18, 240 -> 30,
+// 235 -> 58 and 243 -> 128 us; half and twice the line: 73 and 62 us at 89, 132 and 140 at 127).
 constexpr int kQPlanes = 16, kQFill = 256;
 
 __global__ __launch_bounds__(kQJ * kQK) void k_qggmrf(Vol3 gv, CVol3 xv, int n1, int n2, int n3, float sigma_q,

@@ -23,3 +23,24 @@ def test_qggmrf_planes_match_oracle(ctx, orc, dims):
     want = orc.qggmrf(g, x, 1000.0, 1.2, prec=32)
     got = la.qggmrf(g.copy(), x, 1000.0, 1.2)
     assert np.max(np.abs(got - want)) <= 27 * 2**-23 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("p", [1.0, 1.2, 2.0, 2.5])
+@pytest.mark.parametrize("scale", [1e-30, 1e-3, 1e4])
+def test_qggmrf_powers_match_oracle(ctx, orc, p, scale):
+    """The power of a difference over its range and the exponents' (2 - p positive, zero and
+    negative), an infinite voxel among them: the same finite values within a last bit of each of
+    the 26 terms, and the same values that are not finite."""
+    import lamino_amd as la
+
+    say("qggmrf powers", p, scale)
+    rng = np.random.default_rng(12)
+    x = (rng.standard_normal((7, 9, 14)) * scale).astype(np.float32)
+    x[3, 4, 6] = np.inf
+    g = np.zeros_like(x)
+    with np.errstate(all="ignore"):
+        want = orc.qggmrf(g, x, 2.0, p, prec=32)
+    got = la.qggmrf(g.copy(), x, 2.0, p)
+    ok = np.isfinite(want)
+    assert np.array_equal(ok, np.isfinite(got)) and ok.sum() > ok.size // 2
+    assert np.max(np.abs(got[ok] - want[ok])) <= 27 * 2**-23 * np.max(np.abs(want[ok]))
