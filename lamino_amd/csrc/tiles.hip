@@ -393,6 +393,13 @@ struct TileArgs {
     FastDiv fH, fC;
 };
 
+// Orders a wave's LDS accesses before those that follow, across its lanes: the hardware keeps a
+// wave's order by itself, so this costs no instruction, but the compiler must not move them.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // ------------------------------------------------------------------ spreading
 // One wave per (job, component group).  Batches of 32 points are staged in LDS by
 // lane pairs: lane p < 32 evaluates the z weights of point p and writes wz (re v, im v) into
@@ -477,11 +484,13 @@ __global__ __launch_bounds__(64, spread_waves(W)) void k_tile_spread(
         l += l < 0 ? nf : 0;
         l -= l >= nf ? nf : 0;
         l = min(max(l, 0), lmax);
-        // the wave clears the batch and then writes the stamps (LDS keeps a wave's order)
+        // the wave clears the batch and then writes the stamps
+        wave_lds_order();   // after the last batch's reads
         const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
         for (int q = 0; q < (2 * kSHalf + 255) / 256; ++q)
             if (q * 256 + lane * 4 < 2 * kSHalf) *reinterpret_cast<float4 *>(st_ + q * 256 + lane * 4) = z4;
+        wave_lds_order();
         if (have) {
             if (zl) {
                 const float2 v = half_point_value(make_float2(t.q[0], t.q[1]), make_float2(t.q[2], t.q[3]), p, idx,
@@ -509,6 +518,7 @@ __global__ __launch_bounds__(64, spread_waves(W)) void k_tile_spread(
                 for (int m = 0; m < W; ++m) sy[pt * W + m] = have ? wy[m] : 0.f;
             }
         }
+        wave_lds_order();   // before other lanes read the stamps
     };
 
     // block of the open row, and the window of W planes from yb
