@@ -58,6 +58,11 @@ struct RowY {
 // The points of a line cross a tile in one run of consecutive columns, so the points are
 // sorted as runs (about 10 points each) and not one by one.
 
+// Launches of a wave per item stride over their items: a dimension of a launch holds fewer than
+// 2^32 threads, 2^26 waves, and a plan may have more lines and buckets than that.
+constexpr unsigned kMaxWaveBlocks = 1u << 20;
+dim3 wave_grid(long long items) { return dim3(grid_for((size_t)items, 4, kMaxWaveBlocks)); }
+
 // Wave per 64 consecutive points of a line: the lanes where a new run starts, with its
 // bucket (tile, slot).  PASS 0 counts points and runs per bucket; PASS 1 stores the runs at
 // a cursor (their order inside the bucket is settled by k_run_expand).
@@ -67,39 +72,39 @@ __global__ __launch_bounds__(256) void k_tile_runs(const Geo *__restrict__ geo, 
                                                    unsigned long long *__restrict__ count,
                                                    const unsigned *__restrict__ roff, unsigned *__restrict__ cursor,
                                                    uint2 *__restrict__ runs) {
-    const long long wave = blockIdx.x * 4ll + (threadIdx.x >> 6);
-    if (wave >= nwaves) return;
     const int lane = threadIdx.x & 63;
-    const long long line = wave / cpl;
-    const int chunk = (int)(wave - line * cpl);
-    const int p = (int)(line / tg.Jn), j = (int)(line - (long long)p * tg.Jn);
     const long long S = (long long)R * C, H = (S + 1) / 2;
-    const int k = chunk * 64 + lane;
-    const long long idx = (long long)j * C + k;
-    const bool ok = k < C && idx < H;
-    double tx, ty, tz;
-    point_coords(geo[p], fr, j, k, tx, ty, tz);
-    int bucket = -1;
-    if (ok) {
-        const int ix = wrap0(first_cell(tx, tg.nfx, fr.rx, tg.W), tg.nfx);
-        const int iz = wrap0(first_cell(tz, tg.nfz, fr.rz, tg.W), tg.nfz);
-        const unsigned tile = tg.fTz.div((unsigned)iz) * (unsigned)tg.ntx + tg.fTx.div((unsigned)ix);
-        const int slot = tg.direct ? wrap0(first_cell(ty, tg.nfy, fr.ry, tg.W), tg.nfy)
-                                   : (tg.dir > 0 ? j : tg.Jn - 1 - j);
-        bucket = (int)(tile * (unsigned)tg.nrho + (unsigned)slot);
-    }
-    const int prev = __shfl_up(bucket, 1);
-    const bool start = ok && (lane == 0 || bucket != prev);
-    const unsigned long long starts = __ballot(start), valid = __ballot(ok);
-    if (!start) return;
-    const unsigned long long after = lane == 63 ? 0ull : starts >> (lane + 1);
-    const int end = after ? lane + 1 + __builtin_ctzll(after) : __popcll(valid);
-    const unsigned len = (unsigned)(end - lane);
-    if constexpr (PASS == 0) {
-        atomicAdd(&count[bucket], (1ull << 32) | len);
-    } else {
-        const unsigned pos = roff[bucket] + atomicAdd(&cursor[bucket], 1u);
-        runs[pos] = make_uint2((unsigned)((long long)p * H + idx), len);
+    for (long long wave = blockIdx.x * 4ll + (threadIdx.x >> 6); wave < nwaves; wave += gridDim.x * 4ll) {
+        const long long line = wave / cpl;
+        const int chunk = (int)(wave - line * cpl);
+        const int p = (int)(line / tg.Jn), j = (int)(line - (long long)p * tg.Jn);
+        const int k = chunk * 64 + lane;
+        const long long idx = (long long)j * C + k;
+        const bool ok = k < C && idx < H;
+        double tx, ty, tz;
+        point_coords(geo[p], fr, j, k, tx, ty, tz);
+        int bucket = -1;
+        if (ok) {
+            const int ix = wrap0(first_cell(tx, tg.nfx, fr.rx, tg.W), tg.nfx);
+            const int iz = wrap0(first_cell(tz, tg.nfz, fr.rz, tg.W), tg.nfz);
+            const unsigned tile = tg.fTz.div((unsigned)iz) * (unsigned)tg.ntx + tg.fTx.div((unsigned)ix);
+            const int slot = tg.direct ? wrap0(first_cell(ty, tg.nfy, fr.ry, tg.W), tg.nfy)
+                                       : (tg.dir > 0 ? j : tg.Jn - 1 - j);
+            bucket = (int)(tile * (unsigned)tg.nrho + (unsigned)slot);
+        }
+        const int prev = __shfl_up(bucket, 1);
+        const bool start = ok && (lane == 0 || bucket != prev);
+        const unsigned long long starts = __ballot(start), valid = __ballot(ok);
+        if (!start) continue;
+        const unsigned long long after = lane == 63 ? 0ull : starts >> (lane + 1);
+        const int end = after ? lane + 1 + __builtin_ctzll(after) : __popcll(valid);
+        const unsigned len = (unsigned)(end - lane);
+        if constexpr (PASS == 0) {
+            atomicAdd(&count[bucket], (1ull << 32) | len);
+        } else {
+            const unsigned pos = roff[bucket] + atomicAdd(&cursor[bucket], 1u);
+            runs[pos] = make_uint2((unsigned)((long long)p * H + idx), len);
+        }
     }
 }
 
@@ -190,31 +195,31 @@ __global__ __launch_bounds__(256) void k_run_expand(const unsigned long long *__
                                                     const unsigned *__restrict__ off,
                                                     const unsigned *__restrict__ roff, const uint2 *__restrict__ runs,
                                                     unsigned *__restrict__ ids) {
-    const long long b = blockIdx.x * 4ll + (threadIdx.x >> 6);
-    if (b >= nb) return;
     const int lane = threadIdx.x & 63;
-    const unsigned long long c = count[b];
-    const unsigned n = (unsigned)(c >> 32), npts = (unsigned)c;
-    if (n == 0) return;
-    const unsigned base = off[b];
-    const uint2 *rb = runs + roff[b];
-    for (unsigned i0 = 0; i0 < n; i0 += 64) {
-        const uint2 mine = i0 + lane < n ? rb[i0 + lane] : make_uint2(kNoPoint, 0u);
-        unsigned pos = 0;
-        for (unsigned j0 = 0; j0 < n; j0 += 64) {
-            const uint2 o = j0 + lane < n ? rb[j0 + lane] : make_uint2(kNoPoint, 0u);
-            const int m = (int)min(64u, n - j0);
-            for (int t = 0; t < m; ++t) {
-                const unsigned kt = (unsigned)__builtin_amdgcn_readlane((int)o.x, t);
-                const unsigned lt = (unsigned)__builtin_amdgcn_readlane((int)o.y, t);
-                pos += kt < mine.x ? lt : 0u;
+    for (long long b = blockIdx.x * 4ll + (threadIdx.x >> 6); b < nb; b += gridDim.x * 4ll) {
+        const unsigned long long c = count[b];
+        const unsigned n = (unsigned)(c >> 32), npts = (unsigned)c;
+        if (n == 0) continue;
+        const unsigned base = off[b];
+        const uint2 *rb = runs + roff[b];
+        for (unsigned i0 = 0; i0 < n; i0 += 64) {
+            const uint2 mine = i0 + lane < n ? rb[i0 + lane] : make_uint2(kNoPoint, 0u);
+            unsigned pos = 0;
+            for (unsigned j0 = 0; j0 < n; j0 += 64) {
+                const uint2 o = j0 + lane < n ? rb[j0 + lane] : make_uint2(kNoPoint, 0u);
+                const int m = (int)min(64u, n - j0);
+                for (int t = 0; t < m; ++t) {
+                    const unsigned kt = (unsigned)__builtin_amdgcn_readlane((int)o.x, t);
+                    const unsigned lt = (unsigned)__builtin_amdgcn_readlane((int)o.y, t);
+                    pos += kt < mine.x ? lt : 0u;
+                }
             }
+            if (i0 + lane < n)
+                for (unsigned m = 0; m < mine.y; ++m) ids[base + pos + m] = mine.x + m;
         }
-        if (i0 + lane < n)
-            for (unsigned m = 0; m < mine.y; ++m) ids[base + pos + m] = mine.x + m;
+        const unsigned pad = (4u - (npts & 3u)) & 3u;
+        if ((unsigned)lane < pad) ids[base + npts + lane] = kNoPoint;
     }
-    const unsigned pad = (4u - (npts & 3u)) & 3u;
-    if ((unsigned)lane < pad) ids[base + npts + lane] = kNoPoint;
 }
 
 // Jobs of one tile: its points, in order, cut into equal parts of at most `most` (a row may be
@@ -1100,7 +1105,7 @@ TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
     LAM_HIP(hipMemsetAsync(count.ptr, 0, count.bytes, cx.stream));
     const unsigned cpl = (unsigned)((g.C + 63) / 64);
     const long long nwaves = g.P * Jn * (long long)cpl;
-    const dim3 rgrid((unsigned)((nwaves + 3) / 4));
+    const dim3 rgrid = wave_grid(nwaves);
     hipLaunchKernelGGL(k_tile_runs<0>, rgrid, dim3(256), 0, cx.stream, g.geo.as<Geo>(), nwaves, (int)g.R, (int)g.C, fr,
                        tg, cpl, count.as<unsigned long long>(), (const unsigned *)nullptr, (unsigned *)nullptr,
                        (uint2 *)nullptr);
@@ -1128,7 +1133,7 @@ TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
                        tg, cpl, (unsigned long long *)nullptr, roff.as<unsigned>(), cursor.as<unsigned>(),
                        runs.as<uint2>());
     check_launch();
-    hipLaunchKernelGGL(k_run_expand, dim3((unsigned)((nb + 3) / 4)), dim3(256), 0, cx.stream,
+    hipLaunchKernelGGL(k_run_expand, wave_grid(nb), dim3(256), 0, cx.stream,
                        count.as<unsigned long long>(), nb, tp->off.as<unsigned>(), roff.as<unsigned>(),
                        runs.as<uint2>(), tp->ids.as<unsigned>());
     check_launch();

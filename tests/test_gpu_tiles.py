@@ -58,3 +58,36 @@ def test_one_job_record_budget_changes_only_the_summation_order(monkeypatch, var
     monkeypatch.setenv("LAMINO_NUFFT_SLAB_BYTES", "1")
     # sums of at most a few thousand FP32 terms in another order
     assert _rel(la.adjoint(p, pg, dims), whole) < 1e-5
+
+
+def test_more_buckets_than_one_launch_has_waves(monkeypatch):
+    """2^26 waves are more than a launch holds.  1024 row slots over 67,200 tiles (a wide, flat
+    volume at kernel width 8) are 68.8 million buckets; the same call cut by first y cells has a
+    million.  Both orders sum at most a few thousand FP32 terms per cell."""
+    import lamino_amd as la
+
+    dims, R, C, P = (672, 4, 672), 2048, 8, 2
+    pg = la.PolarGrid.per_projection(np.full(P, np.radians(30.0)), np.array([0.3, 1.7]), R, C)
+    p = np.random.default_rng(19).standard_normal((P, R, C)).astype(np.float32)
+    say("many buckets")
+    rows = la.adjoint(p, pg, dims, eps=1e-6)
+    monkeypatch.setenv("LAMINO_NUFFT_ROWS", "0")
+    assert _rel(rows, la.adjoint(p, pg, dims, eps=1e-6)) < 1e-5
+
+
+def test_more_detector_lines_than_one_launch_has_waves():
+    """65,500 projections (an FFT launch takes up to 65,535 planes) of 1026 half rows are more than
+    2^26 lines, one wave each; the halves of the scan are below that, and their adjoints add up to the whole one's.  A job sums up to 5120 points
+    one after another in FP32, and about 330 jobs are summed per cell: 4 sqrt(5450) 2^-24."""
+    import lamino_amd as la
+
+    dims, R, C, P = (9, 5, 11), 2052, 1, 65500
+    ga = 2 * np.pi * np.arange(P) / P
+    p = np.random.default_rng(20).standard_normal((P, R, C), dtype=np.float32)
+    say("many lines")
+
+    def back(a, b):
+        pg = la.PolarGrid.per_projection(np.full(b - a, np.radians(30.0)), ga[a:b], R, C)
+        return la.adjoint(p[a:b], pg, dims)
+
+    assert _rel(back(0, P), back(0, P // 2) + back(P // 2, P)) < 4 * 5450**0.5 * 2**-24
