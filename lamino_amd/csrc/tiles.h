@@ -37,6 +37,13 @@ struct UnitJob {
     unsigned part, parts;
 };
 
+// Groups of consecutive jobs whose records fit a budget of `cap` planes, one job at least:
+// (first job, its first plane) of each, and the planes of the largest.
+struct JobGroups {
+    size_t cap = 0, most = 0;
+    std::vector<std::pair<unsigned, unsigned>> first;
+};
+
 // Points of one grid ordered by (tile, row slot, point number), each (tile, slot) padded to
 // a multiple of 4 with kNoPoint.
 struct TilePlan {
@@ -49,6 +56,8 @@ struct TilePlan {
     DevBuf jobs;                   // TileJob [njobs], tile by tile
     DevBuf job0;                   // unsigned [ntiles + 1] first job of each tile
     unsigned njobs = 0, planes = 0;   // planes: recorded by all jobs
+    std::vector<unsigned> job_plane;  // host: first plane of each job, once a budget needed groups
+    JobGroups groups;                 // of the budget last used
     DevBuf ujobs;                  // UnitJob [nujobs]
     unsigned nunits = 0, nujobs = 0;
     // cells of each axis as (tile, cell of its block) pairs: starts [nf + 1], then pairs

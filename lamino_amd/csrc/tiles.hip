@@ -1009,6 +1009,35 @@ int row_first(const Grid &g, const NufftPlan &pl, int j) {
     return (int)std::ceil(row_coord(g, pl, j) - 0.5 * pl.w);
 }
 
+// The plan's job groups under the present budget.  The list is kept: as long as the budget
+// stays what it was, spreading waits for nothing on the host and can be captured.
+const JobGroups &job_groups(Ctx &cx, TilePlan &tp) {
+    JobGroups &jg = tp.groups;
+    const size_t cap = std::max<size_t>(1, record_budget() / record_bytes(tp.tg));
+    if (cap == jg.cap) return jg;
+    if (tp.planes > cap && tp.job_plane.empty()) {
+        std::vector<TileJob> jobs(tp.njobs);
+        LAM_HIP(hipMemcpyAsync(jobs.data(), tp.jobs.ptr, sizeof(TileJob) * jobs.size(), hipMemcpyDeviceToHost,
+                               cx.stream));
+        LAM_HIP(hipStreamSynchronize(cx.stream));
+        tp.job_plane.reserve(jobs.size());
+        for (const TileJob &j : jobs) tp.job_plane.push_back(j.plane);
+    }
+    jg.first.assign(1, {0u, 0u});
+    jg.most = tp.planes;
+    if (tp.planes > cap) {
+        jg.most = 0;
+        for (unsigned j = 0; j < tp.njobs; ++j) {
+            const unsigned end = j + 1 < tp.njobs ? tp.job_plane[j + 1] : tp.planes;   // jobs' planes follow each other
+            if (j > jg.first.back().first && end - jg.first.back().second > cap)
+                jg.first.emplace_back(j, tp.job_plane[j]);
+            jg.most = std::max<size_t>(jg.most, end - jg.first.back().second);
+        }
+    }
+    jg.cap = cap;
+    return jg;
+}
+
 }  // namespace
 
 void row_window(const Grid &g, const NufftPlan &pl, int &ylo, int &ly) {
@@ -1198,23 +1227,10 @@ TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
 
 void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c, bool paired, bool add) {
     const TileGeom &tg = tp.tg;
-    const size_t per_plane = record_bytes(tg), cap = std::max<size_t>(1, record_budget() / per_plane);
-    // groups of jobs (first job, first plane) whose records fit the budget; one job at least
-    std::vector<std::pair<unsigned, unsigned>> groups = {{0u, 0u}};
-    size_t most = tp.planes;
-    if (tp.planes > cap) {
-        std::vector<TileJob> jobs(tp.njobs);
-        LAM_HIP(hipMemcpyAsync(jobs.data(), tp.jobs.ptr, sizeof(TileJob) * jobs.size(), hipMemcpyDeviceToHost,
-                               cx.stream));
-        LAM_HIP(hipStreamSynchronize(cx.stream));
-        most = 0;
-        for (unsigned j = 0; j < tp.njobs; ++j) {
-            if (j > groups.back().first && jobs[j].plane + (unsigned)jobs[j].np - groups.back().second > cap)
-                groups.emplace_back(j, jobs[j].plane);
-            most = std::max<size_t>(most, jobs[j].plane + (unsigned)jobs[j].np - groups.back().second);
-        }
-    }
-    pl.rec.ensure(per_plane * most);
+    const size_t per_plane = record_bytes(tg);
+    const JobGroups &jg = job_groups(cx, tp);
+    const auto &groups = jg.first;
+    pl.rec.ensure(per_plane * jg.most);
     const TileArgs a = tile_args(g, pl);
     const int ly = tp.ly > 0 ? tp.ly : tg.nfy, ylo = tp.ly > 0 ? tp.ylo : 0;
     for (size_t k = 0; k < groups.size(); ++k) {

@@ -91,3 +91,59 @@ def test_more_detector_lines_than_one_launch_has_waves():
         return la.adjoint(p[a:b], pg, dims)
 
     assert _rel(back(0, P), back(0, P // 2) + back(P // 2, P)) < 4 * 5450**0.5 * 2**-24
+
+
+@pytest.mark.parametrize("planes", [1, 40, 300])
+def test_adjoint_over_the_record_budget_can_be_captured(monkeypatch, planes):
+    """Once its plan is there, an adjoint whose records exceed the budget (groups of one job, and
+    of several) only launches kernels: it can be captured, and each replay gives the eager call's
+    bits for the input of the moment."""
+    import ctypes
+
+    import lamino_amd as la
+    from lamino_amd._lib import check
+
+    dims, R, C, P = (21, 9, 23), 31, 33, 150
+    monkeypatch.setenv("LAMINO_NUFFT_SLAB_BYTES", str(4096 * planes))   # a record of width 6: 512 complex values
+    say("captured adjoint", planes)
+    ctx = la.Context()
+    lib, stream = ctx.lib, ctypes.c_void_p(ctx.lib.lam_ctx_stream(ctx.h))
+    pg = la.PolarGrid.per_projection(np.full(P, np.radians(33.0)), 0.2 + 2 * np.pi * np.arange(P) / P, R, C, ctx=ctx)
+    proj, out = ctx.alloc((P, R, C)), ctx.alloc((3,) + dims)
+    rng = np.random.default_rng(21)
+    d = (ctypes.c_int64 * 3)(*dims)
+
+    def call():
+        check(lib.lam_adjoint(ctx.h, pg.h, d, 1e-5, ctypes.c_void_p(proj.ptr),
+                              *[ctypes.c_void_p(q) for q in out.comps()]))
+
+    def result():
+        ctx.sync()
+        got = out.download()
+        out.zero()
+        ctx.sync()
+        return got
+
+    proj.upload(rng.standard_normal((P, R, C)).astype(np.float32))
+    call()
+    ctx.sync()
+    graph, launch = ctypes.c_void_p(), ctypes.c_void_p()
+    assert lib.hipStreamBeginCapture(stream, 1) == 0   # this thread's calls
+    try:
+        call()
+    finally:
+        ended = lib.hipStreamEndCapture(stream, ctypes.byref(graph))
+    assert ended == 0
+    assert lib.hipGraphInstantiate(ctypes.byref(launch), graph, None, None, ctypes.c_size_t(0)) == 0
+    for _ in range(3):
+        proj.upload(rng.standard_normal((P, R, C)).astype(np.float32))
+        call()
+        want = result()
+        assert lib.hipGraphLaunch(launch, stream) == 0
+        assert np.array_equal(result(), want) and np.linalg.norm(want) > 0
+    ctx.sync()
+    lib.hipGraphExecDestroy(launch)
+    lib.hipGraphDestroy(graph)
+    monkeypatch.delenv("LAMINO_NUFFT_SLAB_BYTES")
+    call()
+    assert _rel(result(), want) < 1e-5   # the same sums in another order
