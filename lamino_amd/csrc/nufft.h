@@ -64,7 +64,6 @@ struct RowPlan {
     DevBuf wy;                         // float [Jn][W] row weights
     DevBuf iy;                         // int [Jn] unwrapped first y cell of each row
     std::vector<int> iy_host;          // the same on the host
-    DevBuf count;                      // unsigned [Jn][ntiles] points per (row, tile)
     DevBuf nz;                         // unsigned [ntiles][nzw]: bit j % 32 of word j / 32 set when (row j, tile) holds points
     int nzw = 0;
     DevBuf ids;                        // half-point ids sorted by (row, tile, first cell)

@@ -1402,11 +1402,31 @@ void allow_lds(K kernel, size_t bytes) {
     if (bytes > 64 * 1024) LAM_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
 }
 
-// Sorts the binned points: keys (bucket * cells + cell) of `total` points with
-// the per-bucket counts already on the host (hc) and on the device (count), into
+// Device temporaries of a bucket sort: the points' keys (bucket * cells + cell), per bucket the
+// count, its first point and a cursor, and the scattered points.  They sit in a buffer of the
+// plan that is large enough and holds nothing between calls, else in one allocation of their
+// own: on small grids a first pass's time is that of its allocations and waits.
+struct SortTmp {
+    DevBuf own;
+    unsigned *key, *count, *cursor, *offset;
+    unsigned long long *staged;
+    SortTmp(Ctx &cx, NufftPlan &pl, long long total, size_t nb) {
+        const size_t n = std::max<long long>(total, 1), bytes = 12 * n + 12 * nb;
+        const DevBuf *b = pl.slab.bytes >= bytes ? &pl.slab : pl.rec.bytes >= bytes ? &pl.rec : &own;
+        if (b == &own) own.alloc(bytes);
+        staged = b->as<unsigned long long>();
+        key = reinterpret_cast<unsigned *>(staged + n);
+        count = key + n;
+        cursor = count + nb;
+        offset = cursor + nb;
+        LAM_HIP(hipMemsetAsync(count, 0, 2 * sizeof(unsigned) * nb, cx.stream));
+    }
+};
+
+// Sorts the binned points, their keys and counts in t (hc: the counts on the host), into
 // point ids ordered by (bucket, cell, point index).  Returns the ids buffer; the keys are used up.
-DevBuf bucket_sort(Ctx &cx, const DevBuf &key, long long total, unsigned cells, const std::vector<unsigned> &hc,
-                   const DevBuf &count) {
+// Returns before the device is done: t lives until the stream has been waited for.
+DevBuf bucket_sort(Ctx &cx, SortTmp &t, long long total, unsigned cells, const std::vector<unsigned> &hc) {
     const size_t nb = hc.size();
     std::vector<unsigned> ho(nb);
     unsigned long long off = 0;
@@ -1415,26 +1435,21 @@ DevBuf bucket_sort(Ctx &cx, const DevBuf &key, long long total, unsigned cells, 
         off += hc[b];
     }
     LAM_REQUIRE((long long)off == total, LAM_ERR_STATE, "bin counts do not add up to the point count");
-    DevBuf offset(sizeof(unsigned) * nb), cursor(sizeof(unsigned) * nb);
-    DevBuf staged(sizeof(unsigned long long) * std::max<long long>(total, 1));
     DevBuf ids(sizeof(unsigned) * std::max<long long>(total, 1));
-    upload_now(cx, offset.ptr, ho.data(), sizeof(unsigned) * nb);
-    LAM_HIP(hipMemsetAsync(cursor.ptr, 0, cursor.bytes, cx.stream));
+    upload_now(cx, t.offset, ho.data(), sizeof(unsigned) * nb);
     const unsigned grid = grid_for((size_t)total, 256, 1u << 20);
-    hipLaunchKernelGGL(k_bin_scatter, dim3(grid), dim3(256), 0, cx.stream, key.as<unsigned>(), total, cells,
-                       offset.as<unsigned>(), cursor.as<unsigned>(), staged.as<unsigned long long>());
+    hipLaunchKernelGGL(k_bin_scatter, dim3(grid), dim3(256), 0, cx.stream, t.key, total, cells, t.offset, t.cursor,
+                       t.staged);
     check_launch();
     constexpr size_t kMaxBlocks = (size_t)1 << 30;
     const size_t lds = sizeof(unsigned) * cells;
     allow_lds(k_bin_order, lds);
     for (size_t b0 = 0; b0 < nb; b0 += kMaxBlocks) {
         const size_t nblk = std::min(kMaxBlocks, nb - b0);
-        hipLaunchKernelGGL(k_bin_order, dim3((unsigned)nblk), dim3(256), lds, cx.stream,
-                           staged.as<unsigned long long>(), offset.as<unsigned>(), count.as<unsigned>(),
-                           (unsigned)b0, cells, key.as<unsigned>(), ids.as<unsigned>());
+        hipLaunchKernelGGL(k_bin_order, dim3((unsigned)nblk), dim3(256), lds, cx.stream, t.staged, t.offset, t.count,
+                           (unsigned)b0, cells, t.key, ids.as<unsigned>());
         check_launch();
     }
-    LAM_HIP(hipStreamSynchronize(cx.stream));
     return ids;
 }
 
@@ -1448,29 +1463,27 @@ SortedPoints &get_bins(Ctx &cx, Grid &g, NufftPlan &pl, bool half, const BinPara
     const long long ntiles = (long long)bp.nt[0] * bp.nt[1] * bp.nt[2];
     const long long nkeys = ntiles * bp.T[0] * bp.T[1] * bp.T[2];
     LAM_REQUIRE(nkeys <= (1ll << 32), LAM_ERR_ARG, "fine grid too large for 32-bit bin keys");
-    DevBuf key0(sizeof(unsigned) * std::max<long long>(total, 1));
-    DevBuf count(sizeof(unsigned) * ntiles);
-    LAM_HIP(hipMemsetAsync(count.ptr, 0, count.bytes, cx.stream));
+    SortTmp tmp(cx, pl, total, (size_t)ntiles);
     const PointFrame fr = point_frame(g, pl);
     const unsigned grid = grid_for((size_t)total, 256, 1u << 20);
     const Geo *geo = g.geo.as<Geo>();
     if (half) {
         LAM_WIDTH_SWITCH(pl.w, hipLaunchKernelGGL((k_bin_keys<W, true>), dim3(grid), dim3(256), 0, cx.stream, geo, g.P,
                                                   (int)g.R, (int)g.C, pl.nf[0], pl.nf[1], pl.nf[2], fr, bp,
-                                                  key0.as<unsigned>(), count.as<unsigned>()));
+                                                  tmp.key, tmp.count));
     } else {
         LAM_WIDTH_SWITCH(pl.w, hipLaunchKernelGGL((k_bin_keys<W, false>), dim3(grid), dim3(256), 0, cx.stream, geo,
                                                   g.P, (int)g.R, (int)g.C, pl.nf[0], pl.nf[1], pl.nf[2], fr, bp,
-                                                  key0.as<unsigned>(), count.as<unsigned>()));
+                                                  tmp.key, tmp.count));
     }
     check_launch();
     std::vector<unsigned> hc(ntiles);
-    LAM_HIP(hipMemcpyAsync(hc.data(), count.ptr, sizeof(unsigned) * ntiles, hipMemcpyDeviceToHost, cx.stream));
+    LAM_HIP(hipMemcpyAsync(hc.data(), tmp.count, sizeof(unsigned) * ntiles, hipMemcpyDeviceToHost, cx.stream));
     LAM_HIP(hipStreamSynchronize(cx.stream));
     // order: tile, then first cell inside the tile, then point index (deterministic)
     auto sp = std::make_unique<SortedPoints>();
     sp->npoints = total;
-    sp->ids = bucket_sort(cx, key0, total, (unsigned)(bp.T[0] * bp.T[1] * bp.T[2]), hc, count);
+    sp->ids = bucket_sort(cx, tmp, total, (unsigned)(bp.T[0] * bp.T[1] * bp.T[2]), hc);
     std::vector<uint4> chunks;
     unsigned long long off = 0;
     for (long long t = 0; t < ntiles; ++t) {
@@ -1483,8 +1496,8 @@ SortedPoints &get_bins(Ctx &cx, Grid &g, NufftPlan &pl, bool half, const BinPara
         sp->chunks.alloc(sizeof(uint4) * chunks.size());
         LAM_HIP(hipMemcpyAsync(sp->chunks.ptr, chunks.data(), sizeof(uint4) * chunks.size(), hipMemcpyHostToDevice,
                                cx.stream));
-        LAM_HIP(hipStreamSynchronize(cx.stream));
     }
+    LAM_HIP(hipStreamSynchronize(cx.stream));   // the temporaries go
     SortedPoints &ref = *sp;
     g.bins.emplace(std::move(key), std::move(sp));
     return ref;
@@ -1634,19 +1647,17 @@ RowPlan &get_rowplan(Ctx &cx, Grid &g, NufftPlan &pl) {
     rp->iy_host = iyh;
 
     const long long ncount = (long long)rp->Jn * rg.ntiles;
-    DevBuf key0(sizeof(unsigned) * std::max<long long>(total, 1));
-    rp->count.alloc(sizeof(unsigned) * ncount);
-    LAM_HIP(hipMemsetAsync(rp->count.ptr, 0, rp->count.bytes, cx.stream));
+    SortTmp tmp(cx, pl, total, (size_t)ncount);
     const unsigned grid = grid_for((size_t)total, 256, 1u << 20);
     LAM_WIDTH_SWITCH(W, hipLaunchKernelGGL((k_bin_keys_rows<W>), dim3(grid), dim3(256), 0, cx.stream,
                                            g.geo.as<Geo>(), g.P, (int)g.R, (int)g.C, pl.nf[0], pl.nf[2], fr, rg,
-                                           key0.as<unsigned>(), rp->count.as<unsigned>()));
+                                           tmp.key, tmp.count));
     check_launch();
     std::vector<unsigned> hc(ncount);
-    LAM_HIP(hipMemcpyAsync(hc.data(), rp->count.ptr, sizeof(unsigned) * ncount, hipMemcpyDeviceToHost, cx.stream));
+    LAM_HIP(hipMemcpyAsync(hc.data(), tmp.count, sizeof(unsigned) * ncount, hipMemcpyDeviceToHost, cx.stream));
     LAM_HIP(hipStreamSynchronize(cx.stream));
     // order: row, tile, first (z, x) cell inside the tile, then point index (deterministic)
-    rp->ids = bucket_sort(cx, key0, total, (unsigned)(rg.Tz * rg.Tx), hc, rp->count);
+    rp->ids = bucket_sort(cx, tmp, total, (unsigned)(rg.Tz * rg.Tx), hc);
     // one chunk per non-empty (row, tile): its workgroup alone writes that tile's
     // interior and halo record
     std::vector<uint4> chunks;
@@ -1676,8 +1687,8 @@ RowPlan &get_rowplan(Ctx &cx, Grid &g, NufftPlan &pl) {
         rp->chunks.alloc(sizeof(uint4) * chunks.size());
         LAM_HIP(hipMemcpyAsync(rp->chunks.ptr, chunks.data(), sizeof(uint4) * chunks.size(), hipMemcpyHostToDevice,
                                cx.stream));
-        LAM_HIP(hipStreamSynchronize(cx.stream));
     }
+    LAM_HIP(hipStreamSynchronize(cx.stream));   // the temporaries go
     RowPlan &ref = *rp;
     g.rowplans.emplace(std::move(key), std::move(rp));
     return ref;

@@ -5,6 +5,9 @@
 
 namespace lam {
 
+struct TileGeo;   // tiles.hip
+struct RowY;
+
 // Cutting of the (z, x) plane into tiles whose first-cell edges Tz x Tx leave room for the
 // kernel inside one 16 x 16 matrix-core block (T + W - 1 <= 16).  Tile (tz, tx) owns the
 // points whose first kernel cell lies in [tz Tz, (tz + 1) Tz) x [tx Tx, (tx + 1) Tx).
@@ -49,19 +52,19 @@ struct JobGroups {
 struct TilePlan {
     TileGeom tg;
     int ylo = 0, ly = 0;           // the y planes touched: [ylo, ylo + ly) mod nfy (ly 0: all)
-    DevBuf off;                    // unsigned [ntiles * nrho + 1] first id of each (tile, slot)
-    DevBuf ids;                    // point numbers
-    DevBuf rowy;                   // RowY [nrho]
-    DevBuf geo;                    // TileGeo [P]
-    DevBuf jobs;                   // TileJob [njobs], tile by tile
-    DevBuf job0;                   // unsigned [ntiles + 1] first job of each tile
     unsigned njobs = 0, planes = 0;   // planes: recorded by all jobs
+    unsigned nunits = 0, nujobs = 0;
+    DevBuf fixed, index, ids, shares;   // what the pointers below point into
+    const TileGeo *geo = nullptr;       // [P]
+    const RowY *rowy = nullptr;         // [nrho]
+    // cells of each axis as (tile, cell of its block) pairs: starts [nf + 1], then pairs
+    const int *zmap = nullptr, *xmap = nullptr;
+    const unsigned *off = nullptr;      // [ntiles * nrho + 1] first id of each (tile, slot)
+    const unsigned *job0 = nullptr;     // [ntiles + 1] first job of each tile
+    const TileJob *jobs = nullptr;      // [njobs], tile by tile
+    const UnitJob *ujobs = nullptr;     // [nujobs]
     std::vector<unsigned> job_plane;  // host: first plane of each job, once a budget needed groups
     JobGroups groups;                 // of the budget last used
-    DevBuf ujobs;                  // UnitJob [nujobs]
-    unsigned nunits = 0, nujobs = 0;
-    // cells of each axis as (tile, cell of its block) pairs: starts [nf + 1], then pairs
-    DevBuf zmap, xmap;
 };
 
 // The y planes [ylo, ylo + ly) (mod nfy) that the rows of a shared-tilt grid touch (ly 0: all).

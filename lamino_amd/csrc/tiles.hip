@@ -24,12 +24,25 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <type_traits>
 
 #include "nufft_point.h"
 #include "tiles.h"
 
 namespace lam {
+
+// y weights of a row slot and its first plane (unwrapped); direct plans use iy only
+struct RowY {
+    float w[12];
+    int iy, pad[3];
+};
+
+// A projection's geometry as the staging lanes read it: 16 bytes per axis, and float d_i.
+struct __attribute__((aligned(16))) TileGeo {
+    double uz, vz, ux, vx, vy, pad;
+    float d[4];
+};
 
 namespace {
 
@@ -47,12 +60,6 @@ constexpr int kXCells = 32 / NI;
 
 // occupancy hint (waves per SIMD): what the W-plane window leaves room for without spills
 constexpr int spread_waves(int W) { return W <= 6 ? 3 : W <= 8 ? 2 : 1; }
-
-// y weights of a row slot and its first plane (unwrapped); direct plans use iy only
-struct RowY {
-    float w[12];
-    int iy, pad[3];
-};
 
 // ------------------------------------------------------------------ plan building
 // The points of a line cross a tile in one run of consecutive columns, so the points are
@@ -152,8 +159,8 @@ __global__ __launch_bounds__(256) void k_scan_sums(const unsigned long long *__r
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-// one block: sums -> exclusive offsets, and the grand totals in sums[nb]
-__global__ __launch_bounds__(256) void k_scan_top(uint2 *__restrict__ sums, int nb) {
+// one block: sums -> exclusive offsets, and the grand totals
+__global__ __launch_bounds__(256) void k_scan_top(uint2 *__restrict__ sums, int nb, uint2 *__restrict__ grand) {
     uint2 carry = make_uint2(0u, 0u);
     for (int b0 = 0; b0 < nb; b0 += 256) {
         const int b = b0 + threadIdx.x;
@@ -163,7 +170,7 @@ __global__ __launch_bounds__(256) void k_scan_top(uint2 *__restrict__ sums, int 
         carry.x += total.x;
         carry.y += total.y;
     }
-    if (threadIdx.x == 0) sums[nb] = carry;
+    if (threadIdx.x == 0) *grand = carry;
 }
 
 template <bool PAD>
@@ -188,6 +195,72 @@ __global__ __launch_bounds__(256) void k_scan_apply(const unsigned long long *__
         e.x += a[u].x;
         e.y += a[u].y;
     }
+}
+
+// A scan of n counts: offsets of the low and high words in lo and hi (n + 1 entries each), the
+// grand totals in `grand` (pinned host memory).
+struct ScanArgs {
+    const unsigned long long *count = nullptr;
+    long long n = 0;
+    unsigned *lo = nullptr, *hi = nullptr;
+    uint2 *grand = nullptr;
+};
+
+// Up to kScanOne counts: one workgroup per scan, up to two scans, in one launch.  On the smallest
+// grids a plan's time is that of its launches and allocations (see get_tileplan).
+constexpr long long kScanOne = 8 * kScanBlock;
+
+template <bool PAD>
+__global__ __launch_bounds__(256) void k_scan_one(ScanArgs first, ScanArgs second) {
+    const ScanArgs s = blockIdx.x ? second : first;
+    uint2 carry = make_uint2(0u, 0u);
+    for (long long b0 = 0; b0 <= s.n; b0 += kScanBlock) {
+        uint2 a[kScanItems], v = make_uint2(0u, 0u), total;
+        const long long i0 = b0 + threadIdx.x * kScanItems;
+        for (int u = 0; u < kScanItems; ++u) {
+            a[u] = scan_item<PAD>(s.count, i0 + u, s.n);
+            v.x += a[u].x;
+            v.y += a[u].y;
+        }
+        uint2 e = block_scan(v, total);
+        e.x += carry.x;
+        e.y += carry.y;
+        for (int u = 0; u < kScanItems; ++u) {
+            if (i0 + u > s.n) break;
+            s.lo[i0 + u] = e.x;
+            s.hi[i0 + u] = e.y;
+            e.x += a[u].x;
+            e.y += a[u].y;
+        }
+        carry.x += total.x;
+        carry.y += total.y;
+    }
+    if (threadIdx.x == 0) *s.grand = carry;
+}
+
+long long scan_blocks(long long n) { return (n + kScanBlock) / kScanBlock; }   // cover entry n too
+
+template <bool PAD>
+void run_scan(Ctx &cx, const ScanArgs &s, uint2 *sums) {
+    const int nsb = (int)scan_blocks(s.n);
+    hipLaunchKernelGGL(k_scan_sums<PAD>, dim3(nsb), dim3(256), 0, cx.stream, s.count, s.n, sums);
+    check_launch();
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, cx.stream, sums, nsb, s.grand);
+    check_launch();
+    hipLaunchKernelGGL(k_scan_apply<PAD>, dim3(nsb), dim3(256), 0, cx.stream, s.count, s.n, sums, s.lo, s.hi);
+    check_launch();
+}
+
+// sums: scan_blocks(n) entries for the longer of the scans; second.n may be 0
+template <bool PAD>
+void run_scans(Ctx &cx, const ScanArgs &first, const ScanArgs &second, uint2 *sums) {
+    if (std::max(first.n, second.n) <= kScanOne) {
+        hipLaunchKernelGGL(k_scan_one<PAD>, dim3(second.n ? 2 : 1), dim3(256), 0, cx.stream, first, second);
+        check_launch();
+        return;
+    }
+    run_scan<PAD>(cx, first, sums);
+    if (second.n) run_scan<PAD>(cx, second, sums);
 }
 
 // Wave per bucket: its runs in order of their first point number, written out as point ids.
@@ -245,96 +318,109 @@ __device__ __forceinline__ void tile_jobs(const unsigned *__restrict__ o, int nr
     }
 }
 
-// count[tile]: planes its jobs record (low word), jobs (high word)
-__global__ __launch_bounds__(64) void k_job_count(const unsigned *__restrict__ off, const RowY *__restrict__ rowy,
-                                                  unsigned ntiles, int nrho, int W, unsigned most,
-                                                  unsigned long long *__restrict__ count) {
-    const unsigned t = blockIdx.x * 64u + threadIdx.x;
-    if (t >= ntiles) return;
-    unsigned planes = 0, jobs = 0;
-    tile_jobs(off + (long long)t * nrho, nrho, most, [&](unsigned, unsigned, unsigned, int r0, int r1) {
-        planes += (unsigned)(rowy[r1 - 1].iy + W - rowy[r0].iy);
-        ++jobs;
-    });
-    count[t] = ((unsigned long long)jobs << 32) | planes;
-}
-
-__global__ __launch_bounds__(64) void k_job_emit(const unsigned *__restrict__ off, const RowY *__restrict__ rowy,
-                                                 unsigned ntiles, int nrho, int nfy, int W, unsigned most,
-                                                 const unsigned *__restrict__ plane0,
-                                                 const unsigned *__restrict__ job0, TileJob *__restrict__ jobs) {
-    const unsigned t = blockIdx.x * 64u + threadIdx.x;
-    if (t >= ntiles) return;
-    unsigned plane = plane0[t];
-    tile_jobs(off + (long long)t * nrho, nrho, most, [&](unsigned i, unsigned beg, unsigned end, int r0, int r1) {
-        TileJob j;
-        j.tile = t;
-        j.beg = beg;
-        j.end = end;
-        j.r0 = r0;
-        j.r1 = r1;
-        j.y0 = rowy[r0].iy;
-        j.np = rowy[r1 - 1].iy + W - j.y0;
-        j.plane = plane;
-        j.yw = j.y0 % nfy;
-        if (j.yw < 0) j.yw += nfy;
-        plane += (unsigned)j.np;
-        jobs[job0[t] + i] = j;
-    });
-}
-
 // Tiles of one interpolation unit, side by side in x: they share a block of 16 cells.
 constexpr int kUnitTiles = 2;
 
 // Interpolation jobs: a job takes whole row slots [r0, r1) of a unit, or part `part` of `parts`
-// of one slot that alone holds more than a job.
+// of one slot that alone holds more than a job.  The unit's wave holds 64 slots' sizes in its
+// lanes and walks the non-empty ones.
 template <class F>
 __device__ __forceinline__ void unit_jobs(const unsigned *__restrict__ off, unsigned u, const TileGeom &tg,
                                           unsigned most, F emit) {
-    const int ut = kUnitTiles;
+    const int ut = kUnitTiles, lane = threadIdx.x & 63;
     const unsigned nux = (unsigned)(tg.ntx + ut - 1) / (unsigned)ut, uz = u / nux, ux = u - uz * nux;
     const unsigned *o = off + (long long)(uz * (unsigned)tg.ntx + (unsigned)ut * ux) * tg.nrho;
     const int tiles = min(ut, tg.ntx - ut * (int)ux);
     int r0 = -1, last = 0;   // last: one past the last slot with points
     unsigned held = 0;
-    for (int r = 0; r < tg.nrho; ++r) {
-        unsigned n = 0;
-        for (int t = 0; t < tiles; ++t) n += o[t * tg.nrho + r + 1] - o[t * tg.nrho + r];
-        if (n == 0) continue;
-        if (r0 >= 0 && held + n > most) {
-            emit(r0, last, 0u, 1u);
-            r0 = -1;
-            held = 0;
+    for (int rb = 0; rb < tg.nrho; rb += 64) {
+        unsigned size = 0;
+        if (rb + lane < tg.nrho)
+            for (int t = 0; t < tiles; ++t) size += o[t * tg.nrho + rb + lane + 1] - o[t * tg.nrho + rb + lane];
+        for (unsigned long long mask = __ballot(size > 0); mask; mask &= mask - 1ull) {
+            const int i = __builtin_ctzll(mask), r = rb + i;
+            const unsigned n = (unsigned)__builtin_amdgcn_readlane((int)size, i);
+            if (r0 >= 0 && held + n > most) {
+                emit(r0, last, 0u, 1u);
+                r0 = -1;
+                held = 0;
+            }
+            if (n > most) {
+                const unsigned parts = (n + most - 1) / most;
+                for (unsigned k = 0; k < parts; ++k) emit(r, r + 1, k, parts);
+                continue;
+            }
+            if (r0 < 0) r0 = r;
+            held += n;
+            last = r + 1;
         }
-        if (n > most) {
-            const unsigned parts = (n + most - 1) / most;
-            for (unsigned k = 0; k < parts; ++k) emit(r, r + 1, k, parts);
-            continue;
-        }
-        if (r0 < 0) r0 = r;
-        held += n;
-        last = r + 1;
     }
     if (r0 >= 0) emit(r0, last, 0u, 1u);
 }
 
-__global__ __launch_bounds__(64) void k_unit_count(const unsigned *__restrict__ off, TileGeom tg, unsigned nunits,
-                                                   unsigned most, unsigned long long *__restrict__ count) {
-    const unsigned u = blockIdx.x * 64u + threadIdx.x;
-    if (u >= nunits) return;
-    unsigned jobs = 0;
-    unit_jobs(off, u, tg, most, [&](int, int, unsigned, unsigned) { ++jobs; });
-    count[u] = jobs;
+// How a plan's points are shared out.  Workgroups of one wave: the first take 64 tiles' spread
+// jobs, a thread each, the others one unit's interpolation jobs (nunits 0: none).
+struct ShareArgs {
+    const unsigned *off;
+    const RowY *rowy;
+    unsigned jmost, umost, nunits;
+};
+unsigned tile_blocks(const TileGeom &tg) { return (tg.ntiles + 63) / 64; }
+
+// jcount[tile]: planes its jobs record (low word), jobs (high word); ucount[unit]: its jobs
+__global__ __launch_bounds__(64) void k_share_count(ShareArgs A, TileGeom tg, unsigned tblocks,
+                                                    unsigned long long *__restrict__ jcount,
+                                                    unsigned long long *__restrict__ ucount) {
+    if (blockIdx.x >= tblocks) {
+        const unsigned u = blockIdx.x - tblocks;
+        unsigned jobs = 0;
+        unit_jobs(A.off, u, tg, A.umost, [&](int, int, unsigned, unsigned) { ++jobs; });
+        if (threadIdx.x == 0) ucount[u] = jobs;
+        return;
+    }
+    const unsigned t = blockIdx.x * 64u + threadIdx.x;
+    if (t >= tg.ntiles) return;
+    unsigned planes = 0, jobs = 0;
+    tile_jobs(A.off + (long long)t * tg.nrho, tg.nrho, A.jmost, [&](unsigned, unsigned, unsigned, int r0, int r1) {
+        planes += (unsigned)(A.rowy[r1 - 1].iy + tg.W - A.rowy[r0].iy);
+        ++jobs;
+    });
+    jcount[t] = ((unsigned long long)jobs << 32) | planes;
 }
 
-__global__ __launch_bounds__(64) void k_unit_emit(const unsigned *__restrict__ off, TileGeom tg, unsigned nunits,
-                                                  unsigned most, const unsigned *__restrict__ job0,
-                                                  UnitJob *__restrict__ jobs) {
-    const unsigned u = blockIdx.x * 64u + threadIdx.x;
-    if (u >= nunits) return;
-    unsigned j = job0[u];
-    unit_jobs(off, u, tg, most,
-              [&](int r0, int r1, unsigned part, unsigned parts) { jobs[j++] = UnitJob{u, r0, r1, part, parts}; });
+__global__ __launch_bounds__(64) void k_share_emit(ShareArgs A, TileGeom tg, unsigned tblocks,
+                                                   const unsigned *__restrict__ plane0,
+                                                   const unsigned *__restrict__ job0,
+                                                   const unsigned *__restrict__ ujob0, TileJob *__restrict__ jobs,
+                                                   UnitJob *__restrict__ ujobs) {
+    if (blockIdx.x >= tblocks) {
+        const unsigned u = blockIdx.x - tblocks;
+        unsigned j = ujob0[u];
+        unit_jobs(A.off, u, tg, A.umost, [&](int r0, int r1, unsigned part, unsigned parts) {
+            if (threadIdx.x == 0) ujobs[j] = UnitJob{u, r0, r1, part, parts};
+            ++j;
+        });
+        return;
+    }
+    const unsigned t = blockIdx.x * 64u + threadIdx.x;
+    if (t >= tg.ntiles) return;
+    unsigned plane = plane0[t];
+    tile_jobs(A.off + (long long)t * tg.nrho, tg.nrho, A.jmost,
+              [&](unsigned i, unsigned beg, unsigned end, int r0, int r1) {
+                  TileJob j;
+                  j.tile = t;
+                  j.beg = beg;
+                  j.end = end;
+                  j.r0 = r0;
+                  j.r1 = r1;
+                  j.y0 = A.rowy[r0].iy;
+                  j.np = A.rowy[r1 - 1].iy + tg.W - j.y0;
+                  j.plane = plane;
+                  j.yw = j.y0 % tg.nfy;
+                  if (j.yw < 0) j.yw += tg.nfy;
+                  plane += (unsigned)j.np;
+                  jobs[job0[t] + i] = j;
+              });
 }
 
 // ------------------------------------------------------------------ shared by both kernels
@@ -384,12 +470,6 @@ __device__ __forceinline__ double detector_coord(int i, double centre, double st
 #pragma clang fp contract(off)
     return ((double)i - centre) * step;
 }
-
-// A projection's geometry as the staging lanes read it: 16 bytes per axis, and float d_i.
-struct __attribute__((aligned(16))) TileGeo {
-    double uz, vz, ux, vx, vy, pad;
-    float d[4];
-};
 
 struct TileArgs {
     long long S;
@@ -931,10 +1011,18 @@ bool tile_fits(const TileGeom &tg, long long total) {
 // allow (3 per SIMD), within a range.  Measured, spread + merge in us: (89, 21, 89) / 89 with
 // 128, 256, 512 and 1024 points: 79, 67, 73, 83; (179, 43, 179) / 305 with 684, 1367, 2048:
 // 620, 578, 581; (359, 71, 359) / 615 with 4096, 5543, 8192: 3392, 3403, 3516.
-constexpr unsigned kJobMin = 384, kJobMax = 5120, kJobTarget = 6144;
+//
+// First-cell slots take a matrix product per point pair and plane, W times as many, so that a
+// job's own chain is longer: there the least is the square root of the points, which weighs that
+// chain against the jobs that a cell's sum goes over, from 64.  A whole adjoint in us with 64,
+// 96, 128, 192 and 384 points: 4420 points 92, 93, 95, 102, 129; 21,800 132, 119, 113, 115, 138;
+// 60,800 194, 159, 142, 131, 140; 192,000 217, 180, 161, 156, 154.
+constexpr unsigned kJobMin = 384, kJobMinDirect = 64, kJobMax = 5120, kJobTarget = 6144;
 
-unsigned job_points(long long total) {
-    return (unsigned)std::max<long long>(kJobMin, std::min<long long>(kJobMax, total / kJobTarget)) & ~3u;
+unsigned job_points(long long total, bool direct) {
+    const long long least =
+        direct ? std::clamp<long long>((long long)std::sqrt((double)total), kJobMinDirect, kJobMin) : kJobMin;
+    return (unsigned)std::max<long long>(least, std::min<long long>(kJobMax, total / kJobTarget)) & ~3u;
 }
 
 // Points an interpolation job may hold: a job loads W planes of its block before its first
@@ -955,24 +1043,35 @@ int unit_rows(const TilePlan &tp, long long total) {
 
 // (tile, block cell) pairs of every cell of an axis
 std::vector<int> axis_map(int nf, int T, int nt, int W) {
-    std::vector<std::vector<std::pair<int, int>>> m(nf);
-    for (int t = 0; t < nt; ++t) {
-        const int o = t * T, w = std::min(T, nf - o);
-        for (int i = 0; i < w + W - 1; ++i) m[(o + i) % nf].emplace_back(t, i);
-    }
-    std::vector<int> out(nf + 1);
-    for (int x = 0; x < nf; ++x) out[x + 1] = out[x] + (int)m[x].size();
-    for (int x = 0; x < nf; ++x)
-        for (auto &e : m[x]) {
-            out.push_back(e.first);
-            out.push_back(e.second);
-        }
+    const auto each = [&](auto f) {
+        for (int t = 0; t < nt; ++t)
+            for (int i = 0; i < std::min(T, nf - t * T) + W - 1; ++i) f((t * T + i) % nf, t, i);
+    };
+    std::vector<int> out(nf + 1, 0);
+    each([&](int x, int, int) { ++out[x + 1]; });
+    for (int x = 0; x < nf; ++x) out[x + 1] += out[x];
+    std::vector<int> at(out.begin(), out.end() - 1);
+    out.resize(nf + 1 + 2 * (size_t)out[nf]);
+    each([&](int x, int t, int i) {
+        const int e = nf + 1 + 2 * at[x]++;
+        out[e] = t;
+        out[e + 1] = i;
+    });
     return out;
 }
 
-void upload_vec(Ctx &cx, DevBuf &b, const std::vector<int> &v) {
-    b.alloc(sizeof(int) * v.size());
-    upload_now(cx, b.ptr, v.data(), sizeof(int) * v.size());
+// Places parts of one buffer, 16 bytes aligned.
+struct Carve {
+    size_t bytes = 0;
+    size_t take(size_t n) {
+        const size_t at = bytes;
+        bytes += (n + 15) & ~(size_t)15;
+        return at;
+    }
+};
+template <class T>
+T *part(const DevBuf &b, size_t at) {
+    return reinterpret_cast<T *>(b.as<char>() + at);
 }
 
 // bytes of one recorded plane of a job
@@ -1017,7 +1116,7 @@ const JobGroups &job_groups(Ctx &cx, TilePlan &tp) {
     if (cap == jg.cap) return jg;
     if (tp.planes > cap && tp.job_plane.empty()) {
         std::vector<TileJob> jobs(tp.njobs);
-        LAM_HIP(hipMemcpyAsync(jobs.data(), tp.jobs.ptr, sizeof(TileJob) * jobs.size(), hipMemcpyDeviceToHost,
+        LAM_HIP(hipMemcpyAsync(jobs.data(), tp.jobs, sizeof(TileJob) * jobs.size(), hipMemcpyDeviceToHost,
                                cx.stream));
         LAM_HIP(hipStreamSynchronize(cx.stream));
         tp.job_plane.reserve(jobs.size());
@@ -1064,20 +1163,27 @@ TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long
     for (const bool direct : {false, true}) {
         const TileGeom tg = tile_geom(pl.nf, pl.w, R, C, direct);
         const size_t nb = (size_t)tg.ntiles * tg.nrho, ids = total + 3 * std::min(nb, total);
-        const size_t jobs = tg.ntiles + ids / job_points((long long)total) + 1;
+        const size_t jobs = tg.ntiles + ids / job_points((long long)total, direct) + 1;
+        // an interpolation job and the next one of its unit hold more points than one may
+        const size_t ujobs = tg.ntiles + 4 * (ids / unit_points((long long)total)) + 1;
         // a job's planes: its rows' first planes and W - 1 more; the half set spans at most half
         // the period
         const size_t planes = (size_t)tg.ntiles * (size_t)(direct ? tg.nfy : tg.nfy / 2 + 2) + jobs * (size_t)pl.w;
         const size_t largest = record_bytes(tg) * ((size_t)tg.nfy + pl.w);   // of one job
-        b.kept = std::max(b.kept, 4 * (ids + nb + tg.ntiles) + sizeof(TileJob) * jobs + sizeof(TileGeo) * (size_t)P +
+        b.kept = std::max(b.kept, 4 * (ids + nb + tg.ntiles) + sizeof(TileJob) * jobs + sizeof(UnitJob) * ujobs + sizeof(TileGeo) * (size_t)P +
                                       sizeof(RowY) * tg.nrho + 64 * (size_t)(tg.nfz + tg.nfx) + 4096);
-        // counts, run offsets and cursors per bucket, the runs, scan sums
-        b.setup = std::max(b.setup, 17 * nb + 8 * total + 32 * (size_t)tg.ntiles + 65536);
+        b.setup = std::max(b.setup, 8 * total);   // the runs
+        // counts, run offsets and cursors per bucket and scan sums, in the record buffer
+        b.records = std::max(b.records, 17 * nb + 64 * (size_t)tg.ntiles + 65536);
         b.records = std::max(b.records, std::min(record_bytes(tg) * planes, std::max(record_budget(), largest)));
     }
     return b;
 }
 
+// A plan takes few launches, allocations and waits: on small grids the first pass on a new grid is
+// made of them.  With an array per allocation, three launches per scan and a thread per unit,
+// the first adjoint of (9, 5, 11) / 13 x 15 x 12 took 338 us, now 154; (89, 21, 89) / 89 x 89 x 90
+// 470, now 276; (179, 43, 179) / 305 x 305 x 180 1594, now 1251; the headline grid 8776, now 8114.
 TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
     std::vector<long long> key = {pl.nf[0], pl.nf[1], pl.nf[2], pl.w, direct ? 1 : 0};
     auto it = g.tileplans.find(key);
@@ -1115,111 +1221,100 @@ TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
         }
         row_window(g, pl, tp->ylo, tp->ly);
     }
-    tp->rowy.alloc(sizeof(RowY) * rows.size());
-    upload_now(cx, tp->rowy.ptr, rows.data(), sizeof(RowY) * rows.size());
-
-    std::vector<TileGeo> tgeo(g.P);
-    for (long long p = 0; p < g.P; ++p) {
-        const Geo &e = g.geo_host[p];
-        tgeo[p] = TileGeo{e.uz, e.vz, e.ux, e.vx, e.vy, 0.0, {(float)e.d0, (float)e.d1, (float)e.d2, 0.f}};
+    // what the host works out, in one upload
+    {
+        const std::vector<int> zmap = axis_map(tg.nfz, tg.Tz, tg.ntz, W), xmap = axis_map(tg.nfx, tg.Tx, tg.ntx, W);
+        Carve c;
+        const size_t og = c.take(sizeof(TileGeo) * g.P), orow = c.take(sizeof(RowY) * rows.size()),
+                     oz = c.take(sizeof(int) * zmap.size()), ox = c.take(sizeof(int) * xmap.size());
+        std::vector<char> host(c.bytes);
+        for (long long p = 0; p < g.P; ++p) {
+            const Geo &e = g.geo_host[p];
+            const TileGeo t{e.uz, e.vz, e.ux, e.vx, e.vy, 0.0, {(float)e.d0, (float)e.d1, (float)e.d2, 0.f}};
+            std::memcpy(host.data() + og + sizeof(TileGeo) * p, &t, sizeof(t));
+        }
+        std::memcpy(host.data() + orow, rows.data(), sizeof(RowY) * rows.size());
+        std::memcpy(host.data() + oz, zmap.data(), sizeof(int) * zmap.size());
+        std::memcpy(host.data() + ox, xmap.data(), sizeof(int) * xmap.size());
+        tp->fixed.alloc(c.bytes);
+        upload_now(cx, tp->fixed.ptr, host.data(), c.bytes);
+        tp->geo = part<TileGeo>(tp->fixed, og);
+        tp->rowy = part<RowY>(tp->fixed, orow);
+        tp->zmap = part<int>(tp->fixed, oz);
+        tp->xmap = part<int>(tp->fixed, ox);
     }
-    tp->geo.alloc(sizeof(TileGeo) * tgeo.size());
-    upload_now(cx, tp->geo.ptr, tgeo.data(), sizeof(TileGeo) * tgeo.size());
-
-    upload_vec(cx, tp->zmap, axis_map(tg.nfz, tg.Tz, tg.ntz, W));
-    upload_vec(cx, tp->xmap, axis_map(tg.nfx, tg.Tx, tg.ntx, W));
+    tp->nunits = tile_interp_fits(pl.w) && !direct
+                     ? (unsigned)tg.ntz * (unsigned)((tg.ntx + kUnitTiles - 1) / kUnitTiles)
+                     : 0u;
+    Carve ci;
+    const size_t ooff = ci.take(sizeof(unsigned) * (nb + 1)), ojob0 = ci.take(sizeof(unsigned) * (tg.ntiles + 1ull));
+    tp->index.alloc(ci.bytes);
+    unsigned *off = part<unsigned>(tp->index, ooff), *job0 = part<unsigned>(tp->index, ojob0);
+    tp->off = off;
+    tp->job0 = job0;
+    // The temporaries sit in the record buffer, which the spread needs anyway.
+    Carve cs;
+    const size_t ocount = cs.take(sizeof(unsigned long long) * nb), ocursor = cs.take(sizeof(unsigned) * nb),
+                 zeroed = cs.bytes, oroff = cs.take(sizeof(unsigned) * (nb + 1)),
+                 osums = cs.take(sizeof(uint2) * scan_blocks(std::max<long long>(nb, std::max(tg.ntiles, tp->nunits)))),
+                 ojcount = cs.take(sizeof(unsigned long long) * tg.ntiles),
+                 ojplane = cs.take(sizeof(unsigned) * (tg.ntiles + 1ull)),
+                 oucount = cs.take(sizeof(unsigned long long) * tp->nunits),
+                 oujob0 = cs.take(sizeof(unsigned) * (tp->nunits + 1ull)),
+                 ouhigh = cs.take(sizeof(unsigned) * (tp->nunits + 1ull));
+    pl.rec.ensure(cs.bytes);
+    const DevBuf &tmp = pl.rec;
+    auto *count = part<unsigned long long>(tmp, ocount);
+    unsigned *cursor = part<unsigned>(tmp, ocursor), *roff = part<unsigned>(tmp, oroff);
+    uint2 *sums = part<uint2>(tmp, osums), *grand = reinterpret_cast<uint2 *>(cx.sums.get());
 
     // points: runs counted per bucket, scanned, stored, ordered and written out
-    DevBuf count(sizeof(unsigned long long) * nb);
-    LAM_HIP(hipMemsetAsync(count.ptr, 0, count.bytes, cx.stream));
+    LAM_HIP(hipMemsetAsync(tmp.ptr, 0, zeroed, cx.stream));
     const unsigned cpl = (unsigned)((g.C + 63) / 64);
     const long long nwaves = g.P * Jn * (long long)cpl;
     const dim3 rgrid = wave_grid(nwaves);
     hipLaunchKernelGGL(k_tile_runs<0>, rgrid, dim3(256), 0, cx.stream, g.geo.as<Geo>(), nwaves, (int)g.R, (int)g.C, fr,
-                       tg, cpl, count.as<unsigned long long>(), (const unsigned *)nullptr, (unsigned *)nullptr,
-                       (uint2 *)nullptr);
+                       tg, cpl, count, (const unsigned *)nullptr, (unsigned *)nullptr, (uint2 *)nullptr);
     check_launch();
-    const int nsb = (int)((nb + kScanBlock) / kScanBlock);   // covers entry nb too
-    DevBuf sums(sizeof(uint2) * (nsb + 1)), roff(sizeof(unsigned) * (nb + 1));
-    tp->off.alloc(sizeof(unsigned) * (nb + 1));
-    hipLaunchKernelGGL(k_scan_sums<true>, dim3(nsb), dim3(256), 0, cx.stream, count.as<unsigned long long>(), nb,
-                       sums.as<uint2>());
-    check_launch();
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, cx.stream, sums.as<uint2>(), nsb);
-    check_launch();
-    hipLaunchKernelGGL(k_scan_apply<true>, dim3(nsb), dim3(256), 0, cx.stream, count.as<unsigned long long>(), nb,
-                       sums.as<uint2>(), tp->off.as<unsigned>(), roff.as<unsigned>());
-    check_launch();
-    uint2 totals;
-    LAM_HIP(hipMemcpyAsync(&totals, sums.as<uint2>() + nsb, sizeof(totals), hipMemcpyDeviceToHost, cx.stream));
+    run_scans<true>(cx, ScanArgs{count, nb, off, roff, grand}, ScanArgs{}, sums);
     LAM_HIP(hipStreamSynchronize(cx.stream));
-    LAM_REQUIRE((long long)totals.x >= total && (long long)totals.y <= total, LAM_ERR_STATE,
+    const uint2 points = grand[0];
+    LAM_REQUIRE((long long)points.x >= total && (long long)points.y <= total, LAM_ERR_STATE,
                 "bin counts do not add up to the point count");
-    DevBuf runs(sizeof(uint2) * std::max<size_t>(totals.y, 1)), cursor(sizeof(unsigned) * nb);
-    tp->ids.alloc(sizeof(unsigned) * std::max<size_t>(totals.x, 1));
-    LAM_HIP(hipMemsetAsync(cursor.ptr, 0, cursor.bytes, cx.stream));
+    DevBuf own;   // the runs, where the record buffer has no room left for them
+    const size_t orun = cs.take(sizeof(uint2) * points.y);
+    if (cs.bytes > tmp.bytes) own.alloc(sizeof(uint2) * points.y);
+    uint2 *runs = own.ptr ? own.as<uint2>() : part<uint2>(tmp, orun);
+    tp->ids.alloc(sizeof(unsigned) * std::max<size_t>(points.x, 1));
     hipLaunchKernelGGL(k_tile_runs<1>, rgrid, dim3(256), 0, cx.stream, g.geo.as<Geo>(), nwaves, (int)g.R, (int)g.C, fr,
-                       tg, cpl, (unsigned long long *)nullptr, roff.as<unsigned>(), cursor.as<unsigned>(),
-                       runs.as<uint2>());
+                       tg, cpl, (unsigned long long *)nullptr, roff, cursor, runs);
     check_launch();
-    hipLaunchKernelGGL(k_run_expand, wave_grid(nb), dim3(256), 0, cx.stream,
-                       count.as<unsigned long long>(), nb, tp->off.as<unsigned>(), roff.as<unsigned>(),
-                       runs.as<uint2>(), tp->ids.as<unsigned>());
+    hipLaunchKernelGGL(k_run_expand, wave_grid(nb), dim3(256), 0, cx.stream, count, nb, off, roff, runs,
+                       tp->ids.as<unsigned>());
     check_launch();
-    // jobs: counted per tile, scanned, written out
-    const unsigned most = job_points(total);
-    const int njb = (int)((tg.ntiles + (long long)kScanBlock) / kScanBlock);
-    DevBuf jcount(sizeof(unsigned long long) * tg.ntiles), jsums(sizeof(uint2) * (njb + 1)),
-        jplane(sizeof(unsigned) * (tg.ntiles + 1));
-    tp->job0.alloc(sizeof(unsigned) * (tg.ntiles + 1));
-    const dim3 jgrid((tg.ntiles + 63) / 64);
-    hipLaunchKernelGGL(k_job_count, jgrid, dim3(64), 0, cx.stream, tp->off.as<unsigned>(), tp->rowy.as<RowY>(),
-                       tg.ntiles, tg.nrho, W, most, jcount.as<unsigned long long>());
+    // shares: counted per tile and unit, scanned, written out
+    const ShareArgs sa{off, tp->rowy, job_points(total, direct), unit_points(total), tp->nunits};
+    const unsigned tblocks = tile_blocks(tg);
+    const dim3 sgrid(tblocks + tp->nunits);
+    auto *jcount = part<unsigned long long>(tmp, ojcount), *ucount = part<unsigned long long>(tmp, oucount);
+    unsigned *jplane = part<unsigned>(tmp, ojplane), *ujob0 = part<unsigned>(tmp, oujob0);
+    hipLaunchKernelGGL(k_share_count, sgrid, dim3(64), 0, cx.stream, sa, tg, tblocks, jcount, ucount);
     check_launch();
-    hipLaunchKernelGGL(k_scan_sums<false>, dim3(njb), dim3(256), 0, cx.stream, jcount.as<unsigned long long>(),
-                       (long long)tg.ntiles, jsums.as<uint2>());
-    check_launch();
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, cx.stream, jsums.as<uint2>(), njb);
-    check_launch();
-    hipLaunchKernelGGL(k_scan_apply<false>, dim3(njb), dim3(256), 0, cx.stream, jcount.as<unsigned long long>(),
-                       (long long)tg.ntiles, jsums.as<uint2>(), jplane.as<unsigned>(), tp->job0.as<unsigned>());
-    check_launch();
-    LAM_HIP(hipMemcpyAsync(&totals, jsums.as<uint2>() + njb, sizeof(totals), hipMemcpyDeviceToHost, cx.stream));
+    run_scans<false>(cx, ScanArgs{jcount, tg.ntiles, jplane, job0, grand + 1},
+                     ScanArgs{ucount, tp->nunits, ujob0, part<unsigned>(tmp, ouhigh), grand + 2}, sums);
     LAM_HIP(hipStreamSynchronize(cx.stream));
-    tp->planes = totals.x;
-    tp->njobs = totals.y;
-    tp->jobs.alloc(sizeof(TileJob) * std::max<size_t>(totals.y, 1));
-    hipLaunchKernelGGL(k_job_emit, jgrid, dim3(64), 0, cx.stream, tp->off.as<unsigned>(), tp->rowy.as<RowY>(),
-                       tg.ntiles, tg.nrho, tg.nfy, W, most, jplane.as<unsigned>(), tp->job0.as<unsigned>(),
-                       tp->jobs.as<TileJob>());
+    tp->planes = grand[1].x;
+    tp->njobs = grand[1].y;
+    tp->nujobs = tp->nunits ? grand[2].x : 0u;
+    Carve cw;
+    const size_t ojobs = cw.take(sizeof(TileJob) * tp->njobs), oujobs = cw.take(sizeof(UnitJob) * tp->nujobs);
+    tp->shares.alloc(std::max<size_t>(cw.bytes, 16));
+    tp->jobs = part<TileJob>(tp->shares, ojobs);
+    tp->ujobs = part<UnitJob>(tp->shares, oujobs);
+    hipLaunchKernelGGL(k_share_emit, sgrid, dim3(64), 0, cx.stream, sa, tg, tblocks, jplane, job0, ujob0,
+                       part<TileJob>(tp->shares, ojobs), part<UnitJob>(tp->shares, oujobs));
     check_launch();
-    if (tile_interp_fits(pl.w) && !direct) {
-        tp->nunits = (unsigned)tg.ntz * (unsigned)((tg.ntx + kUnitTiles - 1) / kUnitTiles);
-        const unsigned umost = unit_points(total);
-        const int nub = (int)((tp->nunits + (long long)kScanBlock) / kScanBlock);
-        DevBuf ucount(sizeof(unsigned long long) * tp->nunits), usums(sizeof(uint2) * (nub + 1)),
-            ujob(sizeof(unsigned) * (tp->nunits + 1)), uhigh(sizeof(unsigned) * (tp->nunits + 1));
-        const dim3 ugrid((tp->nunits + 63) / 64);
-        hipLaunchKernelGGL(k_unit_count, ugrid, dim3(64), 0, cx.stream, tp->off.as<unsigned>(), tg, tp->nunits, umost,
-                           ucount.as<unsigned long long>());
-        check_launch();
-        hipLaunchKernelGGL(k_scan_sums<false>, dim3(nub), dim3(256), 0, cx.stream, ucount.as<unsigned long long>(),
-                           (long long)tp->nunits, usums.as<uint2>());
-        check_launch();
-        hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(256), 0, cx.stream, usums.as<uint2>(), nub);
-        check_launch();
-        hipLaunchKernelGGL(k_scan_apply<false>, dim3(nub), dim3(256), 0, cx.stream, ucount.as<unsigned long long>(),
-                           (long long)tp->nunits, usums.as<uint2>(), ujob.as<unsigned>(), uhigh.as<unsigned>());
-        check_launch();
-        LAM_HIP(hipMemcpyAsync(&totals, usums.as<uint2>() + nub, sizeof(totals), hipMemcpyDeviceToHost, cx.stream));
-        LAM_HIP(hipStreamSynchronize(cx.stream));
-        tp->nujobs = totals.x;
-        tp->ujobs.alloc(sizeof(UnitJob) * std::max<size_t>(totals.x, 1));
-        hipLaunchKernelGGL(k_unit_emit, ugrid, dim3(64), 0, cx.stream, tp->off.as<unsigned>(), tg, tp->nunits, umost,
-                           ujob.as<unsigned>(), tp->ujobs.as<UnitJob>());
-        check_launch();
-    }
-    LAM_HIP(hipStreamSynchronize(cx.stream));   // the temporaries go
+    if (own.ptr) LAM_HIP(hipStreamSynchronize(cx.stream));   // it goes
     TilePlan &ref = *tp;
     g.tileplans.emplace(std::move(key), std::move(tp));
     return ref;
@@ -1240,9 +1335,9 @@ void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c,
             const dim3 grid((j1 - j0) * (unsigned)(3 / tile_comps(pl.w)));
 #define LAM_TILE_SPREAD(DIRECT)                                                                                  \
     LAM_TILE_WIDTH(pl.w, hipLaunchKernelGGL((k_tile_spread<W, tile_comps(W), DIRECT>), grid, dim3(64), 0, cx.stream, \
-                                            pl.rec.as<float2>(), c, tp.geo.as<TileGeo>(), tp.off.as<unsigned>(), \
-                                            tp.ids.as<unsigned>(), tp.rowy.as<RowY>(),                           \
-                                            tp.jobs.as<TileJob>() + j0, a, tg, groups[k].second, paired ? 1 : 0))
+                                            pl.rec.as<float2>(), c, tp.geo, tp.off, \
+                                            tp.ids.as<unsigned>(), tp.rowy,                           \
+                                            tp.jobs + j0, a, tg, groups[k].second, paired ? 1 : 0))
             if (tg.direct) {
                 LAM_TILE_SPREAD(true);
             } else {
@@ -1255,9 +1350,9 @@ void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c,
         const dim3 mgrid((unsigned)((3 * tg.nfx + 255) / 256) * (unsigned)tg.nfz *
                          (unsigned)((ly + kMergePlanes - 1) / kMergePlanes));
         LAM_TILE_WIDTH(pl.w, hipLaunchKernelGGL((k_tile_merge<tile_comps(W)>), mgrid, dim3(256), 0, cx.stream,
-                                                pl.fine.as<float2>(), pl.rec.as<float2>(), tp.jobs.as<TileJob>(),
-                                                tp.job0.as<unsigned>(), j0, j1, groups[k].second, tp.zmap.as<int>(),
-                                                tp.xmap.as<int>(), tg, ylo, ly, add || k > 0 ? 1 : 0));
+                                                pl.fine.as<float2>(), pl.rec.as<float2>(), tp.jobs,
+                                                tp.job0, j0, j1, groups[k].second, tp.zmap,
+                                                tp.xmap, tg, ylo, ly, add || k > 0 ? 1 : 0));
         check_launch();
     }
 }
@@ -1279,8 +1374,8 @@ void tile_interp(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, float2 *c) {
     allow(pl.w == 4 ? &k_tile_interp<4> : &k_tile_interp<6>);
 #define LAM_TILE_INTERP(WW)                                                                                         \
     hipLaunchKernelGGL((k_tile_interp<WW>), dim3(tp.nujobs), dim3(kUnitThreads), lds, cx.stream, pl.fine.as<float2>(), \
-                       c, tp.geo.as<TileGeo>(), tp.off.as<unsigned>(), tp.ids.as<unsigned>(), tp.rowy.as<RowY>(),   \
-                       tp.ujobs.as<UnitJob>(), a, tg, nr)
+                       c, tp.geo, tp.off, tp.ids.as<unsigned>(), tp.rowy,   \
+                       tp.ujobs, a, tg, nr)
     if (pl.w == 4) LAM_TILE_INTERP(4);
     else LAM_TILE_INTERP(6);
 #undef LAM_TILE_INTERP

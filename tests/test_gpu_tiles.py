@@ -147,3 +147,21 @@ def test_adjoint_over_the_record_budget_can_be_captured(monkeypatch, planes):
     monkeypatch.delenv("LAMINO_NUFFT_SLAB_BYTES")
     call()
     assert _rel(result(), want) < 1e-5   # the same sums in another order
+
+
+@pytest.mark.parametrize("dims,R,C,P", [((48, 6, 40), 11, 24, 5), ((48, 6, 40), 81, 24, 5), ((48, 6, 40), 141, 24, 5),
+                                        ((64, 6, 64), 201, 16, 4), ((64, 6, 64), 201, 70, 3)])
+def test_plans_scanned_in_one_workgroup_and_in_several(dims, R, C, P):
+    """Counts of less than one block of 2048, of several in one workgroup (864 to 10,224 buckets),
+    and of several workgroups (31,512); row slots below and above a wave's 64."""
+    import lamino_amd as la
+    import oracle as orc
+
+    say("plan scans", dims, R, C, P)
+    rng = np.random.default_rng(22)
+    al, ga = np.full(P, np.radians(31.0)), 0.3 + 2 * np.pi * np.arange(P) / P
+    pg = la.PolarGrid.per_projection(al, ga, R, C)
+    p = rng.standard_normal((P, R, C)).astype(np.float32)
+    assert _rel(la.adjoint(p, pg, dims), orc.adjoint(p, dims, al, ga, eps=1e-12)) < _tol(1e-5)
+    m = rng.standard_normal((3,) + dims).astype(np.float32)
+    assert _rel(la.forward(m, pg), orc.forward(m, al, ga, R, C, eps=1e-12)) < _tol(1e-5)
