@@ -142,7 +142,7 @@ Staging *Server::take_staging(size_t bytes) {
 void Server::finish(Job *j, lam_status st, const std::string &err) {
     {
         std::lock_guard<std::mutex> lk(mu);
-        j->info.end_s = now();
+        if (j->info.end_s == 0) j->info.end_s = now();
         j->info.status = st;
         j->err = err;
         j->finished = true;
@@ -251,6 +251,8 @@ void Server::worker(int slot) {
             std::lock_guard<std::mutex> lk(mu);
             in_use -= j->info.footprint_est;
             --running;
+            // ended before another worker can take the budget; a job with files ends with them
+            if (!to_writer) j->info.end_s = now();
             j->info.footprint_peak = peak;
             j->proj.clear();
             j->proj.shrink_to_fit();

@@ -142,6 +142,22 @@ def test_budget_admission_serialises_jobs_that_do_not_fit(ctx):
         assert b0 >= a1, spans
 
 
+def test_jobs_admitted_one_at_a_time_have_disjoint_times(ctx):
+    """A job's end is stamped when it gives its budget back, so the next job's start comes after
+    it, over many short jobs."""
+    import lamino_amd as la
+    from lamino_amd.serve import Server
+
+    jobs = [_job(60 + k % 3, rd=(5, 3, 5)) for k in range(60)]
+    prm = _params(1)
+    budget = int(max(la.api.mbir_footprint(1, ds, rd, prm) for ds, rd in jobs) * 1.5)
+    with Server(budget_bytes=budget, slots=3, mode="graph") as s:
+        ids = [s.submit(1, ds, rd, prm) for ds, rd in jobs]
+        infos = [s.wait(i)[1] for i in ids]
+    spans = sorted((i["start_s"], i["end_s"]) for i in infos)
+    assert all(b[0] >= a[1] for a, b in zip(spans, spans[1:])), spans
+
+
 def test_over_budget_job_is_rejected(ctx):
     from lamino_amd import _lib
     from lamino_amd.serve import Server
