@@ -250,8 +250,10 @@ def forward(magnetization, pg: PolarGrid, gamma: float | None = None, eps: float
 
 
 def autotune_bins(pg: PolarGrid, recon_dims, eps: float = DEFAULT_EPS):
-    """Times spreading tile shapes for this grid and volume and keeps the fastest
-    for later calls with the same shapes; returns ((Tz, Ty, Tx), spread+interp ms)."""
+    """Times tile shapes of the kernels that read one (shared tilt: MBIR1's and MBIR2's row
+    spreader, and the forward's row interpolator at kernel widths above 6; else the binned
+    interpolator) for this grid and volume and keeps the fastest for later calls with the same
+    shapes; returns ((Tz, Ty, Tx), ms of those kernels)."""
     T = (ctypes.c_int * 3)()
     ms = ctypes.c_double()
     check(pg.ctx.lib.lam_autotune_bins(pg.ctx.h, pg.h, _dims(recon_dims), float(eps), T, ctypes.byref(ms)))

@@ -107,9 +107,10 @@ void mbir_run(Ctx &cx, const lam_dataset *ds, int nds, const long long rd[3], co
         std::vector<double> gam(D.nproj);
         for (long long p = 0; p < D.nproj; ++p) gam[p] = D.gamma ? D.gamma[p] : D.gamma_const;
         grids.push_back(make_grid(cx, D.alpha, gam.data(), D.nproj, R2, C2));
-        // the graph form picks its spreading tiles by measurement, once per shape, on an
-        // evenly spaced subset of the projections (same planes' density, fewer of them)
-        if (mode == MbirMode::Graph && !bins_tuned(cx, *grids.back(), od, eps)) {
+        const SpreadOrder order = pr.method == 3 ? SpreadOrder::Tiles : SpreadOrder::Rows;
+        // where the spreader has a tiling, the graph form picks it by measurement, once per
+        // shape, on an evenly spaced subset of the projections (same planes' density, fewer)
+        if (mode == MbirMode::Graph && spread_wants_tuning(cx, *grids.back(), od, eps, order)) {
             constexpr long long kTuneProjections = 64;
             const long long Pt = std::min<long long>(D.nproj, kTuneProjections);
             std::vector<double> ta(Pt), tg(Pt);
@@ -122,8 +123,7 @@ void mbir_run(Ctx &cx, const lam_dataset *ds, int nds, const long long rd[3], co
             autotune_bins(cx, *sub, od, eps, nullptr);
         }
         float *ys[3] = {yT.v().c[0], yT.v().c[1], yT.v().c[2]};
-        adjoint(cx, *grids.back(), od, eps, padded.as<float>(), ys, true,
-                pr.method == 3 ? SpreadOrder::Tiles : SpreadOrder::Rows);
+        adjoint(cx, *grids.back(), od, eps, padded.as<float>(), ys, true, order);
     }
     raw.release();
     padded.release();

@@ -131,11 +131,11 @@ void forward_multi(Ctx &cx, Grid *const *grids, int ngrids, const long long dims
                    const float *const m[3], float *const *proj);
 void adjoint_multi(Ctx &cx, Grid *const *grids, int ngrids, const long long dims[3], double eps,
                    const float *const *proj, float *const m[3], bool accumulate);
-// Picks the spreading/interpolation tile shape of this grid and fine grid by
-// timing candidates; the choice is kept in cx.bin_tune.  best_ms: spread+interp time.
+// Picks the tile shape of this grid and fine grid by timing the kernels that read one; the
+// choice is kept in cx.bin_tune.  best_ms: the time of those kernels.
 std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], double eps, double *best_ms);
-// whether a tuned shape exists (in this context or the process-wide table)
-bool bins_tuned(Ctx &cx, Grid &g, const long long dims[3], double eps);
+// Whether a spread in this order reads a tuned tile shape that is not there yet.
+bool spread_wants_tuning(Ctx &cx, Grid &g, const long long dims[3], double eps, SpreadOrder order);
 // Device bytes of the row-factorised projectors of one shared-tilt grid of P
 // projections of R x C on the fine grid of dims: slab: the row group's slabs
 // and halos and the tile spreader's records (kept by the plan, shared by grids

@@ -2234,25 +2234,29 @@ void sysmat_nufft(Ctx &cx, Grid &g, const long long dims[3], double eps, const f
     crop_deapod(cx, pl, y, nullptr, 3, 1.0f / (float)(g.R * g.C), false);
 }
 
-// Times the three-component spreader and interpolator of this grid on the
-// fine grid of `dims` for a list of tile shapes (cubic, and flattened ones for
-// thin or long axes) that fit the LDS budget, and records the fastest in the
-// context's table, where every later spread/interp of the same shapes finds
-// it.  Results do not depend on the tile shape beyond FP32 summation order.
-bool bins_tuned(Ctx &cx, Grid &g, const long long dims[3], double eps) {
+// Chooses tile shapes for this grid on the fine grid of `dims` by timing, and records the
+// fastest in the context's table, where later calls of the same shapes find it.  Timed are the
+// kernels that read the choice.  Shared tilt: the row spreader (MBIR1's and MBIR2's
+// backprojections), and the row interpolator where the forward takes it (widths above 6), for a
+// list of 2-D tilings.  Else the interpolator of the 3-D bins, for cubic shapes and flattened
+// ones for thin or long axes that fit the LDS budget.  Results do not depend on the shape beyond
+// FP32 summation order.
+bool spread_wants_tuning(Ctx &cx, Grid &g, const long long dims[3], double eps, SpreadOrder order) {
     NufftPlan &pl = get_nufft_plan(cx, dims, eps);
+    if (order != SpreadOrder::Rows || !use_rows(g, pl)) return false;   // the tiles read no tuned shape
     std::array<int, 3> T;
-    return lookup_tuned(cx, tune_key(g, pl, 3), T);
+    return !lookup_tuned(cx, tune_key(g, pl, 3), T);
 }
 
 std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], double eps, double *best_ms) {
     NufftPlan &pl = get_nufft_plan(cx, dims, eps);
     if (use_rows(g, pl)) {
-        // The projectors of this grid take the row path: time one spread +
-        // interpolation for each distinct 2-D tiling the candidate edges give (each
-        // with its own point bins), keep the fastest's bins and record its tiling
-        // as (Tz, W, Tx) in the row table; the 3-D table gets the default 3-D tile
-        // so that the grid counts as tuned.
+        // Time each distinct 2-D tiling the candidate edges give (each with its own point
+        // bins) and record the fastest as (Tz, W, Tx) in the row table; the 3-D table gets
+        // the default 3-D tile so that the grid counts as tuned.  The fastest's bins, the
+        // slabs and the halos stay only where the forward uses them.
+        const bool interp_rows = !tile_interp_fits(pl.w);
+        const bool had_slab = pl.slab.bytes > 0, had_halo = pl.halo.bytes > 0;
         ensure_fine(pl, 3);
         const size_t M = (size_t)(g.P * g.R * g.C);
         cx.work[0].ensure(sizeof(float2) * M);
@@ -2283,7 +2287,7 @@ std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], doub
                 for (int rep = 0; rep < 2; ++rep) {
                     LAM_HIP(hipEventRecord(e0, cx.stream));
                     launch_spread(cx, g, pl, cbuf, true, false, false, SpreadOrder::Rows);
-                    launch_interp(cx, g, pl, cbuf, true);
+                    if (interp_rows) launch_interp(cx, g, pl, cbuf, true);
                     LAM_HIP(hipEventRecord(e1, cx.stream));
                     LAM_HIP(hipEventSynchronize(e1));
                     float ms = 0.f;
@@ -2310,6 +2314,11 @@ std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], doub
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         LAM_REQUIRE(best[0] != 0, LAM_ERR_STATE, "no row tiling fits this grid");
+        if (!interp_rows) {
+            g.rowplans.erase(plan_key(best[0], best[2]));
+            if (!had_slab) pl.slab.release();
+        }
+        if (!had_halo) pl.halo.release();
         const BinParams bp = bin_params(cx, g, pl, 3);
         const std::array<int, 3> T3 = {bp.T[0], bp.T[1], bp.T[2]};
         cx.bin_tune[rkey] = best;
@@ -2341,11 +2350,10 @@ std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], doub
         for (const auto &T : kCands) {
             if (!bins_fit(T, pl, 3)) continue;
             cx.bin_tune[key] = {T[0], T[1], T[2]};
-            launch_spread(cx, g, pl, cbuf, true);   // builds this shape's bins
+            launch_interp(cx, g, pl, cbuf, true);   // builds this shape's bins
             float t = 0.f;
             for (int rep = 0; rep < 2; ++rep) {
                 LAM_HIP(hipEventRecord(e0, cx.stream));
-                launch_spread(cx, g, pl, cbuf, true);
                 launch_interp(cx, g, pl, cbuf, true);
                 LAM_HIP(hipEventRecord(e1, cx.stream));
                 LAM_HIP(hipEventSynchronize(e1));

@@ -209,6 +209,41 @@ def test_autotuned_tiles_keep_projector_parity(ctx, orc):
     assert rel(a1, orc.adjoint(proj, dims, al, ga)) < 1e-4
 
 
+@pytest.mark.parametrize("method,det,tunes", [(1, 45, True), (2, 47, True), (3, 49, False)])
+def test_graph_jobs_tune_only_what_they_read(ctx, monkeypatch, capfd, method, det, tunes):
+    """The row tiling is read by MBIR1's and MBIR2's backprojection and by nothing in MBIR3."""
+    from lamino_amd.serve import Server
+
+    monkeypatch.setenv("LAMINO_TUNE_VERBOSE", "1")
+    ds, rd = _job(80 + method, rd=(21, 9, 23), det=det)   # shapes that no other test tunes
+    with Server(slots=1, mode="graph") as s:
+        x, _ = s.wait(s.submit(method, ds, rd, _params(method)))
+    assert np.isfinite(x).all()
+    assert ("row tiling" in capfd.readouterr().err) == tunes
+
+
+def test_tuning_leaves_no_row_slabs_where_nothing_reads_them(ctx):
+    """At width 6 neither projector takes the row path, so the tuner's point bins and slabs (here
+    77 MB) go when it is done."""
+    import ctypes
+
+    import lamino_amd as la
+
+    hip = ctx.lib
+    free0, free1, total = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_size_t()
+    dims, R, C, P = (127, 31, 127), 51, 53, 8
+    pg = la.PolarGrid.per_projection(np.full(P, np.radians(30.0)), 2 * np.pi * np.arange(P) / P, R, C)
+    la.adjoint(np.ones((P, R, C), np.float32), pg, dims)
+    la.forward(np.ones((3,) + dims, np.float32), pg)
+    ctx.sync()
+    assert hip.hipMemGetInfo(ctypes.byref(free0), ctypes.byref(total)) == 0
+    la.autotune_bins(pg, dims)
+    ctx.sync()
+    assert hip.hipMemGetInfo(ctypes.byref(free1), ctypes.byref(total)) == 0
+    say("tuning kept", free0.value - free1.value)
+    assert free0.value - free1.value < 16 << 20
+
+
 def test_row_path_autotuner_chooses_a_tiling_and_keeps_parity(ctx, orc):
     """On the row path (projections sharing the tilt) the autotuner times several 2-D
     tilings of the (z, x) fine plane, each with its own point bins, and keeps the
