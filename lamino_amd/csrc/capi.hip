@@ -257,30 +257,33 @@ size_t mbir_footprint(const lam_dataset *ds, int nds, const long long rd[3], con
     for (int a = 0; a < 3; ++a) od[a] = pad_n(rd[a], vpad);
     const size_t n = (size_t)(od[0] * od[1] * od[2]);
     const double eps = pr.eps > 0 ? pr.eps : 1e-5;
-    size_t nf = 1, lt = 1, tiles = 1;
+    size_t nf = 1, lt = 1;
     for (int a = 0; a < 3; ++a) {
-        const size_t f = nufft_fine_len(od[a], eps);
-        nf *= f;
-        tiles *= (f + 1) / 2;                       // bins are never smaller than 2 cells
+        nf *= nufft_fine_len(od[a], eps);
         lt *= (size_t)toep_len(od[a]);
     }
-    size_t raw = 0, padded = 0, spectra = 0, bintmp = 0, bins = 0, rows_slab = 0;
+    size_t raw = 0, padded = 0, spectra = 0, bintmp = 0, bins = 0, slab = 0, records = 0;
     for (int g = 0; g < nds; ++g) {
         const lam_dataset &D = ds[g];
         const size_t R2 = (size_t)pad_n(D.nrows, dpad), C2 = (size_t)pad_n(D.ncols, dpad);
-        const size_t P = (size_t)D.nproj, M = P * R2 * C2, half = P * ((R2 * C2 + 1) / 2);
+        const size_t P = (size_t)D.nproj, M = P * R2 * C2;
         raw = std::max(raw, 4 * P * (size_t)D.nrows * (size_t)D.ncols);
         padded = std::max(padded, 4 * M);
         spectra = std::max(spectra, 8 * M);
-        // sort keys, the bucket-scattered (cell, index) pairs, bucket offsets and cursors
-        bintmp = std::max(bintmp, 16 * half + 12 * tiles + ((size_t)16 << 20));
-        // sorted ids, chunk list, geometry; twice: the autotuner holds two tile shapes at once
-        bins += 2 * (4 * half + 16 * (half / 1024 + tiles)) + 128 * P;
-        // the row-factorised projectors (grids sharing the tilt; counted for every grid)
-        const RowBytes rb = row_path_bytes(od, eps, (long long)P, (long long)R2, (long long)C2);
-        rows_slab = std::max(rows_slab, rb.slab);
-        bintmp = std::max(bintmp, rb.setup);
-        bins += rb.kept;
+        // the spreader that the job takes: by its method and whether the dataset shares the
+        // tilt (no angles given: either)
+        const bool shared = !D.alpha || std::all_of(D.alpha, D.alpha + P, [&](double a) { return a == D.alpha[0]; });
+        size_t kept = 0;
+        for (const bool s : {true, false}) {
+            if (D.alpha && s != shared) continue;
+            const SpreadBytes sb = spread_bytes(od, eps, (long long)P, (long long)R2, (long long)C2, s,
+                                                pr.method == 3 ? SpreadOrder::Tiles : SpreadOrder::Rows);
+            slab = std::max(slab, sb.slab);
+            records = std::max(records, sb.records);
+            bintmp = std::max(bintmp, sb.setup);
+            kept = std::max(kept, sb.kept);
+        }
+        bins += kept + 128 * P;   // and the geometry
     }
     const size_t fine = 24 * nf;                                   // 3 complex components
     const size_t toep = 24 * lt * (1 + (pr.method == 3 ? (size_t)nds : 0)) + 32 * lt;
@@ -290,7 +293,7 @@ size_t mbir_footprint(const lam_dataset *ds, int nds, const long long rd[3], con
     if (pr.method == 3) solve += 36 * n;                           // xold y g
     const size_t crop = 8 * (size_t)(rd[0] * rd[1] * rd[2]);      // cropped + transposed component
     const size_t slack = 64ull << 20;                              // plans, reductions, twiddles
-    return 12 * n + raw + padded + spectra + bintmp + bins + rows_slab + fine + toep + solve + crop + slack;
+    return 12 * n + raw + padded + spectra + bintmp + bins + slab + records + fine + toep + solve + crop + slack;
 }
 
 }  // namespace lam

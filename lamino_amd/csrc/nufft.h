@@ -136,15 +136,16 @@ void adjoint_multi(Ctx &cx, Grid *const *grids, int ngrids, const long long dims
 std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], double eps, double *best_ms);
 // Whether a spread in this order reads a tuned tile shape that is not there yet.
 bool spread_wants_tuning(Ctx &cx, Grid &g, const long long dims[3], double eps, SpreadOrder order);
-// Device bytes of the row-factorised projectors of one shared-tilt grid of P
-// projections of R x C on the fine grid of dims: slab: the row group's slabs
-// and halos and the tile spreader's records (kept by the plan, shared by grids
-// of the same dims), kept: the grid's point bins, setup: temporaries while
-// they are built.
-struct RowBytes {
-    size_t slab = 0, kept = 0, setup = 0;
+// Upper bounds of the device bytes of one backprojection of a grid of P projections of R x C on
+// the fine grid of dims: slab and records: the row spreader's slabs and halos, the tile
+// spreader's plane records (buffers of the plan, shared by grids of the same dims); kept: the
+// grid's point bins; setup: temporaries while they are built.  shared: the projections share
+// the tilt.
+struct SpreadBytes {
+    size_t slab = 0, records = 0, kept = 0, setup = 0;
 };
-RowBytes row_path_bytes(const long long dims[3], double eps, long long P, long long R, long long C);
+SpreadBytes spread_bytes(const long long dims[3], double eps, long long P, long long R, long long C, bool shared,
+                         SpreadOrder order);
 
 }  // namespace lam
 

@@ -1705,30 +1705,38 @@ int rows_per_group(const RowPlan &rp, const NufftPlan &pl) {
 
 }  // namespace
 
-// Upper bound of what the row path allocates for one grid (see nufft.h).
-RowBytes row_path_bytes(const long long dims[3], double eps, long long P, long long R, long long C) {
+SpreadBytes spread_bytes(const long long dims[3], double eps, long long P, long long R, long long C, bool shared,
+                         SpreadOrder order) {
     NufftPlan pl;   // shapes only
     pl.w = width_for_eps(eps);
     for (int a = 0; a < 3; ++a) pl.nf[a] = (int)nufft_fine_len(dims[a], eps);
-    RowBytes b;
-    if (!row_geom(pl).Tz) return b;
-    const long long H = (R * C + 1) / 2, Jn = (H - 1) / C + 1, half = P * H;
+    Grid g;
+    g.P = P;
+    g.R = R;
+    g.C = C;
+    g.shared_tilt = shared;
+    SpreadBytes b;
+    const bool rows = use_rows(g, pl);
+    if (order == SpreadOrder::Tiles || !rows) {
+        const TileBytes tb = tile_bytes(dims, eps, P, R, C, !rows);
+        b.records = tb.records;
+        b.kept = tb.kept;
+        b.setup = tb.setup;
+        return b;
+    }
+    const size_t Jn = (size_t)half_rows(g), half = (size_t)(P * ((R * C + 1) / 2));
     // the largest over the tilings the autotuner may choose
     for (const auto &t : kRowTileCands) {
         const RowGeom rg = row_geom(pl, t[0], t[1]);
         if (!rg.Tz) continue;
         const size_t per_row = row_slab_bytes(pl) + row_halo_bytes(rg);
-        const size_t groups_rows = std::max<size_t>(1, std::min<size_t>((size_t)Jn, slab_budget() / per_row));
-        b.slab = std::max(b.slab, groups_rows * per_row);
-        const size_t cells = (size_t)Jn * rg.ntiles;
-        // ids, counts + chunks, row weights, the non-empty bit table
-        b.kept = std::max(b.kept, 4 * (size_t)half + 20 * cells + 8 * (size_t)Jn * pl.w + cells / 8 + 4 * rg.ntiles);
+        b.slab = std::max(b.slab, per_row * std::max<size_t>(1, std::min<size_t>(Jn, slab_budget() / per_row)));
+        const size_t cells = Jn * rg.ntiles;
+        // ids, chunks, row weights, the non-empty bit table
+        b.kept = std::max(b.kept, 4 * half + 16 * cells + 8 * Jn * pl.w + cells / 8 + 4 * rg.ntiles);
+        // keys, scattered points, counts, cursors and offsets (SortTmp)
+        b.setup = std::max(b.setup, 12 * half + 12 * cells + 4096);
     }
-    b.setup = 16 * (size_t)half + ((size_t)16 << 20);                // sort keys / spare ids, sort scratch
-    const TileBytes tb = tile_bytes(dims, eps, P, R, C);
-    b.slab += tb.records;
-    b.kept += tb.kept;
-    b.setup = std::max(b.setup, tb.setup);
     return b;
 }
 

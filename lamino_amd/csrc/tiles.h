@@ -89,6 +89,6 @@ void tile_interp(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, float2 *c);
 struct TileBytes {
     size_t kept = 0, setup = 0, records = 0;
 };
-TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long R, long long C);
+TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long R, long long C, bool direct);
 
 }  // namespace lam

@@ -1154,29 +1154,27 @@ bool tile_plan_fits(const Grid &g, const NufftPlan &pl, bool direct) {
     return tile_fits(tile_geom(pl.nf, pl.w, g.R, g.C, direct), g.P * ((g.R * g.C + 1) / 2));
 }
 
-TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long R, long long C) {
+TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long R, long long C, bool direct) {
     NufftPlan pl;   // shapes only
     pl.w = width_for_eps(eps);
     for (int a = 0; a < 3; ++a) pl.nf[a] = (int)nufft_fine_len(dims[a], eps);
     const size_t total = (size_t)P * (size_t)((R * C + 1) / 2);
+    const TileGeom tg = tile_geom(pl.nf, pl.w, R, C, direct);
+    const size_t nb = (size_t)tg.ntiles * tg.nrho, ids = total + 3 * std::min(nb, total);
+    const size_t jobs = tg.ntiles + ids / job_points((long long)total, direct) + 1;
+    // an interpolation job and the next one of its unit hold more points than one may
+    const size_t ujobs = tg.ntiles + 4 * (ids / unit_points((long long)total)) + 1;
+    // a job's planes: its rows' first planes and W - 1 more; the half set spans at most half
+    // the period
+    const size_t planes = (size_t)tg.ntiles * (size_t)(direct ? tg.nfy : tg.nfy / 2 + 2) + jobs * (size_t)pl.w;
+    const size_t largest = record_bytes(tg) * ((size_t)tg.nfy + pl.w);   // of one job
     TileBytes b;
-    for (const bool direct : {false, true}) {
-        const TileGeom tg = tile_geom(pl.nf, pl.w, R, C, direct);
-        const size_t nb = (size_t)tg.ntiles * tg.nrho, ids = total + 3 * std::min(nb, total);
-        const size_t jobs = tg.ntiles + ids / job_points((long long)total, direct) + 1;
-        // an interpolation job and the next one of its unit hold more points than one may
-        const size_t ujobs = tg.ntiles + 4 * (ids / unit_points((long long)total)) + 1;
-        // a job's planes: its rows' first planes and W - 1 more; the half set spans at most half
-        // the period
-        const size_t planes = (size_t)tg.ntiles * (size_t)(direct ? tg.nfy : tg.nfy / 2 + 2) + jobs * (size_t)pl.w;
-        const size_t largest = record_bytes(tg) * ((size_t)tg.nfy + pl.w);   // of one job
-        b.kept = std::max(b.kept, 4 * (ids + nb + tg.ntiles) + sizeof(TileJob) * jobs + sizeof(UnitJob) * ujobs + sizeof(TileGeo) * (size_t)P +
-                                      sizeof(RowY) * tg.nrho + 64 * (size_t)(tg.nfz + tg.nfx) + 4096);
-        b.setup = std::max(b.setup, 8 * total);   // the runs
-        // counts, run offsets and cursors per bucket and scan sums, in the record buffer
-        b.records = std::max(b.records, 17 * nb + 64 * (size_t)tg.ntiles + 65536);
-        b.records = std::max(b.records, std::min(record_bytes(tg) * planes, std::max(record_budget(), largest)));
-    }
+    b.kept = 4 * (ids + nb + tg.ntiles) + sizeof(TileJob) * jobs + sizeof(UnitJob) * ujobs +
+             sizeof(TileGeo) * (size_t)P + sizeof(RowY) * tg.nrho + 64 * (size_t)(tg.nfz + tg.nfx) + 4096;
+    b.setup = 8 * total;   // the runs
+    // counts, run offsets and cursors per bucket and scan sums, in the record buffer
+    b.records = std::max(17 * nb + 64 * (size_t)tg.ntiles + 65536,
+                         std::min(record_bytes(tg) * planes, std::max(record_budget(), largest)));
     return b;
 }
 

@@ -244,6 +244,25 @@ def test_tuning_leaves_no_row_slabs_where_nothing_reads_them(ctx):
     assert free0.value - free1.value < 16 << 20
 
 
+@pytest.mark.parametrize("method", [1, 2, 3])
+@pytest.mark.parametrize("varying", [False, True])
+@pytest.mark.parametrize("eps", [1e-5, 1e-6])
+def test_peak_within_the_estimate_for_each_spreader(ctx, method, varying, eps):
+    """The row spreader, the tile spreader's row slots and its first-cell slots, at both widths."""
+    import dataclasses
+
+    from lamino_amd.serve import Server
+
+    ds, rd = _job(90, rd=(63, 15, 63), nds=2, P=90, det=63)
+    if varying:
+        ds = [(p, a + 0.01 * np.arange(a.size), g) for p, a, g in ds]
+    with Server(slots=1, mode="graph") as s:
+        x, info = s.wait(s.submit(method, ds, rd, dataclasses.replace(_params(method), eps=eps)))
+    say("peak", info["footprint_peak"] >> 20, "of", info["footprint_est"] >> 20, "MiB")
+    assert np.isfinite(x).all()
+    assert 0 < info["footprint_peak"] <= info["footprint_est"]
+
+
 def test_row_path_autotuner_chooses_a_tiling_and_keeps_parity(ctx, orc):
     """On the row path (projections sharing the tilt) the autotuner times several 2-D
     tilings of the (z, x) fine plane, each with its own point bins, and keeps the

@@ -162,3 +162,23 @@ def test_fastdiv_matches_integer_division(tmp_path):
                     os.path.join(ROOT, "tests", "cxx", "test_fastdiv.cpp"), "-o", exe], check=True)
     r = subprocess.run([exe], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
+
+
+# shared-tilt jobs: (volume, detector, projections, datasets) -> MiB of MBIR1, 2, 3 that a server
+# admitted them with when the row spreader was the only one
+ADMITTED_MIB = {((9, 5, 11), 9, 8, 1): (81, 82, 82), ((31, 7, 31), 31, 60, 1): (105, 118, 120),
+                ((63, 15, 63), 63, 90, 2): (315, 421, 469), ((127, 31, 127), 127, 180, 2): (1954, 2823, 3204),
+                ((255, 51, 255), 255, 360, 3): (13905, 21322, 25436),
+                ((511, 51, 511), 511, 360, 2): (43747, 58386, 68315)}
+
+
+@pytest.mark.parametrize("shape", list(ADMITTED_MIB))
+def test_footprints_count_one_spreader(shape):
+    """A job's backprojection takes one spreader, chosen by its method, so its estimate holds that
+    one's memory and not the sum of both."""
+    import lamino_amd as la
+
+    vol, det, P, nds = shape
+    ds = [(np.zeros((P, det, det), np.float32), np.full(P, 0.5), np.zeros(P)) for _ in range(nds)]
+    got = [la.mbir_footprint(m, ds, vol, la.ReconParams()) / 2**20 for m in (1, 2, 3)]
+    assert all(g <= w + 1 for g, w in zip(got, ADMITTED_MIB[shape])), got
