@@ -44,8 +44,9 @@ if _queues < 8:
 
 METRIC = "fwd+adj NUFFT projections/s, CG iters/s vs plain form; p50/p99 recon latency"
 HBM_PEAK_GBS = 8000.0
-KERNEL_SCOPES = ("interp", "spread", "fft_axis", "deapod_pad", "crop_deapod", "bin_points", "spread_rows2d",
-                 "y_expand", "y_contract", "interp_rows2d", "toep_mul", "toep_xfused")
+FP32_MATRIX_PEAK_TFLOPS = 157.3
+KERNEL_SCOPES = ("interp", "spread", "fft_axis", "deapod_pad", "crop_deapod", "bin_points", "tile_spread",
+                 "tile_merge", "tile_interp", "toep_mul", "toep_xfused")
 
 
 def parse():
@@ -148,12 +149,6 @@ class Projectors:
         self.m = m
         self.md = self.ctx.to_device(m)
         self.grids = [la.PolarGrid.per_projection(s.alpha, s.gamma, self.det, self.det) for s in work.scans]
-        # the row tiling of the projectors, chosen by timing candidates on the first dataset's
-        # grid (the others share its shapes and take the same tiling)
-        t0 = time.perf_counter()
-        tile, tile_ms = la.autotune_bins(self.grids[0], self.vol)
-        self.tuning = {"row_tiling": [tile[0], tile[2]], "spread_interp_ms": round(tile_ms, 3),
-                       "tuning_s": round(time.perf_counter() - t0, 3)}
         self.projs = [self.ctx.alloc((self.P, self.det, self.det), np.float32) for _ in range(self.G)]
         self.grid_arr = (ctypes.c_void_p * self.G)(*[g.h for g in self.grids])
         self.proj_arr = (ctypes.c_void_p * self.G)(*[p.ptr for p in self.projs])
@@ -178,7 +173,7 @@ class Projectors:
         from lamino_amd import _lib
 
         lib, ctx = self.ctx.lib, self.ctx
-        # the first step builds every grid's point bins (key, bucket scatter, in-bucket order)
+        # the first step builds every grid's point plan (runs, order, shares)
         _lib.check(lib.lam_timing_enable(ctx.h, 1))
         _lib.check(lib.lam_timing_only(ctx.h, b"bin_points"))
         self.step()
@@ -283,28 +278,33 @@ def roofline(pr, kernels, spread_ms, spread_cnt, workload_key):
     out = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
            "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": hbm_traffic_from_profiles("spread", workload_key),
            "kernel": "spread", "bytes_per_launch": bytes_alg, "avg_launch_ms": round(avg_ms, 4)}
-    # The roofs that bind the row-factorised kernels: per half-plane point the 2-D spreader
-    # read-modify-writes W^2 cells x 3 complex components (2 x 24 B each) in its LDS box and
-    # the 2-D interpolator reads them once (LDS roof; peak = 256 CUs x 128 B/clk x 2.4 GHz,
-    # an estimate from the CU's LDS width, not a published figure); the y passes stream the
-    # row slabs and the fine grid (HBM roof).
+    # The roofs of the tile kernels (kernel width 6).  The spreader takes two half-plane points
+    # per 32 x 32 x 2 FP32 matrix product; its vector instructions share the SIMDs with those,
+    # so the matrix roof alone is not all that binds it.  The interpolator reads W^2 cells of
+    # three complex values per point from LDS (peak = 256 CUs x 128 B/clk x 2.4 GHz, an estimate
+    # from the CU's LDS width, not a published figure).  The merge streams the recorded planes
+    # and the fine grid; its bytes are those that the counters read in the committed profile.
     w = 6
     half_points = P * ((det * det + 1) // 2)
-    rows = ((det * det + 1) // 2 - 1) // det + 1
-    slab = nf[0] * nf[2] * 24
     lds_peak_tbs = 256 * 128 * 2.4e9 / 1e12
     binding = {}
-    for k, per_pt in (("spread_rows2d", 2 * 24 * w ** 2), ("interp_rows2d", 24 * w ** 2)):
-        if k in kernels:
-            n_launch = kernels[k]["launches"] / max(1, kernels["spread" if k.startswith("spread") else "interp"]["launches"])
-            tbs = half_points * per_pt / (kernels[k]["avg_ms"] * n_launch / 1e3) / 1e12
-            binding[k] = {"roof": "lds", "achieved_tbs": round(tbs, 2), "peak_tbs": round(lds_peak_tbs, 1),
-                          "frac": round(tbs / lds_peak_tbs, 3)}
-    for k, nbytes in (("y_contract", Nfine * 24 + rows * slab), ("y_expand", rows * slab + Nfine * 24)):
-        if k in kernels:
-            n_launch = kernels[k]["launches"] / max(1, kernels["spread" if k == "y_expand" else "interp"]["launches"])
-            gbs = nbytes / (kernels[k]["avg_ms"] * n_launch / 1e3) / 1e9
-            binding[k] = {"roof": "hbm", "achieved_gbs": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 3)}
+
+    def per_call(k, whole):
+        """ms of kernel k in one call of the operation `whole`."""
+        return kernels[k]["avg_ms"] * kernels[k]["launches"] / max(1, kernels[whole]["launches"])
+
+    if "tile_spread" in kernels:
+        tf = half_points * 2 * 32 * 32 / (per_call("tile_spread", "spread") / 1e3) / 1e12
+        binding["tile_spread"] = {"roof": "fp32 matrix", "achieved_tflops": round(tf, 1),
+                                  "peak_tflops": FP32_MATRIX_PEAK_TFLOPS, "frac": round(tf / FP32_MATRIX_PEAK_TFLOPS, 3)}
+    if "tile_interp" in kernels:
+        tbs = half_points * 24 * w ** 2 / (per_call("tile_interp", "interp") / 1e3) / 1e12
+        binding["tile_interp"] = {"roof": "lds", "achieved_tbs": round(tbs, 2), "peak_tbs": round(lds_peak_tbs, 1),
+                                  "frac": round(tbs / lds_peak_tbs, 3)}
+    merged = hbm_traffic_from_profiles("tile_merge", workload_key)
+    if "tile_merge" in kernels and merged:
+        gbs = merged / (per_call("tile_merge", "spread") / 1e3) / 1e9
+        binding["tile_merge"] = {"roof": "hbm", "achieved_gbs": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 3)}
     out["binding"] = binding
     return out
 
@@ -317,12 +317,18 @@ def run_recon(la, synth, work, graph: bool):
 
     datasets, _ = synth.simulate(work, project)
     prm = synth.recon_params(work)
+    tiling = None
+    if work.method != 3:   # the row spreader's tiling, which the graph form picks by timing too
+        vol, det = work.solver_shapes()
+        scan = work.scans[0]
+        tile, _ = la.autotune_bins(la.PolarGrid.per_projection(scan.alpha, scan.gamma, det, det), vol)
+        tiling = [tile[0], tile[2]]
     tr0 = time.perf_counter()
     rec, st = la.api._mbir(work.method, datasets, work.recon_dims, prm, stats=True)
     tr = time.perf_counter() - tr0
     out = {"method": f"MBIR{work.method}", "recon_s": round(tr, 4), "setup_s": round(st["setup_s"], 4),
            "solve_s": round(st["solve_s"], 4), "normal_ops": st["normal_ops"], "cg_iters": st["cg_iters"],
-           "outer_iters": st["outer_iters"], "finite": bool(np.isfinite(rec).all())}
+           "outer_iters": st["outer_iters"], "finite": bool(np.isfinite(rec).all()), "row_tiling": tiling}
     if work.method == 3:
         out["s_per_iteration"] = round(st["solve_s"] / max(1, st["outer_iters"]), 5)
         out["lipschitz"] = st["lipschitz"]
@@ -485,8 +491,7 @@ WORKLOAD_KEY = {1: "plain_cg_89x21x89_det89", 2: "split_bregman_179x43x179_det30
 def describe(work, pr):
     return (f"{work.name}; padded volume {list(pr.vol)}, detector {pr.det}x{pr.det}, {pr.G} x {pr.P} projections; "
             "step = forward of all datasets (one shared fine-grid transform) + adjoint of each (3 components); "
-            "row tiling autotuned and point binning "
-            "built once per grid before the timed steps")
+            "point plans built once per grid before the timed steps")
 
 
 def main():
@@ -536,8 +541,8 @@ def main():
         cpu = cpu_baseline(pr, args.cpu_projections or {1: 24, 2: 12, 3: 4}[args.config])
         log("cpu:", cpu)
     head = {"workload": describe(work, pr), "padded_volume": list(pr.vol), "detector": pr.det, "datasets": pr.G,
-            "projections": pr.P, "nufft_eps": la.api.DEFAULT_EPS, "point_binning": "cached per grid (built by the autotuner and in warmup)",
-            "bin_build_ms": pr.bin_ms, "autotune": pr.tuning}
+            "projections": pr.P, "nufft_eps": la.api.DEFAULT_EPS, "point_binning": "cached per grid (built in warmup)",
+            "bin_build_ms": pr.bin_ms}
     kernels_ms = {k: round(v["total_ms"] / diag_steps, 4) for k, v in kernels.items()}
     pr.release()
 
@@ -549,7 +554,7 @@ def main():
         p2 = Projectors(la, w)
         ms2, _, _ = p2.timed(max(5, args.steps), args.warmup)
         extra[f"config{ci}"] = {"workload": describe(w, p2), "projections_per_s": round(p2.G * p2.P / (ms2 / 1e3), 2),
-                                "ms_per_step": round(ms2, 4), "autotune": p2.tuning, **p2.cg(args.cg_iters)}
+                                "ms_per_step": round(ms2, 4), **p2.cg(args.cg_iters)}
         log(f"config {ci}:", extra[f"config{ci}"])
         p2.release()
 

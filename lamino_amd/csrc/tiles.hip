@@ -1329,7 +1329,7 @@ void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c,
     for (size_t k = 0; k < groups.size(); ++k) {
         const unsigned j0 = groups[k].first, j1 = k + 1 < groups.size() ? groups[k + 1].first : tp.njobs;
         if (j1 > j0) {
-            TimedScope ts(cx, "spread_rows2d");
+            TimedScope ts(cx, "tile_spread");
             const dim3 grid((j1 - j0) * (unsigned)(3 / tile_comps(pl.w)));
 #define LAM_TILE_SPREAD(DIRECT)                                                                                  \
     LAM_TILE_WIDTH(pl.w, hipLaunchKernelGGL((k_tile_spread<W, tile_comps(W), DIRECT>), grid, dim3(64), 0, cx.stream, \
@@ -1344,7 +1344,7 @@ void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c,
 #undef LAM_TILE_SPREAD
             check_launch();
         }
-        TimedScope ts(cx, "y_expand");
+        TimedScope ts(cx, "tile_merge");
         const dim3 mgrid((unsigned)((3 * tg.nfx + 255) / 256) * (unsigned)tg.nfz *
                          (unsigned)((ly + kMergePlanes - 1) / kMergePlanes));
         LAM_TILE_WIDTH(pl.w, hipLaunchKernelGGL((k_tile_merge<tile_comps(W)>), mgrid, dim3(256), 0, cx.stream,
@@ -1362,7 +1362,7 @@ bool tile_interp_fits(int w) { return w <= 6; }
 void tile_interp(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, float2 *c) {
     const TileGeom &tg = tp.tg;
     const TileArgs a = tile_args(g, pl);
-    TimedScope ts(cx, "interp_rows2d");
+    TimedScope ts(cx, "tile_interp");
     const int nr = unit_rows(tp, g.P * ((g.R * g.C + 1) / 2));
     const size_t lds = (size_t)nr * kUnitCells * 3 * sizeof(float2);
     auto allow = [&](auto k) {
