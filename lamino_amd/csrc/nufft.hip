@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <mutex>
 #include <string>
 
@@ -1569,6 +1570,13 @@ bool use_rows(const Grid &g, const NufftPlan &pl) {
     return rows_fit(g, row_geom(pl)) && tile_plan_fits(g, pl, false);
 }
 
+// LAMINO_NUFFT_ROWS=spread: every adjoint of a grid that has a row form takes the row spreader
+// (MBIR1's and MBIR2's), which no projector call reaches otherwise.
+bool rows_spread_asked() {
+    const char *e = std::getenv("LAMINO_NUFFT_ROWS");
+    return e && std::strcmp(e, "spread") == 0;
+}
+
 // Tile edge targets (z, x) the row-path autotuner times; the first is the untuned default.
 // (Measured, spread + interpolation of one dataset: at (359, 71, 359) / 615 x 615, 360
 // projections, 12 x 15 9.73 ms against 10.11 for the default 16 x 15 and 11.00 for 24 x 20;
@@ -1856,7 +1864,7 @@ void interp_w(Ctx &cx, Grid &g, NufftPlan &pl, float2 *c, const BinParams &bp, S
 // order: which of the three-component spreaders (see SpreadOrder)
 void launch_spread(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, bool half, bool paired = false,
                    bool add = false, SpreadOrder order = SpreadOrder::Tiles) {
-    if (half && order == SpreadOrder::Rows && use_rows(g, pl)) {
+    if (half && (order == SpreadOrder::Rows || rows_spread_asked()) && use_rows(g, pl)) {
         RowPlan &rp = get_rowplan(cx, g, pl);
         // One row group whose y window does not wrap writes every plane of the window
         // once, and the transforms that follow read only the window: no zeroing.
