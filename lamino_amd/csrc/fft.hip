@@ -78,7 +78,7 @@ struct KParams {
     int rad[24], st_len[24], st_sign[24], st_g[24], st_ns[24], st_tw[24];
     const float2 *tw;                     // the plan's twiddle tables (stage s from st_tw[s])
     const float2 *chirp, *bhat;
-    FastDiv fL, fN, fM, fLi, fPad;        // tile lines, length, inner length, lines per o2 row, M - N
+    FastDiv fL, fM, fLi, fPad;            // tile lines, inner length, lines per o2 row, M - N
     FastDiv fNbf[24], fNs[24];            // per stage: butterflies per line (len / R), span Ns
     int isn, osn;                         // element strides along the transform (fit 32 bits)
     // Rader plans: n = S * Q; the S-point transforms run over the Q columns of
@@ -429,14 +429,6 @@ __device__ __forceinline__ void rader_pointwise(float2 *buf, const KParams &P) {
 }
 
 __device__ __forceinline__ int remap(int o, int split, int gap) { return o < split ? o : o + gap; }
-
-// position m in the cyclic window [lo, lo + len) of a length-n line (len 0: no window)
-__device__ __forceinline__ bool in_window(int m, int lo, int len, int n) {
-    if (len <= 0) return true;
-    int d = m - lo;
-    if (d < 0) d += n;
-    return d < len;
-}
 
 // The tile of this workgroup, numbered per XCD (xcd_order): consecutive tiles along
 // the contiguous index share cache lines in the inner-index passes (four 615-point
@@ -1070,7 +1062,6 @@ void run_axis(Ctx &cx, const FftPlan &plan, AxisPass a) {
     P.isn = (int)a.isn;
     P.osn = (int)a.osn;
     P.fL = FastDiv((unsigned)P.L);
-    P.fN = FastDiv((unsigned)plan.n);
     P.fM = FastDiv((unsigned)plan.m);
     P.fLi = FastDiv((unsigned)P.Li);
     P.fPad = FastDiv((unsigned)std::max(1, plan.m - plan.n));

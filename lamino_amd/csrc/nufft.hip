@@ -267,20 +267,17 @@ __device__ __forceinline__ long long box_to_fine(const TileBox &b, const BinPara
 constexpr int kStage = 128;   // points staged per batch
 
 // Staged point record, in 32-bit words: [0] box cell of the point's first
-// kernel cell, [1] parity bits (lz & 1) | (ly & 1) << 1, [4, 4 + 2 NC) the NC
-// complex values, then wz[W], wy[W], wx[W].  Records are 16-byte aligned.
-template <int W, int NC>
+// kernel cell, [1] parity bits (lz & 1) | (ly & 1) << 1, [4, 6) the complex
+// value, then wz[W], wy[W], wx[W].  Records are 16-byte aligned.
+template <int W>
 struct StageLayout {
     static constexpr int VQ = 4;
-    static constexpr int WZ = VQ + 2 * NC;
+    static constexpr int WZ = VQ + 2;
     static constexpr int WY = WZ + W;
     static constexpr int WX = WY + W;
     static constexpr int SW = (WX + W + 3) / 4 * 4;
     static_assert(W % 2 == 0 && WZ % 2 == 0, "weight pairs must be 8-byte aligned");
 };
-
-template <int W, int NC>
-constexpr int stage_words() { return StageLayout<W, NC>::SW; }
 
 template <int W>
 __global__ __launch_bounds__(256) void k_spread_tiled(float2 *__restrict__ fine, const float2 *__restrict__ c,
@@ -288,8 +285,8 @@ __global__ __launch_bounds__(256) void k_spread_tiled(float2 *__restrict__ fine,
                                                       int nfz, int nfy, int nfx, float beta, PointFrame fr,
                                                       BinParams bp, const unsigned *__restrict__ ids,
                                                       const uint4 *__restrict__ chunks) {
-    constexpr int NC = 1;
-    using SL = StageLayout<W, NC>;
+    constexpr int NC = 1;   // the three-component form is the tile spreader's
+    using SL = StageLayout<W>;
     constexpr int SW = SL::SW;
     constexpr int HW = W / 2;
     constexpr int NOWN = HW * HW * W;     // cells of one point owned by one wave
@@ -856,11 +853,11 @@ __device__ __forceinline__ Box2 box2(unsigned jt, int j0, const RowGeom &rg) {
 
 // Points per (row, tile) average ~140 at the benchmark shape: 128 threads per
 // workgroup (measured: 0.47 ms per launch at 256 threads, 0.43 at 128).  The
-// occupancy hint has the compiler fit the kernel in fewer registers (W = 6: 63
-// VGPRs instead of 112, 8 waves per SIMD, which the LDS allows): 0.343 -> 0.290
-// ms.  Width 4 takes a hint of 5 and widths from 12 none, where 6 would spill.
+// occupancy hint has the compiler fit the kernel in fewer registers (measured at
+// W = 6: 63 VGPRs instead of 112, 0.343 -> 0.290 ms).  Width 12 takes none,
+// where 6 would spill.
 constexpr int kRowsInterpThreads = 128;
-constexpr int rows_interp_waves(int W) { return W == 4 ? 5 : W >= 12 ? 1 : 6; }
+constexpr int rows_interp_waves(int W) { return W >= 12 ? 1 : 6; }
 
 // type 2, step 2: the chunk's 2-D box of its row's slab is staged in LDS
 // ([ncell][3]); each point gathers W^2 x 3 values and writes sum_i d_i c_i and
@@ -1332,7 +1329,7 @@ size_t box_cells(const int T[3], int w) {
 }
 
 size_t spread_lds_bytes(const int T[3], int w, int nc) {
-    const size_t sw = (size_t)(4 + 2 * nc + 3 * w + 3) / 4 * 4;   // StageLayout<w, nc>::SW
+    const size_t sw = (size_t)(4 + 2 * nc + 3 * w + 3) / 4 * 4;   // the spreader's staged record, nc values
     return box_cells(T, w) * nc * 8 + (size_t)kStage * sw * 4;
 }
 
@@ -1567,7 +1564,7 @@ bool use_rows(const Grid &g, const NufftPlan &pl) {
     if (!g.shared_tilt) return false;
     const char *e = std::getenv("LAMINO_NUFFT_ROWS");
     if (e && e[0] == '0') return false;
-    return rows_fit(g, row_geom(pl)) && tile_plan_fits(g, pl, false);
+    return rows_fit(g, row_geom(pl));
 }
 
 // LAMINO_NUFFT_ROWS=spread: every adjoint of a grid that has a row form takes the row spreader
@@ -1903,7 +1900,7 @@ void launch_interp(Ctx &cx, Grid &g, NufftPlan &pl, float2 *c, bool half) {
     if (half && use_rows(g, pl)) {
         RowPlan &rp = get_rowplan(cx, g, pl);
         TimedScope ts(cx, "interp");
-        LAM_WIDTH_SWITCH(pl.w, (interp_rows_w<W>(cx, g, pl, c, rp)));
+        LAM_WIDTH_SWITCH(pl.w, if constexpr (W > 6) interp_rows_w<W>(cx, g, pl, c, rp));   // narrower ones: tiles
         return;
     }
     const BinParams bp = bin_params(cx, g, pl, nc);

@@ -8,9 +8,11 @@ namespace lam {
 struct TileGeo;   // tiles.hip
 struct RowY;
 
-// Cutting of the (z, x) plane into tiles whose first-cell edges Tz x Tx leave room for the
-// kernel inside one 16 x 16 matrix-core block (T + W - 1 <= 16).  Tile (tz, tx) owns the
-// points whose first kernel cell lies in [tz Tz, (tz + 1) Tz) x [tx Tx, (tx + 1) Tx).
+// Cutting of the (z, x) plane into tiles of Tz x Tx first cells.  Tile (tz, tx) owns the points
+// whose first kernel cell lies in [tz Tz, (tz + 1) Tz) x [tx Tx, (tx + 1) Tx).  With its halo a
+// tile fits one 32 x 32 matrix-core block of (z, re/im) rows and (x, component) columns: 16 z
+// cells (Tz + W - 1 <= 16), and in x 10 cells of three components or, for widths above 8, 32
+// cells of one.
 struct TileGeom {
     int W = 0;
     int Tz = 0, Tx = 0, ntz = 0, ntx = 0;
@@ -69,9 +71,6 @@ struct TilePlan {
 
 // The y planes [ylo, ylo + ly) (mod nfy) that the rows of a shared-tilt grid touch (ly 0: all).
 void row_window(const Grid &g, const NufftPlan &pl, int &ylo, int &ly);
-
-// Whether the plan's buckets and point list have 32-bit numbers.
-bool tile_plan_fits(const Grid &g, const NufftPlan &pl, bool direct);
 
 TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct);
 

@@ -1000,7 +1000,8 @@ TileGeom tile_geom(const int nf[3], int W, long long R, long long C, bool direct
 }
 
 // Whether the buckets and the padded point list (up to 3 fillers per non-empty bucket) have
-// 32-bit numbers.
+// 32-bit numbers.  What the row form and the 3-D bins took always fits: fewer than 2^31 points,
+// and at most 2^32 cells per row (or of the fine grid) for tiles of 27 or more.
 bool tile_fits(const TileGeom &tg, long long total) {
     const long long nb = (long long)tg.ntiles * tg.nrho;
     return nb < (1ll << 31) - kScanBlock && total + 3 * std::min(nb, total) < (1ll << 32);
@@ -1148,10 +1149,6 @@ void row_window(const Grid &g, const NufftPlan &pl, int &ylo, int &ly) {
         ylo = ((lo % pl.nf[1]) + pl.nf[1]) % pl.nf[1];
         ly = len;
     }
-}
-
-bool tile_plan_fits(const Grid &g, const NufftPlan &pl, bool direct) {
-    return tile_fits(tile_geom(pl.nf, pl.w, g.R, g.C, direct), g.P * ((g.R * g.C + 1) / 2));
 }
 
 TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long R, long long C, bool direct) {
@@ -1364,12 +1361,8 @@ void tile_interp(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, float2 *c) {
     const TileArgs a = tile_args(g, pl);
     TimedScope ts(cx, "tile_interp");
     const int nr = unit_rows(tp, g.P * ((g.R * g.C + 1) / 2));
+    static_assert(sizeof(float2) * 3 * kUnitRows * kUnitCells <= 64 * 1024, "no larger LDS limit to ask for");
     const size_t lds = (size_t)nr * kUnitCells * 3 * sizeof(float2);
-    auto allow = [&](auto k) {
-        if (lds > 64 * 1024)
-            LAM_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    };
-    allow(pl.w == 4 ? &k_tile_interp<4> : &k_tile_interp<6>);
 #define LAM_TILE_INTERP(WW)                                                                                         \
     hipLaunchKernelGGL((k_tile_interp<WW>), dim3(tp.nujobs), dim3(kUnitThreads), lds, cx.stream, pl.fine.as<float2>(), \
                        c, tp.geo, tp.off, tp.ids.as<unsigned>(), tp.rowy,   \
