@@ -490,13 +490,15 @@ struct Ranges {
 // A thread's lines and positions.  INNER: it stays on line tid % L and takes every (NT / L)-th
 // position (the threads past a whole number of rows of L idle: one of 256 at L = 17, 16 at
 // L = 48), so that a row of the tile is loaded contiguously; otherwise a wave takes every
-// fourth line, its lanes along the line.  Positions are a constant step apart: an element costs
+// fourth line, its lanes along the line, or several lines side by side when they are at most 32
+// long (with 64 lanes on a line of 13, the adjoint of 94 x 18 x 94 / 270 x 13 x 212 took 197 us
+// instead of 172).  Positions are a constant step apart: an element costs
 // an addition to its address.  Numbering the tile's elements instead cost each of them two index
 // divisions, the range tests and a 64-bit product, about half of the vector instructions of
 // these passes, which kept 70 to 98 % of the issue slots busy at the larger grids: the passes of
 // the normal operator at 359 x 71 x 359 went from 1591 to 1408 us, those of the three-dataset
 // adjoint there (615 x 615 detector) from 3209 to 2927 us.
-template <int INNER, int NT>
+template <int INNER, int NT, bool SHORT>
 struct TileThread {
     int l, l_step, row, rows;
     __device__ __forceinline__ explicit TileThread(const KParams &P) {
@@ -505,6 +507,12 @@ struct TileThread {
             row = (int)P.fL.div(threadIdx.x);
             l = row < rows ? (int)threadIdx.x - row * P.L : P.L;
             l_step = P.L;
+        } else if (SHORT) {
+            const int bits = P.n <= 8 ? 3 : P.n <= 16 ? 4 : 5;   // of the lanes on a line
+            rows = 1 << bits;
+            row = (int)threadIdx.x & (rows - 1);
+            l = (int)threadIdx.x >> bits;
+            l_step = NT >> bits;
         } else {
             rows = 64;
             row = (int)(threadIdx.x & 63);
@@ -517,14 +525,14 @@ struct TileThread {
 // Loads the tile: each thread issues the global loads of kLoadBatch elements before it writes
 // any to LDS (one at a time, the passes ran at a latency-bound ~2 TB/s).  Positions outside the
 // ranges read as zero.
-template <int INNER, int NT, int MODE>
+template <int INNER, int NT, int MODE, bool SHORT>
 __device__ __forceinline__ void load_tile(float2 *__restrict__ buf, const KParams &P, int kind, const Ranges &rg,
                                           const long long *base_in, const short *pos, bool has2) {
     constexpr bool CPLX = MODE == LD_COMPLEX || MODE == LD_COMPLEX_PAIR;
     using T = std::conditional_t<CPLX, float2, float>;
     const AxisPass &a = P.a;
     const int L = P.L, M = P.m, N = P.n;
-    const TileThread<INNER, NT> tt(P);
+    const TileThread<INNER, NT, SHORT> tt(P);
     for (int l = tt.l; l < L; l += tt.l_step) {
         const long long lb = base_in[l];
         if (lb < 0) continue;
@@ -573,13 +581,13 @@ __device__ __forceinline__ void load_tile(float2 *__restrict__ buf, const KParam
 }
 
 // Stores the tile, kLoadBatch LDS reads at a time.
-template <int INNER, int NT, int MODE>
+template <int INNER, int NT, int MODE, bool SHORT>
 __device__ __forceinline__ void store_tile(const float2 *__restrict__ buf, const KParams &P, int kind,
                                            const Ranges &rg, const long long *base_out, const short *pos, bool put2) {
     using T = std::conditional_t<MODE == ST_COMPLEX, float2, float>;
     const AxisPass &a = P.a;
     const int L = P.L, M = P.m, N = P.n;
-    const TileThread<INNER, NT> tt(P);
+    const TileThread<INNER, NT, SHORT> tt(P);
     for (int l = tt.l; l < L; l += tt.l_step) {
         const long long lb = base_out[l];
         if (lb < 0) continue;
@@ -623,8 +631,8 @@ __device__ __forceinline__ void store_tile(const float2 *__restrict__ buf, const
 
 // DQ != 0: the instantiation for qdirect plans with prime factor Q = DQ (the S-point
 // stages, then direct_q_stage); its own kernel so that the other plans' passes keep
-// their register allocation.
-template <int INNER, int NT, int MAXLEN, int WAVES, int DQ = 0>
+// their register allocation.  SHORT: the one for contiguous lines of at most 32 points.
+template <int INNER, int NT, int MAXLEN, int WAVES, int DQ = 0, bool SHORT = false>
 __global__ __launch_bounds__(NT, WAVES) void k_fft_axis(KParams P) {
     extern __shared__ float2 buf[];
     const int kind = DQ ? (int)KIND_RADER : P.kind;
@@ -657,10 +665,10 @@ __global__ __launch_bounds__(NT, WAVES) void k_fft_axis(KParams P) {
 
     const Ranges rin(nv, a.nv2, a.ld_lo, a.ld_len, N), rout(ns, a.ns2, a.st_lo, a.st_len, N);
     switch (a.ld_mode) {
-        case LD_COMPLEX: load_tile<INNER, NT, LD_COMPLEX>(buf, P, kind, rin, base_in, pos_lds, has2); break;
-        case LD_REAL: load_tile<INNER, NT, LD_REAL>(buf, P, kind, rin, base_in, pos_lds, has2); break;
-        case LD_REAL_PAIR: load_tile<INNER, NT, LD_REAL_PAIR>(buf, P, kind, rin, base_in, pos_lds, has2); break;
-        default: load_tile<INNER, NT, LD_COMPLEX_PAIR>(buf, P, kind, rin, base_in, pos_lds, has2); break;
+        case LD_COMPLEX: load_tile<INNER, NT, LD_COMPLEX, SHORT>(buf, P, kind, rin, base_in, pos_lds, has2); break;
+        case LD_REAL: load_tile<INNER, NT, LD_REAL, SHORT>(buf, P, kind, rin, base_in, pos_lds, has2); break;
+        case LD_REAL_PAIR: load_tile<INNER, NT, LD_REAL_PAIR, SHORT>(buf, P, kind, rin, base_in, pos_lds, has2); break;
+        default: load_tile<INNER, NT, LD_COMPLEX_PAIR, SHORT>(buf, P, kind, rin, base_in, pos_lds, has2); break;
     }
     if (kind == KIND_BLUESTEIN) {
         const int pad = M - N;
@@ -717,10 +725,10 @@ __global__ __launch_bounds__(NT, WAVES) void k_fft_axis(KParams P) {
     }
 
     switch (a.st_mode) {
-        case ST_COMPLEX: store_tile<INNER, NT, ST_COMPLEX>(buf, P, kind, rout, base_out, pos_lds, put2); break;
-        case ST_REAL: store_tile<INNER, NT, ST_REAL>(buf, P, kind, rout, base_out, pos_lds, put2); break;
-        case ST_IMAG: store_tile<INNER, NT, ST_IMAG>(buf, P, kind, rout, base_out, pos_lds, put2); break;
-        default: store_tile<INNER, NT, ST_REAL_PAIR>(buf, P, kind, rout, base_out, pos_lds, put2); break;
+        case ST_COMPLEX: store_tile<INNER, NT, ST_COMPLEX, SHORT>(buf, P, kind, rout, base_out, pos_lds, put2); break;
+        case ST_REAL: store_tile<INNER, NT, ST_REAL, SHORT>(buf, P, kind, rout, base_out, pos_lds, put2); break;
+        case ST_IMAG: store_tile<INNER, NT, ST_IMAG, SHORT>(buf, P, kind, rout, base_out, pos_lds, put2); break;
+        default: store_tile<INNER, NT, ST_REAL_PAIR, SHORT>(buf, P, kind, rout, base_out, pos_lds, put2); break;
     }
 }
 
@@ -1119,6 +1127,9 @@ void run_axis(Ctx &cx, const FftPlan &plan, AxisPass a) {
     } else if (plan.m <= kLdsComplex) {
         if (inner)
             hipLaunchKernelGGL((k_fft_axis<1, kThreads, kLdsComplex, kFftWaves>), grid, dim3(kThreads), lds, cx.stream, P);
+        else if (plan.n <= 32)
+            hipLaunchKernelGGL((k_fft_axis<0, kThreads, kLdsComplex, kFftWaves, 0, true>), grid, dim3(kThreads), lds,
+                               cx.stream, P);
         else
             hipLaunchKernelGGL((k_fft_axis<0, kThreads, kLdsComplex, kFftWaves>), grid, dim3(kThreads), lds, cx.stream, P);
     } else {

@@ -24,3 +24,16 @@ def test_fft2_at_tile_edges(ctx, orc, shape, shifted):
     x64 = x.astype(np.complex128)
     want = orc.shift2(np.fft.fft2(orc.shift2(x64, inverse=False)), inverse=True) if shifted else np.fft.fft2(x64)
     assert rel(la.fft2(x, -1, shifted=shifted), want) < 6 * 2**-24 * (1 + np.log2(shape[1] * shape[2]))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 4, 7, 8, 9, 13, 15, 16, 17, 23, 31, 32, 33, 34, 41, 63, 64, 65])
+@pytest.mark.parametrize("planes,rows", [(1, 5), (3, 37), (7, 130)])
+def test_short_contiguous_lines(ctx, orc, planes, rows, n):
+    """Lines of up to 32 points share a wave, eight to thirty-two lanes each; one longer and the
+    last partial tile.  The bound is that of the test above."""
+    import lamino_amd as la
+
+    say("short lines", planes, rows, n)
+    rng = np.random.default_rng(8)
+    x = (rng.standard_normal((planes, rows, n)) + 1j * rng.standard_normal((planes, rows, n))).astype(np.complex64)
+    assert rel(la.fft2(x, -1), np.fft.fft2(x.astype(np.complex128))) < 6 * 2**-24 * (1 + np.log2(rows * n))
