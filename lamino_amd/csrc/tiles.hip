@@ -1089,6 +1089,14 @@ size_t record_budget() {
     return (size_t)8 << 30;
 }
 
+// Room made for `need` bytes of records: up to an eighth more, within the budget, so that the next
+// grid of the shape, whose jobs record a little more or less, finds it large enough.
+size_t record_room(size_t need) {
+    size_t step = 1 << 16;
+    while (16 * step <= need) step *= 2;
+    return std::max(need, std::min((need + step - 1) / step * step, record_budget()));
+}
+
 TileArgs tile_args(const Grid &g, const NufftPlan &pl) {
     TileArgs a;
     a.S = g.R * g.C;
@@ -1170,8 +1178,8 @@ TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long
              sizeof(TileGeo) * (size_t)P + sizeof(RowY) * tg.nrho + 64 * (size_t)(tg.nfz + tg.nfx) + 4096;
     b.setup = 8 * total;   // the runs
     // counts, run offsets and cursors per bucket and scan sums, in the record buffer
-    b.records = std::max(17 * nb + 64 * (size_t)tg.ntiles + 65536,
-                         std::min(record_bytes(tg) * planes, std::max(record_budget(), largest)));
+    b.records = record_room(std::max(17 * nb + 64 * (size_t)tg.ntiles + 65536,
+                                     std::min(record_bytes(tg) * planes, std::max(record_budget(), largest))));
     return b;
 }
 
@@ -1257,7 +1265,7 @@ TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
                  oucount = cs.take(sizeof(unsigned long long) * tp->nunits),
                  oujob0 = cs.take(sizeof(unsigned) * (tp->nunits + 1ull)),
                  ouhigh = cs.take(sizeof(unsigned) * (tp->nunits + 1ull));
-    pl.rec.ensure(cs.bytes);
+    if (pl.rec.bytes < cs.bytes) pl.rec.ensure(record_room(cs.bytes));
     const DevBuf &tmp = pl.rec;
     auto *count = part<unsigned long long>(tmp, ocount);
     unsigned *cursor = part<unsigned>(tmp, ocursor), *roff = part<unsigned>(tmp, oroff);
@@ -1320,7 +1328,7 @@ void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c,
     const size_t per_plane = record_bytes(tg);
     const JobGroups &jg = job_groups(cx, tp);
     const auto &groups = jg.first;
-    pl.rec.ensure(per_plane * jg.most);
+    if (pl.rec.bytes < per_plane * jg.most) pl.rec.ensure(record_room(per_plane * jg.most));
     const TileArgs a = tile_args(g, pl);
     const int ly = tp.ly > 0 ? tp.ly : tg.nfy, ylo = tp.ly > 0 ? tp.ylo : 0;
     for (size_t k = 0; k < groups.size(); ++k) {
