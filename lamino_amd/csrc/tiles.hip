@@ -296,12 +296,20 @@ __global__ __launch_bounds__(256) void k_run_expand(const unsigned long long *__
 }
 
 // Jobs of one tile: its points, in order, cut into equal parts of at most `most` (a row may be
-// cut too).  emit(i, beg, end, r0, r1): part i holds ids [beg, end) of slots [r0, r1).
+// cut too).  A tile that would have more than kDeep jobs, as in small volumes under many points,
+// takes sqrt(n / deep) of them, at least kDeep: a cell's sum goes over the tile's jobs one after
+// another, which then outweighs a job's own chain (`deep`: a job's time in the sum over a point's
+// in a job).  Whole adjoints in us, with jobs of `most` and so: (9, 5, 11) / 200 x 200 x 200 4219
+// and 858, (22, 22, 3) / 349 x 9 x 250 at width 10 952 and 392, first-cell slots (5, 32, 32) / 52 x
+// 203 x 120 535 and 395; with a quarter and four times `deep` the first takes 1100 and 997.
+// emit(i, beg, end, r0, r1): part i holds ids [beg, end) of slots [r0, r1).
+constexpr unsigned kDeep = 24;
 template <class F>
-__device__ __forceinline__ void tile_jobs(const unsigned *__restrict__ o, int nrho, unsigned most, F emit) {
+__device__ __forceinline__ void tile_jobs(const unsigned *__restrict__ o, int nrho, unsigned most, float deep, F emit) {
     const unsigned first = o[0], n = o[nrho] - first;
     if (n == 0) return;
-    const unsigned parts = (n + most - 1) / most;
+    unsigned parts = (n + most - 1) / most;
+    if (parts > kDeep) parts = min(parts, max(kDeep, (unsigned)sqrtf((float)n / deep)));
     const unsigned step = ((n + parts - 1) / parts + 3u) & ~3u;
     auto below = [&](unsigned v) {   // slots whose points start at or before v
         int lo = 0, hi = nrho;
@@ -364,6 +372,7 @@ struct ShareArgs {
     const unsigned *off;
     const RowY *rowy;
     unsigned jmost, umost, nunits;
+    float deep;
 };
 unsigned tile_blocks(const TileGeom &tg) { return (tg.ntiles + 63) / 64; }
 
@@ -381,7 +390,7 @@ __global__ __launch_bounds__(64) void k_share_count(ShareArgs A, TileGeom tg, un
     const unsigned t = blockIdx.x * 64u + threadIdx.x;
     if (t >= tg.ntiles) return;
     unsigned planes = 0, jobs = 0;
-    tile_jobs(A.off + (long long)t * tg.nrho, tg.nrho, A.jmost, [&](unsigned, unsigned, unsigned, int r0, int r1) {
+    tile_jobs(A.off + (long long)t * tg.nrho, tg.nrho, A.jmost, A.deep, [&](unsigned, unsigned, unsigned, int r0, int r1) {
         planes += (unsigned)(A.rowy[r1 - 1].iy + tg.W - A.rowy[r0].iy);
         ++jobs;
     });
@@ -405,7 +414,7 @@ __global__ __launch_bounds__(64) void k_share_emit(ShareArgs A, TileGeom tg, uns
     const unsigned t = blockIdx.x * 64u + threadIdx.x;
     if (t >= tg.ntiles) return;
     unsigned plane = plane0[t];
-    tile_jobs(A.off + (long long)t * tg.nrho, tg.nrho, A.jmost,
+    tile_jobs(A.off + (long long)t * tg.nrho, tg.nrho, A.jmost, A.deep,
               [&](unsigned i, unsigned beg, unsigned end, int r0, int r1) {
                   TileJob j;
                   j.tile = t;
@@ -1296,7 +1305,7 @@ TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
                        tp->ids.as<unsigned>());
     check_launch();
     // shares: counted per tile and unit, scanned, written out
-    const ShareArgs sa{off, tp->rowy, job_points(total, direct), unit_points(total), tp->nunits};
+    const ShareArgs sa{off, tp->rowy, job_points(total, direct), unit_points(total), tp->nunits, direct ? 160.f / W : 96.f};
     const unsigned tblocks = tile_blocks(tg);
     const dim3 sgrid(tblocks + tp->nunits);
     auto *jcount = part<unsigned long long>(tmp, ojcount), *ucount = part<unsigned long long>(tmp, oucount);

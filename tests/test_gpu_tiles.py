@@ -165,3 +165,20 @@ def test_plans_scanned_in_one_workgroup_and_in_several(dims, R, C, P):
     assert _rel(la.adjoint(p, pg, dims), orc.adjoint(p, dims, al, ga, eps=1e-12)) < _tol(1e-5)
     m = rng.standard_normal((3,) + dims).astype(np.float32)
     assert _rel(la.forward(m, pg), orc.forward(m, al, ga, R, C, eps=1e-12)) < _tol(1e-5)
+
+
+@pytest.mark.parametrize("dims,R,C,P,eps,varying", [((9, 5, 11), 60, 60, 150, 1e-5, False), ((3, 3, 3), 60, 61, 100, 1e-5, False),
+                                                    ((22, 22, 3), 149, 9, 150, 1e-8, False), ((5, 3, 3), 91, 31, 100, 1e-3, True),
+                                                    ((20, 14, 15), 61, 61, 120, 1e-8, True)])
+def test_tiles_with_many_jobs(dims, R, C, P, eps, varying):
+    """Small volumes under many points: tiles of more than 24 jobs, whose jobs are longer."""
+    import lamino_amd as la
+    import oracle as orc
+
+    say("deep tiles", dims, R, C, P, eps, varying)
+    rng = np.random.default_rng(24)
+    al = np.linspace(0.05, 3.0, P) if varying else np.full(P, np.radians(31.0))
+    ga = np.full(P, 0.4) if varying else 0.3 + 2 * np.pi * np.arange(P) / P
+    p = rng.standard_normal((P, R, C)).astype(np.float32)
+    a = la.adjoint(p, la.PolarGrid.per_projection(al, ga, R, C), dims, eps=eps)
+    assert _rel(a, orc.adjoint(p, dims, al, ga, eps=1e-12)) < _tol(eps)
