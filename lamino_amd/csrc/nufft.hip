@@ -18,6 +18,7 @@
 #include "fastdiv.h"
 #include "nufft.h"
 #include "nufft_point.h"
+#include "ops.h"
 #include "tiles.h"
 
 
@@ -267,26 +268,26 @@ __device__ __forceinline__ long long box_to_fine(const TileBox &b, const BinPara
 constexpr int kStage = 128;   // points staged per batch
 
 // Staged point record, in 32-bit words: [0] box cell of the point's first
-// kernel cell, [1] parity bits (lz & 1) | (ly & 1) << 1, [4, 6) the complex
-// value, then wz[W], wy[W], wx[W].  Records are 16-byte aligned.
-template <int W>
+// kernel cell, [1] parity bits (lz & 1) | (ly & 1) << 1, [4, 4 + 2 NC) the NC
+// complex values, then wz[W], wy[W], wx[W].  Records are 16-byte aligned.
+template <int W, int NC>
 struct StageLayout {
     static constexpr int VQ = 4;
-    static constexpr int WZ = VQ + 2;
+    static constexpr int WZ = VQ + 2 * NC;
     static constexpr int WY = WZ + W;
     static constexpr int WX = WY + W;
     static constexpr int SW = (WX + W + 3) / 4 * 4;
     static_assert(W % 2 == 0 && WZ % 2 == 0, "weight pairs must be 8-byte aligned");
 };
 
-template <int W>
+template <int W, bool HALF>
 __global__ __launch_bounds__(256) void k_spread_tiled(float2 *__restrict__ fine, const float2 *__restrict__ c,
                                                       const Geo *__restrict__ geo, long long P, int R, int C,
                                                       int nfz, int nfy, int nfx, float beta, PointFrame fr,
                                                       BinParams bp, const unsigned *__restrict__ ids,
-                                                      const uint4 *__restrict__ chunks) {
-    constexpr int NC = 1;   // the three-component form is the tile spreader's
-    using SL = StageLayout<W>;
+                                                      const uint4 *__restrict__ chunks, int paired) {
+    constexpr int NC = HALF ? 3 : 1;
+    using SL = StageLayout<W, NC>;
     constexpr int SW = SL::SW;
     constexpr int HW = W / 2;
     constexpr int NOWN = HW * HW * W;     // cells of one point owned by one wave
@@ -302,7 +303,7 @@ __global__ __launch_bounds__(256) void k_spread_tiled(float2 *__restrict__ fine,
     const int zpar = wave >> 1, ypar = wave & 1;
     const int HYX = bx.HY * bx.HX;
     const long long S = (long long)R * C;
-    const long long H = S;
+    const long long H = HALF ? (S + 1) / 2 : S;
 
     // this lane's cells of a point: (a, b, e) = (zoff + 2 ia, yoff + 2 ib, e)
     int loff[NCH], wzo[NCH], wyo[NCH], wxo[NCH];
@@ -362,7 +363,13 @@ __global__ __launch_bounds__(256) void k_spread_tiled(float2 *__restrict__ fine,
             const int j = (int)(idx / C), k = (int)(idx - (long long)j * C);
             const Geo g = geo[p];
             float2 vc[NC];
-            vc[0] = c[p * S + idx];
+            if constexpr (HALF) {
+                const long long mir = S - 1 - idx;
+                const float2 *pc = c + (paired ? p & ~1ll : p) * S;
+                half_point_combine(pc[idx], pc[mir], p, idx, S, g, paired, vc);
+            } else {
+                vc[0] = c[p * S + idx];
+            }
             Placed<W> pt;
             place<W>(g, fr, j, k, nfz, nfy, nfx, beta, pt);
             const int lz = wrap0(pt.iz, nfz) - bx.oz, ly = wrap0(pt.iy, nfy) - bx.oy, lx = wrap0(pt.ix, nfx) - bx.ox;
@@ -1722,6 +1729,14 @@ SpreadBytes spread_bytes(const long long dims[3], double eps, long long P, long 
     g.shared_tilt = shared;
     SpreadBytes b;
     const bool rows = use_rows(g, pl);
+    const size_t half = (size_t)(P * ((R * C + 1) / 2));
+    if (!rows && !first_cell_tiles_pay(g, pl)) {
+        size_t bins = 1;   // of at least 2 x 2 x 2 cells
+        for (int a = 0; a < 3; ++a) bins *= (size_t)(pl.nf[a] + 1) / 2;
+        b.kept = 2 * (4 * half + 16 * (half / kChunk + bins));   // ids and chunks; the tuner holds two
+        b.setup = 12 * half + 12 * bins + 4096;
+        return b;
+    }
     if (order == SpreadOrder::Tiles || !rows) {
         const TileBytes tb = tile_bytes(dims, eps, P, R, C, !rows);
         b.records = tb.records;
@@ -1729,7 +1744,7 @@ SpreadBytes spread_bytes(const long long dims[3], double eps, long long P, long 
         b.setup = tb.setup;
         return b;
     }
-    const size_t Jn = (size_t)half_rows(g), half = (size_t)(P * ((R * C + 1) / 2));
+    const size_t Jn = (size_t)half_rows(g);
     // the largest over the tilings the autotuner may choose
     for (const auto &t : kRowTileCands) {
         const RowGeom rg = row_geom(pl, t[0], t[1]);
@@ -1837,13 +1852,13 @@ void spread_rows_w(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, RowPlan &rp
     }
 }
 
-template <int W>
-void spread_w(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, const BinParams &bp, SortedPoints &sp) {
-    const size_t lds = spread_lds_bytes(bp.T, W, 1);
-    allow_lds(&k_spread_tiled<W>, lds);
-    hipLaunchKernelGGL((k_spread_tiled<W>), dim3((unsigned)sp.nchunks), dim3(256), lds, cx.stream,
+template <int W, bool HALF>
+void spread_w(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, const BinParams &bp, SortedPoints &sp, bool paired) {
+    const size_t lds = spread_lds_bytes(bp.T, W, HALF ? 3 : 1);
+    allow_lds(&k_spread_tiled<W, HALF>, lds);
+    hipLaunchKernelGGL((k_spread_tiled<W, HALF>), dim3((unsigned)sp.nchunks), dim3(256), lds, cx.stream,
                        pl.fine.as<float2>(), c, g.geo.as<Geo>(), g.P, (int)g.R, (int)g.C, pl.nf[0], pl.nf[1], pl.nf[2],
-                       pl.beta, point_frame(g, pl), bp, sp.ids.as<unsigned>(), sp.chunks.as<uint4>());
+                       pl.beta, point_frame(g, pl), bp, sp.ids.as<unsigned>(), sp.chunks.as<uint4>(), paired ? 1 : 0);
 }
 
 template <int W, bool HALF>
@@ -1873,19 +1888,26 @@ void launch_spread(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, bool half, 
         LAM_WIDTH_SWITCH(pl.w, (spread_rows_w<W>(cx, g, pl, c, rp, paired, stores)));
         return;
     }
-    if (half) {
-        TilePlan &tp = get_tileplan(cx, g, pl, !use_rows(g, pl));
+    const bool rows = half && use_rows(g, pl);
+    if (half && (rows || first_cell_tiles_pay(g, pl))) {
+        TilePlan &tp = get_tileplan(cx, g, pl, !rows);
         TimedScope ts(cx, "spread");
         tile_spread(cx, g, pl, tp, c, paired, add);
         return;
     }
-    const BinParams bp = bin_params(cx, g, pl, 1);
-    SortedPoints &sp = get_bins(cx, g, pl, false, bp);
-    if (!add)
-        LAM_HIP(hipMemsetAsync(pl.fine.ptr, 0, sizeof(float2) * (size_t)pl.nf[0] * pl.nf[1] * pl.nf[2], cx.stream));
+    const int nc = half ? 3 : 1;
+    const BinParams bp = bin_params(cx, g, pl, nc);
+    SortedPoints &sp = get_bins(cx, g, pl, half, bp);
+    const size_t cells = (size_t)pl.nf[0] * pl.nf[1] * pl.nf[2] * nc;
+    if (!add && half) fill(cx, 2 * (long long)cells, pl.fine.as<float>(), 0.f);   // a kernel: capturable
+    else if (!add) LAM_HIP(hipMemsetAsync(pl.fine.ptr, 0, sizeof(float2) * cells, cx.stream));
     if (sp.nchunks == 0) return;
     TimedScope ts(cx, "spread");
-    LAM_WIDTH_SWITCH(pl.w, (spread_w<W>(cx, g, pl, c, bp, sp)));
+    if (half) {
+        LAM_WIDTH_SWITCH(pl.w, (spread_w<W, true>(cx, g, pl, c, bp, sp, paired)));
+    } else {
+        LAM_WIDTH_SWITCH(pl.w, (spread_w<W, false>(cx, g, pl, c, bp, sp, false)));
+    }
     check_launch();
 }
 
@@ -2251,12 +2273,13 @@ void sysmat_nufft(Ctx &cx, Grid &g, const long long dims[3], double eps, const f
 // fastest in the context's table, where later calls of the same shapes find it.  Timed are the
 // kernels that read the choice.  Shared tilt: the row spreader (MBIR1's and MBIR2's
 // backprojections), and the row interpolator where the forward takes it (widths above 6), for a
-// list of 2-D tilings.  Else the interpolator of the 3-D bins, for cubic shapes and flattened
-// ones for thin or long axes that fit the LDS budget.  Results do not depend on the shape beyond
+// list of 2-D tilings.  Else the interpolator of the 3-D bins, and their spreader where no tiles
+// are, for cubic shapes and flattened ones for thin or long axes that fit the LDS budget.  Results do not depend on the shape beyond
 // FP32 summation order.
 bool spread_wants_tuning(Ctx &cx, Grid &g, const long long dims[3], double eps, SpreadOrder order) {
     NufftPlan &pl = get_nufft_plan(cx, dims, eps);
-    if (order != SpreadOrder::Rows || !use_rows(g, pl)) return false;   // the tiles read no tuned shape
+    // the tiles read no tuned shape
+    if (use_rows(g, pl) ? order != SpreadOrder::Rows : first_cell_tiles_pay(g, pl)) return false;
     std::array<int, 3> T;
     return !lookup_tuned(cx, tune_key(g, pl, 3), T);
 }
@@ -2363,11 +2386,15 @@ std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], doub
         for (const auto &T : kCands) {
             if (!bins_fit(T, pl, 3)) continue;
             cx.bin_tune[key] = {T[0], T[1], T[2]};
-            launch_interp(cx, g, pl, cbuf, true);   // builds this shape's bins
+            const auto both = [&] {   // the spreader where it reads the bins too
+                if (!first_cell_tiles_pay(g, pl)) launch_spread(cx, g, pl, cbuf, true);
+                launch_interp(cx, g, pl, cbuf, true);
+            };
+            both();   // builds this shape's bins
             float t = 0.f;
             for (int rep = 0; rep < 2; ++rep) {
                 LAM_HIP(hipEventRecord(e0, cx.stream));
-                launch_interp(cx, g, pl, cbuf, true);
+                both();
                 LAM_HIP(hipEventRecord(e1, cx.stream));
                 LAM_HIP(hipEventSynchronize(e1));
                 float ms = 0.f;

@@ -72,6 +72,9 @@ struct TilePlan {
 // The y planes [ylo, ylo + ly) (mod nfy) that the rows of a shared-tilt grid touch (ly 0: all).
 void row_window(const Grid &g, const NufftPlan &pl, int &ylo, int &ly);
 
+// Whether the spread of a grid without row slots goes by tiles (first-cell slots) or by 3-D bins.
+bool first_cell_tiles_pay(const Grid &g, const NufftPlan &pl);
+
 TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct);
 
 // fine (+)= the type-1 spread of the half point set.  add = false writes every plane of the

@@ -296,20 +296,23 @@ __global__ __launch_bounds__(256) void k_run_expand(const unsigned long long *__
 }
 
 // Jobs of one tile: its points, in order, cut into equal parts of at most `most` (a row may be
-// cut too).  A tile that would have more than kDeep jobs, as in small volumes under many points,
-// takes sqrt(n / deep) of them, at least kDeep: a cell's sum goes over the tile's jobs one after
+// cut too).  A tile that would have more than `many` jobs, as in small volumes under many points,
+// takes sqrt(n / deep) of them, at least `many`: a cell's sum goes over the tile's jobs one after
 // another, which then outweighs a job's own chain (`deep`: a job's time in the sum over a point's
 // in a job).  Whole adjoints in us, with jobs of `most` and so: (9, 5, 11) / 200 x 200 x 200 4219
 // and 858, (22, 22, 3) / 349 x 9 x 250 at width 10 952 and 392, first-cell slots (5, 32, 32) / 52 x
-// 203 x 120 535 and 395; with a quarter and four times `deep` the first takes 1100 and 997.
+// 203 x 120 535 and 395; with a quarter and four times `deep` the first takes 1100 and 997.  With
+// 24, 12, 8 and 6 for `many` first-cell slots take 0.870, 0.854, 0.848 and 0.847 of the 3-D bins'
+// time over 90 small grids.
 // emit(i, beg, end, r0, r1): part i holds ids [beg, end) of slots [r0, r1).
-constexpr unsigned kDeep = 24;
+constexpr unsigned kDeep = 24, kDeepDirect = 8;
 template <class F>
-__device__ __forceinline__ void tile_jobs(const unsigned *__restrict__ o, int nrho, unsigned most, float deep, F emit) {
+__device__ __forceinline__ void tile_jobs(const unsigned *__restrict__ o, int nrho, unsigned most, unsigned many,
+                                          float deep, F emit) {
     const unsigned first = o[0], n = o[nrho] - first;
     if (n == 0) return;
     unsigned parts = (n + most - 1) / most;
-    if (parts > kDeep) parts = min(parts, max(kDeep, (unsigned)sqrtf((float)n / deep)));
+    if (parts > many) parts = max(many, min(parts, (unsigned)sqrtf((float)n / deep)));
     const unsigned step = ((n + parts - 1) / parts + 3u) & ~3u;
     auto below = [&](unsigned v) {   // slots whose points start at or before v
         int lo = 0, hi = nrho;
@@ -371,7 +374,7 @@ __device__ __forceinline__ void unit_jobs(const unsigned *__restrict__ off, unsi
 struct ShareArgs {
     const unsigned *off;
     const RowY *rowy;
-    unsigned jmost, umost, nunits;
+    unsigned jmost, umost, nunits, many;
     float deep;
 };
 unsigned tile_blocks(const TileGeom &tg) { return (tg.ntiles + 63) / 64; }
@@ -390,7 +393,7 @@ __global__ __launch_bounds__(64) void k_share_count(ShareArgs A, TileGeom tg, un
     const unsigned t = blockIdx.x * 64u + threadIdx.x;
     if (t >= tg.ntiles) return;
     unsigned planes = 0, jobs = 0;
-    tile_jobs(A.off + (long long)t * tg.nrho, tg.nrho, A.jmost, A.deep, [&](unsigned, unsigned, unsigned, int r0, int r1) {
+    tile_jobs(A.off + (long long)t * tg.nrho, tg.nrho, A.jmost, A.many, A.deep, [&](unsigned, unsigned, unsigned, int r0, int r1) {
         planes += (unsigned)(A.rowy[r1 - 1].iy + tg.W - A.rowy[r0].iy);
         ++jobs;
     });
@@ -414,7 +417,7 @@ __global__ __launch_bounds__(64) void k_share_emit(ShareArgs A, TileGeom tg, uns
     const unsigned t = blockIdx.x * 64u + threadIdx.x;
     if (t >= tg.ntiles) return;
     unsigned plane = plane0[t];
-    tile_jobs(A.off + (long long)t * tg.nrho, tg.nrho, A.jmost, A.deep,
+    tile_jobs(A.off + (long long)t * tg.nrho, tg.nrho, A.jmost, A.many, A.deep,
               [&](unsigned i, unsigned beg, unsigned end, int r0, int r1) {
                   TileJob j;
                   j.tile = t;
@@ -1168,6 +1171,20 @@ void row_window(const Grid &g, const NufftPlan &pl, int &ylo, int &ly) {
     }
 }
 
+// The 3-D bins' spreader, which the forward of such grids shares its plan with, is the better one
+// where the tiles' fixed costs show (fewer than 2048 points; a whole adjoint at 98 to 1976 points
+// takes 52 to 113 us with it and 0.76 to 1.61 of that by tiles, 1.13 at the median), and where all
+// points crowd into a few tiles: (4, 4, 4) / 236 x 31 x 44 299 us against 422, (15, 7, 3) / 209 x
+// 352 x 68 at width 10 1451 against 3173; above width 8 the line lies at fewer points, since three
+// waves then stage each ((4, 4, 4) / 281 x 27 x 2 at width 10 104 and 195).  Elsewhere the tiles
+// are: (60, 15, 60) / 200 x 200 x 200 1141 and 850, (11, 3, 11) / 80 x 28 x 21 at width 8 213 and 173.
+bool first_cell_tiles_pay(const Grid &g, const NufftPlan &pl) {
+    const TileGeom tg = tile_geom(pl.nf, pl.w, g.R, g.C, true);
+    const long long total = g.P * ((g.R * g.C + 1) / 2);
+    const bool crowded = (tg.ntiles < 24 && total > 32768ll * tg.ntiles) || (tile_comps(pl.w) == 1 && tg.ntiles < 6);
+    return total >= 2048 && !crowded;
+}
+
 TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long R, long long C, bool direct) {
     NufftPlan pl;   // shapes only
     pl.w = width_for_eps(eps);
@@ -1305,7 +1322,8 @@ TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
                        tp->ids.as<unsigned>());
     check_launch();
     // shares: counted per tile and unit, scanned, written out
-    const ShareArgs sa{off, tp->rowy, job_points(total, direct), unit_points(total), tp->nunits, direct ? 160.f / W : 96.f};
+    const ShareArgs sa{off, tp->rowy, job_points(total, direct), unit_points(total), tp->nunits, direct ? kDeepDirect : kDeep,
+                       direct ? 160.f / W : 96.f};
     const unsigned tblocks = tile_blocks(tg);
     const dim3 sgrid(tblocks + tp->nunits);
     auto *jcount = part<unsigned long long>(tmp, ojcount), *ucount = part<unsigned long long>(tmp, oucount);

@@ -182,3 +182,32 @@ def test_tiles_with_many_jobs(dims, R, C, P, eps, varying):
     p = rng.standard_normal((P, R, C)).astype(np.float32)
     a = la.adjoint(p, la.PolarGrid.per_projection(al, ga, R, C), dims, eps=eps)
     assert _rel(a, orc.adjoint(p, dims, al, ga, eps=1e-12)) < _tol(eps)
+
+
+@pytest.mark.parametrize("dims,R,C,P,eps,tiles", [((9, 5, 11), 13, 15, 20, 1e-5, False), ((9, 5, 11), 13, 15, 21, 1e-5, True),
+                                                  ((4, 4, 4), 61, 61, 40, 1e-3, False), ((4, 4, 4), 61, 61, 30, 1e-3, True),
+                                                  ((4, 4, 4), 41, 31, 20, 1e-8, False), ((6, 5, 7), 41, 31, 20, 1e-10, True),
+                                                  ((31, 9, 31), 45, 45, 60, 1e-6, True)])
+def test_first_cell_grids_on_both_sides_of_the_line(ctx, dims, R, C, P, eps, tiles):
+    """Grids of varying tilt: fewer than 2048 points, points crowded into a few tiles and wide
+    kernels over fewer than six tiles go by 3-D bins; both against the oracle."""
+    import ctypes
+
+    import lamino_amd as la
+    import oracle as orc
+    from lamino_amd._lib import check
+
+    say("first-cell line", dims, R, C, P, eps, tiles)
+    rng = np.random.default_rng(25)
+    al, ga = np.linspace(0.05, 3.0, P), np.full(P, 0.4)
+    pg = la.PolarGrid.per_projection(al, ga, R, C)
+    p = rng.standard_normal((P, R, C)).astype(np.float32)
+    check(ctx.lib.lam_timing_enable(ctx.h, 1))
+    a = la.adjoint(p, pg, dims, eps=eps)
+    ms, n = ctypes.c_double(), ctypes.c_int64()
+    check(ctx.lib.lam_timing_query(ctx.h, b"tile_spread", ctypes.byref(ms), ctypes.byref(n)))
+    check(ctx.lib.lam_timing_enable(ctx.h, 0))
+    assert (n.value > 0) == tiles
+    assert _rel(a, orc.adjoint(p, dims, al, ga, eps=1e-12)) < _tol(eps)
+    acc = la.adjoint_multi([p, p], [pg, pg], dims, eps=eps)
+    assert _rel(acc, 2 * a) < 1e-5   # the second grid adds into the first one's fine grid
