@@ -211,3 +211,22 @@ def test_first_cell_grids_on_both_sides_of_the_line(ctx, dims, R, C, P, eps, til
     assert _rel(a, orc.adjoint(p, dims, al, ga, eps=1e-12)) < _tol(eps)
     acc = la.adjoint_multi([p, p], [pg, pg], dims, eps=eps)
     assert _rel(acc, 2 * a) < 1e-5   # the second grid adds into the first one's fine grid
+
+
+@pytest.mark.parametrize("varying", [False, True])
+@pytest.mark.parametrize("P", [255, 256, 257, 700, 2500])
+def test_buckets_of_many_runs_keep_the_points_order(P, varying):
+    """Up to 256 runs of a bucket are ranked by a wave, more by a workgroup.  The order of a bucket's
+    points is theirs, so two plans give the same bits, and the sums are the oracle's."""
+    import lamino_amd as la
+    import oracle as orc
+
+    dims, R, C = (9, 5, 11), 11, 13
+    say("many runs", P, varying)
+    rng = np.random.default_rng(26)
+    al = np.linspace(0.05, 3.0, P) if varying else np.full(P, np.radians(31.0))
+    ga = np.full(P, 0.4) if varying else 0.3 + 2 * np.pi * np.arange(P) / P
+    p = rng.standard_normal((P, R, C)).astype(np.float32)
+    one, two = (la.adjoint(p, la.PolarGrid.per_projection(al, ga, R, C), dims) for _ in range(2))
+    assert np.array_equal(one, two)
+    assert _rel(one, orc.adjoint(p, dims, al, ga, eps=1e-12)) < _tol(1e-5)
