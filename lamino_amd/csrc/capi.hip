@@ -270,13 +270,15 @@ size_t mbir_footprint(const lam_dataset *ds, int nds, const long long rd[3], con
         raw = std::max(raw, 4 * P * (size_t)D.nrows * (size_t)D.ncols);
         padded = std::max(padded, 4 * M);
         spectra = std::max(spectra, 8 * M);
-        // the spreader that the job takes: by its method and whether the dataset shares the
-        // tilt (no angles given: either)
-        const bool shared = !D.alpha || std::all_of(D.alpha, D.alpha + P, [&](double a) { return a == D.alpha[0]; });
+        // the spreader that the job takes: by its method and the dataset's tilt (no angles given:
+        // any of a flat, a steep and a varying one's)
+        const double flat = 0.0, steep = 1.5707963267948966;
+        const bool shared = D.alpha && std::all_of(D.alpha, D.alpha + P, [&](double a) { return a == D.alpha[0]; });
+        std::vector<const double *> tilts = {shared ? D.alpha : nullptr};
+        if (!D.alpha) tilts = {&flat, &steep, nullptr};
         size_t kept = 0;
-        for (const bool s : {true, false}) {
-            if (D.alpha && s != shared) continue;
-            const SpreadBytes sb = spread_bytes(od, eps, (long long)P, (long long)R2, (long long)C2, s,
+        for (const double *t : tilts) {
+            const SpreadBytes sb = spread_bytes(od, eps, (long long)P, (long long)R2, (long long)C2, t,
                                                 pr.method == 3 ? SpreadOrder::Tiles : SpreadOrder::Rows);
             slab = std::max(slab, sb.slab);
             records = std::max(records, sb.records);

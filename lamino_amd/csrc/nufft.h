@@ -139,12 +139,12 @@ bool spread_wants_tuning(Ctx &cx, Grid &g, const long long dims[3], double eps, 
 // Upper bounds of the device bytes of one backprojection of a grid of P projections of R x C on
 // the fine grid of dims: slab and records: the row spreader's slabs and halos, the tile
 // spreader's plane records (buffers of the plan, shared by grids of the same dims); kept: the
-// grid's point bins; setup: temporaries while they are built.  shared: the projections share
-// the tilt.
+// grid's point bins; setup: temporaries while they are built.  tilt: of all projections (null:
+// it varies).
 struct SpreadBytes {
     size_t slab = 0, records = 0, kept = 0, setup = 0;
 };
-SpreadBytes spread_bytes(const long long dims[3], double eps, long long P, long long R, long long C, bool shared,
+SpreadBytes spread_bytes(const long long dims[3], double eps, long long P, long long R, long long C, const double *tilt,
                          SpreadOrder order);
 
 }  // namespace lam

@@ -1717,7 +1717,7 @@ int rows_per_group(const RowPlan &rp, const NufftPlan &pl) {
 
 }  // namespace
 
-SpreadBytes spread_bytes(const long long dims[3], double eps, long long P, long long R, long long C, bool shared,
+SpreadBytes spread_bytes(const long long dims[3], double eps, long long P, long long R, long long C, const double *tilt,
                          SpreadOrder order) {
     NufftPlan pl;   // shapes only
     pl.w = width_for_eps(eps);
@@ -1726,7 +1726,9 @@ SpreadBytes spread_bytes(const long long dims[3], double eps, long long P, long 
     g.P = P;
     g.R = R;
     g.C = C;
-    g.shared_tilt = shared;
+    g.shared_tilt = tilt != nullptr;
+    g.geo_host.resize(1);
+    g.geo_host[0].vy = tilt ? -std::sin(*tilt) : 0.0;
     SpreadBytes b;
     const bool rows = use_rows(g, pl);
     const size_t half = (size_t)(P * ((R * C + 1) / 2));
@@ -1737,8 +1739,8 @@ SpreadBytes spread_bytes(const long long dims[3], double eps, long long P, long 
         b.setup = 12 * half + 12 * bins + 4096;
         return b;
     }
-    if (order == SpreadOrder::Tiles || !rows) {
-        const TileBytes tb = tile_bytes(dims, eps, P, R, C, !rows);
+    if (!rows || (order == SpreadOrder::Tiles && row_tiles_pay(g, pl))) {
+        const TileBytes tb = tile_bytes(pl, P, R, C, !rows);
         b.records = tb.records;
         b.kept = tb.kept;
         b.setup = tb.setup;
@@ -1876,7 +1878,8 @@ void interp_w(Ctx &cx, Grid &g, NufftPlan &pl, float2 *c, const BinParams &bp, S
 // order: which of the three-component spreaders (see SpreadOrder)
 void launch_spread(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, bool half, bool paired = false,
                    bool add = false, SpreadOrder order = SpreadOrder::Tiles) {
-    if (half && (order == SpreadOrder::Rows || rows_spread_asked()) && use_rows(g, pl)) {
+    const bool rows = half && use_rows(g, pl);
+    if (rows && (order == SpreadOrder::Rows || rows_spread_asked() || !row_tiles_pay(g, pl))) {
         RowPlan &rp = get_rowplan(cx, g, pl);
         // One row group whose y window does not wrap writes every plane of the window
         // once, and the transforms that follow read only the window: no zeroing.
@@ -1888,7 +1891,6 @@ void launch_spread(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, bool half, 
         LAM_WIDTH_SWITCH(pl.w, (spread_rows_w<W>(cx, g, pl, c, rp, paired, stores)));
         return;
     }
-    const bool rows = half && use_rows(g, pl);
     if (half && (rows || first_cell_tiles_pay(g, pl))) {
         TilePlan &tp = get_tileplan(cx, g, pl, !rows);
         TimedScope ts(cx, "spread");
@@ -2279,7 +2281,7 @@ void sysmat_nufft(Ctx &cx, Grid &g, const long long dims[3], double eps, const f
 bool spread_wants_tuning(Ctx &cx, Grid &g, const long long dims[3], double eps, SpreadOrder order) {
     NufftPlan &pl = get_nufft_plan(cx, dims, eps);
     // the tiles read no tuned shape
-    if (use_rows(g, pl) ? order != SpreadOrder::Rows : first_cell_tiles_pay(g, pl)) return false;
+    if (use_rows(g, pl) ? order != SpreadOrder::Rows && row_tiles_pay(g, pl) : first_cell_tiles_pay(g, pl)) return false;
     std::array<int, 3> T;
     return !lookup_tuned(cx, tune_key(g, pl, 3), T);
 }
@@ -2290,7 +2292,7 @@ std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], doub
         // Time each distinct 2-D tiling the candidate edges give (each with its own point
         // bins) and record the fastest as (Tz, W, Tx) in the row table; the 3-D table gets
         // the default 3-D tile so that the grid counts as tuned.  The fastest's bins, the
-        // slabs and the halos stay only where the forward uses them.
+        // slabs and the halos stay only where the grid's projectors use them.
         const bool interp_rows = !tile_interp_fits(pl.w);
         const bool had_slab = pl.slab.bytes > 0, had_halo = pl.halo.bytes > 0;
         ensure_fine(pl, 3);
@@ -2350,11 +2352,10 @@ std::array<int, 3> autotune_bins(Ctx &cx, Grid &g, const long long dims[3], doub
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
         LAM_REQUIRE(best[0] != 0, LAM_ERR_STATE, "no row tiling fits this grid");
-        if (!interp_rows) {
-            g.rowplans.erase(plan_key(best[0], best[2]));
-            if (!had_slab) pl.slab.release();
-        }
-        if (!had_halo) pl.halo.release();
+        const bool spread_rows = !row_tiles_pay(g, pl);
+        if (!interp_rows && !spread_rows) g.rowplans.erase(plan_key(best[0], best[2]));
+        if (!interp_rows && !spread_rows && !had_slab) pl.slab.release();
+        if (!spread_rows && !had_halo) pl.halo.release();
         const BinParams bp = bin_params(cx, g, pl, 3);
         const std::array<int, 3> T3 = {bp.T[0], bp.T[1], bp.T[2]};
         cx.bin_tune[rkey] = best;

@@ -72,6 +72,9 @@ struct TilePlan {
 // The y planes [ylo, ylo + ly) (mod nfy) that the rows of a shared-tilt grid touch (ly 0: all).
 void row_window(const Grid &g, const NufftPlan &pl, int &ylo, int &ly);
 
+// Whether the spread of a shared-tilt grid goes by tiles (row slots) or by the row form.
+bool row_tiles_pay(const Grid &g, const NufftPlan &pl);
+
 // Whether the spread of a grid without row slots goes by tiles (first-cell slots) or by 3-D bins.
 bool first_cell_tiles_pay(const Grid &g, const NufftPlan &pl);
 
@@ -91,6 +94,6 @@ void tile_interp(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, float2 *c);
 struct TileBytes {
     size_t kept = 0, setup = 0, records = 0;
 };
-TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long R, long long C, bool direct);
+TileBytes tile_bytes(const NufftPlan &pl, long long P, long long R, long long C, bool direct);   // pl: w and nf
 
 }  // namespace lam

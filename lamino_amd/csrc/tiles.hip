@@ -1167,12 +1167,11 @@ size_t record_budget() {
     return (size_t)8 << 30;
 }
 
-// Room made for `need` bytes of records: up to an eighth more, within the budget, so that the next
-// grid of the shape, whose jobs record a little more or less, finds it large enough.
-size_t record_room(size_t need) {
-    size_t step = 1 << 16;
-    while (16 * step <= need) step *= 2;
-    return std::max(need, std::min((need + step - 1) / step * step, record_budget()));
+// Room made for `need` bytes of records, of at most `bound`: more than asked for, so that the next
+// grid of the shape, whose jobs record more or less, finds it large enough.  Twice the need while
+// that is small (the records of a few projections vary with their angles), else an eighth more.
+size_t record_room(size_t need, size_t bound) {
+    return std::max(need, std::min(bound, need <= ((size_t)128 << 20) ? 2 * need : need + need / 8));
 }
 
 TileArgs tile_args(const Grid &g, const NufftPlan &pl) {
@@ -1237,24 +1236,39 @@ void row_window(const Grid &g, const NufftPlan &pl, int &ylo, int &ly) {
     }
 }
 
+// A tile records the planes between its first row and its last, 4 KB each however few points are
+// on them, where the row form moves a slab per row; the tiles are cheaper per point (about 40 ps
+// against 67).  Where the rows are few against the planes they span, or the points few on both,
+// the records outweigh that: whole adjoints by tiles and by rows took 359 and 203 us at (33, 166,
+// 166) / 79 x 16 x 67, width 8; 640 and 440 at (130, 130, 130) / 34 x 167 x 68; 149 and 203 at
+// (89, 21, 89) / 89 x 89 x 90, whose records exceed the slabs by 30 bytes a point.  Of 250 laminography
+// scans (tilts of 25 to 40 degrees, thin volumes of 40 to 260) the line at 160 bytes a point and 60 MB
+// sends 4 by rows, all at width 8 and none of them faster by tiles, and leaves 2 by tiles that rows
+// would take 3 to 6 % less for.  Over 1000 arbitrary grids it halves those that tiles are more than a
+// tenth slower for, from 137; most of the rest are volumes of a few cells.
+bool row_tiles_pay(const Grid &g, const NufftPlan &pl) {
+    const TileGeom tg = tile_geom(pl.nf, pl.w, g.R, g.C, false);
+    const double span = std::min<double>(tg.nfy, std::floor(tg.Jn * std::fabs(g.geo_host[0].vy) * tg.nfy / (double)g.R) + pl.w);
+    const double tiles = (double)tg.ntiles * span * (double)record_bytes(tg);
+    const double slabs = (double)tg.Jn * tg.nfz * tg.nfx * 3 * sizeof(float2);
+    return tiles - slabs <= 160.0 * (double)(g.P * ((g.R * g.C + 1) / 2)) + 6e7;
+}
+
 // The 3-D bins' spreader, which the forward of such grids shares its plan with, is the better one
 // where the tiles' fixed costs show (fewer than 2048 points; a whole adjoint at 98 to 1976 points
 // takes 52 to 113 us with it and 0.76 to 1.61 of that by tiles, 1.13 at the median), and where all
 // points crowd into a few tiles: (4, 4, 4) / 236 x 31 x 44 299 us against 422, (15, 7, 3) / 209 x
-// 352 x 68 at width 10 1451 against 3173; above width 8 the line lies at fewer points, since three
+// 352 x 68 at width 10 1451 against 3173, (14, 14, 14) / 207 x 297 x 58 at width 8 775 and 1158; above width 8 the line lies at fewer points, since three
 // waves then stage each ((4, 4, 4) / 281 x 27 x 2 at width 10 104 and 195).  Elsewhere the tiles
 // are: (60, 15, 60) / 200 x 200 x 200 1141 and 850, (11, 3, 11) / 80 x 28 x 21 at width 8 213 and 173.
 bool first_cell_tiles_pay(const Grid &g, const NufftPlan &pl) {
     const TileGeom tg = tile_geom(pl.nf, pl.w, g.R, g.C, true);
     const long long total = g.P * ((g.R * g.C + 1) / 2);
-    const bool crowded = (tg.ntiles < 24 && total > 32768ll * tg.ntiles) || (tile_comps(pl.w) == 1 && tg.ntiles < 6);
+    const bool crowded = (tg.ntiles < 64 && total > 32768ll * tg.ntiles) || (tile_comps(pl.w) == 1 && tg.ntiles < 6);
     return total >= 2048 && !crowded;
 }
 
-TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long R, long long C, bool direct) {
-    NufftPlan pl;   // shapes only
-    pl.w = width_for_eps(eps);
-    for (int a = 0; a < 3; ++a) pl.nf[a] = (int)nufft_fine_len(dims[a], eps);
+TileBytes tile_bytes(const NufftPlan &pl, long long P, long long R, long long C, bool direct) {
     const size_t total = (size_t)P * (size_t)((R * C + 1) / 2);
     const TileGeom tg = tile_geom(pl.nf, pl.w, R, C, direct);
     const size_t nb = (size_t)tg.ntiles * tg.nrho, ids = total + 3 * std::min(nb, total);
@@ -1270,8 +1284,8 @@ TileBytes tile_bytes(const long long dims[3], double eps, long long P, long long
              sizeof(TileGeo) * (size_t)P + sizeof(RowY) * tg.nrho + 64 * (size_t)(tg.nfz + tg.nfx) + 4096;
     b.setup = 17 * total + 4096;   // the runs, twice, and the list of long buckets
     // counts, run offsets and cursors per bucket and scan sums, in the record buffer
-    b.records = record_room(std::max(17 * nb + 64 * (size_t)tg.ntiles + 65536,
-                                     std::min(record_bytes(tg) * planes, std::max(record_budget(), largest))));
+    b.records = std::max(17 * nb + 64 * (size_t)tg.ntiles + 65536,
+                         std::min(record_bytes(tg) * planes, std::max(record_budget(), largest)));
     return b;
 }
 
@@ -1357,7 +1371,8 @@ TilePlan &get_tileplan(Ctx &cx, Grid &g, NufftPlan &pl, bool direct) {
                  oucount = cs.take(sizeof(unsigned long long) * tp->nunits),
                  oujob0 = cs.take(sizeof(unsigned) * (tp->nunits + 1ull)),
                  ouhigh = cs.take(sizeof(unsigned) * (tp->nunits + 1ull));
-    if (pl.rec.bytes < cs.bytes) pl.rec.ensure(record_room(cs.bytes));
+    if (pl.rec.bytes < cs.bytes)
+        pl.rec.ensure(record_room(cs.bytes, tile_bytes(pl, g.P, g.R, g.C, direct).records));
     const DevBuf &tmp = pl.rec;
     auto *count = part<unsigned long long>(tmp, ocount);
     unsigned *cursor = part<unsigned>(tmp, ocursor), *roff = part<unsigned>(tmp, oroff);
@@ -1433,7 +1448,8 @@ void tile_spread(Ctx &cx, Grid &g, NufftPlan &pl, TilePlan &tp, const float2 *c,
     const size_t per_plane = record_bytes(tg);
     const JobGroups &jg = job_groups(cx, tp);
     const auto &groups = jg.first;
-    if (pl.rec.bytes < per_plane * jg.most) pl.rec.ensure(record_room(per_plane * jg.most));
+    if (pl.rec.bytes < per_plane * jg.most)
+        pl.rec.ensure(record_room(per_plane * jg.most, tile_bytes(pl, g.P, g.R, g.C, tg.direct != 0).records));
     const TileArgs a = tile_args(g, pl);
     const int ly = tp.ly > 0 ? tp.ly : tg.nfy, ylo = tp.ly > 0 ? tp.ylo : 0;
     for (size_t k = 0; k < groups.size(); ++k) {

@@ -100,3 +100,22 @@ def test_tuned_row_tiling_keeps_parity(ctx, orc, monkeypatch, eps):
     assert ms > 0 and T[0] >= 2 and T[2] >= 2
     assert rel(a1, a0) < 1e-5 and rel(y1, y0) < 1e-5
     assert rel(a1, orc.adjoint(p, dims, al, ga, eps=1e-12)) < 1e-4
+
+
+@pytest.mark.parametrize("dims,R,C,P,eps,tilt,tiles", [((60, 60, 60), 17, 40, 20, 1e-5, 60.0, False), ((60, 60, 60), 17, 40, 20, 1e-5, 0.0, True),
+                                                       ((31, 31, 31), 17, 40, 20, 1e-5, 60.0, True), ((48, 40, 60), 41, 43, 2, 1e-6, 90.0, False),
+                                                       ((48, 40, 60), 41, 43, 2, 1e-8, 35.0, True), ((48, 12, 60), 41, 43, 60, 1e-6, 35.0, True)])
+def test_adjoints_on_both_sides_of_the_line(ctx, orc, dims, R, C, P, eps, tilt, tiles):
+    """Few rows against the planes they span go by rows, the others by tiles; one grid adds into
+    what the other left."""
+    import lamino_amd as la
+
+    rng = np.random.default_rng(125)
+    al, ga = np.full(P, np.radians(tilt)), 0.4 + 2 * np.pi * np.arange(P) / P
+    pg = la.PolarGrid.per_projection(al, ga, R, C)
+    p = rng.standard_normal((P, R, C)).astype(np.float32)
+    a, ran = _ran(ctx, lambda: la.adjoint(p, pg, dims, eps=eps), ["spread_rows2d", "tile_spread"])
+    assert (ran["tile_spread"] > 0) == tiles and (ran["spread_rows2d"] > 0) == (not tiles), ran
+    w = {v: k for k, v in EPS.items()}[eps]
+    assert rel(a, orc.adjoint(p, dims, al, ga, eps=1e-12)) < _tol(w)
+    assert rel(la.adjoint_multi([p, p], [pg, pg], dims, eps=eps), 2 * a) < 1e-5

@@ -223,15 +223,15 @@ def test_graph_jobs_tune_only_what_they_read(ctx, monkeypatch, capfd, method, de
 
 
 def test_tuning_leaves_no_row_slabs_where_nothing_reads_them(ctx):
-    """At width 6 neither projector takes the row path, so the tuner's point bins and slabs (here
-    77 MB) go when it is done."""
+    """At width 6 neither projector of a grid of many points takes the row path, so the tuner's point
+    bins and slabs (here 77 MB) go when it is done."""
     import ctypes
 
     import lamino_amd as la
 
     hip = ctx.lib
     free0, free1, total = ctypes.c_size_t(), ctypes.c_size_t(), ctypes.c_size_t()
-    dims, R, C, P = (127, 31, 127), 51, 53, 8
+    dims, R, C, P = (127, 31, 127), 51, 53, 400
     pg = la.PolarGrid.per_projection(np.full(P, np.radians(30.0)), 2 * np.pi * np.arange(P) / P, R, C)
     la.adjoint(np.ones((P, R, C), np.float32), pg, dims)
     la.forward(np.ones((3,) + dims, np.float32), pg)
