@@ -113,7 +113,8 @@ std::unique_ptr<Grid> make_grid(Ctx &cx, const double *alpha, const double *gamm
 // against: conjugate gradients on the normal operator multiply a change in the last bits of
 // yT about a hundredfold (measured over 60 jobs: 2e-7 in yT becomes up to 5e-5 of MBIR1's
 // result and 1.4e-5 of MBIR2's, 2e-7 of MBIR3's), so a job's result stays what it was.
-// Grids whose tilt varies have no row form and take the tiles.
+// Grids whose tilt varies have no row form.  Tiles leaves the choice to row_tiles_pay and
+// first_cell_tiles_pay (tiles.h).
 enum class SpreadOrder { Tiles, Rows };
 
 // Projectors and NUFFT entry points (device pointers, context stream)

@@ -17,10 +17,11 @@
 // (89, 21, 89) / 89 x 89 x 90: 0.112 -> 0.070 ms; grids whose tilt varies, (127, 31, 127) /
 // 181 x 181 x 120: 1.55 -> 0.50 ms.  fp32 matrix instructions and vector instructions share
 // the SIMD on gfx950 (measured: a wave of each side by side takes the sum of their times;
-// a bf16 one overlaps), so what bounds the kernel is their sum: 2.29e9 + 2.99e9 SIMD cycles
-// of the 7.0e9 of a launch at the largest shape.  Hence the 32 x 32 block of all components:
+// a bf16 one overlaps), so what bounds the kernel is their sum: 2.29e9 + 3.24e9 SIMD cycles
+// of the 6.63e9 of a launch at the largest shape.  Hence the 32 x 32 block of all components:
 // with one wave per component and 16 x 16 blocks the matrix part is half as much again, and
-// the launch took 3.65 ms against 2.9 ms.
+// the launch took 3.65 ms against 2.9 ms.  Where other forms are the better ones: row_tiles_pay and
+// first_cell_tiles_pay below.
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
