@@ -1873,6 +1873,12 @@ void interp_w(Ctx &cx, Grid &g, NufftPlan &pl, float2 *c, const BinParams &bp, S
                        pl.beta, point_frame(g, pl), bp, sp.ids.as<unsigned>(), sp.chunks.as<uint4>());
 }
 
+// The three components' fine grid to zero, by a kernel: an adjoint may be captured in a graph, and
+// replays of memset nodes have given wrong results.
+void clear_fine(Ctx &cx, NufftPlan &pl) {
+    fill(cx, 6ll * pl.nf[0] * pl.nf[1] * pl.nf[2], pl.fine.as<float>(), 0.f);
+}
+
 // paired: c holds detector-pair spectra (det_fft2_real_pairs), three-component form only
 // add: accumulate into the fine grid's current contents (no zero fill, no stores)
 // order: which of the three-component spreaders (see SpreadOrder)
@@ -1885,8 +1891,7 @@ void launch_spread(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, bool half, 
         // once, and the transforms that follow read only the window: no zeroing.
         const bool stores = !add && rows_per_group(rp, pl) >= rp.Jn && rp.ly > 0;
         if (!stores && !add)
-            LAM_HIP(hipMemsetAsync(pl.fine.ptr, 0, sizeof(float2) * (size_t)pl.nf[0] * pl.nf[1] * pl.nf[2] * 3,
-                                   cx.stream));
+            clear_fine(cx, pl);
         TimedScope ts(cx, "spread");
         LAM_WIDTH_SWITCH(pl.w, (spread_rows_w<W>(cx, g, pl, c, rp, paired, stores)));
         return;
@@ -1900,9 +1905,9 @@ void launch_spread(Ctx &cx, Grid &g, NufftPlan &pl, const float2 *c, bool half, 
     const int nc = half ? 3 : 1;
     const BinParams bp = bin_params(cx, g, pl, nc);
     SortedPoints &sp = get_bins(cx, g, pl, half, bp);
-    const size_t cells = (size_t)pl.nf[0] * pl.nf[1] * pl.nf[2] * nc;
-    if (!add && half) fill(cx, 2 * (long long)cells, pl.fine.as<float>(), 0.f);   // a kernel: capturable
-    else if (!add) LAM_HIP(hipMemsetAsync(pl.fine.ptr, 0, sizeof(float2) * cells, cx.stream));
+    if (!add && half) clear_fine(cx, pl);
+    else if (!add)
+        LAM_HIP(hipMemsetAsync(pl.fine.ptr, 0, sizeof(float2) * (size_t)pl.nf[0] * pl.nf[1] * pl.nf[2], cx.stream));
     if (sp.nchunks == 0) return;
     TimedScope ts(cx, "spread");
     if (half) {
@@ -2236,8 +2241,7 @@ void adjoint_multi(Ctx &cx, Grid *const *grids, int ngrids, const long long dims
     // union is not what the first grid writes, so the whole fine grid starts at zero
     bool add = false;
     if (ngrids > 1 && yw.len == 0) {
-        LAM_HIP(hipMemsetAsync(pl.fine.ptr, 0, sizeof(float2) * (size_t)pl.nf[0] * pl.nf[1] * pl.nf[2] * 3,
-                               cx.stream));
+        clear_fine(cx, pl);
         add = true;
     }
     const float scale = 1.0f / (float)(grids[0]->R * grids[0]->C);

@@ -93,11 +93,11 @@ def test_more_detector_lines_than_one_launch_has_waves():
     assert _rel(back(0, P), back(0, P // 2) + back(P // 2, P)) < 4 * 5450**0.5 * 2**-24
 
 
-@pytest.mark.parametrize("planes", [1, 40, 300])
-def test_adjoint_over_the_record_budget_can_be_captured(monkeypatch, planes):
-    """Once its plan is there, an adjoint whose records exceed the budget (groups of one job, and
-    of several) only launches kernels: it can be captured, and each replay gives the eager call's
-    bits for the input of the moment."""
+@pytest.mark.parametrize("planes,rows", [(1, "1"), (40, "1"), (300, "1"), (40, "spread"), (300, "spread")])
+def test_adjoint_over_the_record_budget_can_be_captured(monkeypatch, planes, rows):
+    """Once its plan is there, an adjoint whose records (row slabs) exceed the budget, in groups of one
+    job (row) and of several, only launches kernels: it can be captured, and each replay gives the
+    eager call's bits for the input of the moment."""
     import ctypes
 
     import lamino_amd as la
@@ -105,7 +105,8 @@ def test_adjoint_over_the_record_budget_can_be_captured(monkeypatch, planes):
 
     dims, R, C, P = (21, 9, 23), 31, 33, 150
     monkeypatch.setenv("LAMINO_NUFFT_SLAB_BYTES", str(4096 * planes))   # a record of width 6: 512 complex values
-    say("captured adjoint", planes)
+    monkeypatch.setenv("LAMINO_NUFFT_ROWS", rows)
+    say("captured adjoint", planes, rows)
     ctx = la.Context()
     lib, stream = ctx.lib, ctypes.c_void_p(ctx.lib.lam_ctx_stream(ctx.h))
     pg = la.PolarGrid.per_projection(np.full(P, np.radians(33.0)), 0.2 + 2 * np.pi * np.arange(P) / P, R, C, ctx=ctx)
